@@ -800,6 +800,323 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2
         }
 }
 
+// ---------------------------------------------------------------------------
+// FP32 backprojection of 32 slices on the matrix cores, with both operands
+// split into FP16 hi + lo parts (22 bits each).
+//
+// For one angle a 4 x 4 pixel block reads at most 8 consecutive samples of a
+// sinogram row (scale <= kSplitMaxScale), each pixel two of them with weights
+// 1 - f and f.  As a matrix product that is a 16 x 8 weight matrix, two
+// entries per row, times the 8 samples of every slice; four angles side by
+// side fill the K = 32 of v_mfma_f32_16x16x32_f16:
+//   A [16 pixels][4 angles x 8 samples]: lane m + 16 g holds the 8 weights of
+//     pixel m at angle g,
+//   B [4 angles x 8 samples][16 slices]: lane n + 16 g the samples of slice n.
+// Three products per 16 slices, hi hi + lo hi + hi lo, accumulate in FP32;
+// the dropped lo lo term is 2^-24 of a product.  The pixels' coordinates and
+// weights cost the vector unit about 24 instructions per 64 (pixel, angle)
+// pairs whatever the number of slices, where bp_linear_kernel spends 2.8 per
+// pair and slice.
+//
+// Weight placement: with kb the block's first sample (an even detector, so
+// two samples share a dword) and q = floor(t) - kb in [0, 6], the eight
+// weights are the dword (1 - f, f) moved to half q of 16 bytes.  The four
+// v_perm selectors that do it come from an LDS table indexed by q; a second,
+// all-zero table serves the angles that pad the last group of four.
+//
+// The samples come packed by split_pack_kernel: per angle rows of two
+// adjacent detectors, row R (detectors 2R, 2R + 1) being 32 dwords of hi
+// pairs, one per slice, then 32 of lo pairs, with a zero row at either end.
+// A chunk's rows go from global memory straight to LDS (16 bytes per lane, no
+// registers or vector instructions); two row buffers, one barrier per chunk.  Odd angles' rows are
+// shifted by 64 bytes, so that the two angles whose lanes are read together
+// use different banks.  A block's 4 rows may run past its angle's rows: their
+// weights are zero and what they hold is finite (the next angle's rows, or
+// the zeroed end of the buffer).
+//
+// Bound: LDS reads.  A block's operands take 5 KB per 64 (pixel, angle) pairs
+// (4 KB of samples, 1 KB of selectors) at the ~105 bytes per clock and CU that
+// two-address reads deliver, against about 195 clocks of vector and matrix
+// issue; more waves (6 or 8 per SIMD rather than 4) hide the rest: a wave
+// issues one instruction in 8 clocks at best.  512^2 x 1000 angles, 32 slices:
+// 15.6 us per slice with two launches in flight (packing included, 0.65),
+// bp_linear_kernel 24.5; relative RMSE against float64 2.64e-6 and 2.60e-6.
+// ---------------------------------------------------------------------------
+typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+constexpr int kSplitSlices = 32;          // slices per workgroup
+constexpr int kSplitRow = 256;            // bytes of a packed row
+constexpr double kSplitMaxScale = 1.17;   // 3 sqrt(2) scale + 0.02 <= 5: q stays <= 6 after the alignment
+constexpr int kSplitInfo = 128;           // ring of angle records
+constexpr int kSplitSlack = 6;            // zeroed rows after a buffer
+
+// Packed rows of one angle, the two zero rows included.
+__host__ __device__ constexpr int split_rows(int D) { return (D + 1) / 2 + 2; }
+// Staged rows of one angle, a multiple of the 4 a wave copies at once: W + 1
+// samples from up to three before the window.
+__host__ __device__ constexpr int split_staged(int W) { return ((W + 5) / 2 + 3) / 4 * 4; }
+__host__ __device__ constexpr int split_buffer(int AE, int W)
+{
+    return (AE * split_staged(W) + kSplitSlack) * kSplitRow + 64;
+}
+// Selector tables (2 x 8 x 16 B), two row buffers, the angle records (16 + 16 B).
+__host__ __device__ constexpr int split_lds(int AE, int W) { return 256 + 2 * split_buffer(AE, W) + kSplitInfo * 32; }
+
+// x from lane 0 of each row of 16 lanes
+__device__ __forceinline__ float row_first(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150, 0xf, 0xf, true));
+}
+// x minus the low (high) FP16 half of h in one instruction
+__device__ __forceinline__ float less_low(float x, unsigned h)
+{
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
+    return r;
+}
+__device__ __forceinline__ float less_high(float x, unsigned h)
+{
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
+    return r;
+}
+// (a, b) as FP16 hi and lo pairs
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& hi, unsigned& lo)
+{
+    hi = __builtin_bit_cast(unsigned, __builtin_convertvector((f2_t{a, b}), h2_t));
+    lo = __builtin_bit_cast(unsigned, __builtin_convertvector((f2_t{less_low(a, hi), less_high(b, hi)}), h2_t));
+}
+
+// [slices][P][D] FP32 -> packed rows (value * scale); workgroup (x, y): detectors
+// 64 x .. 64 x + 63 of angle y; slices past the last one are written as zero.
+__global__ void __launch_bounds__(256) split_pack_kernel(const float* __restrict__ sino, int slices, int P, int D,
+                                                         float scale, unsigned* __restrict__ packed)
+{
+    __shared__ unsigned tile[32][65];
+    const int p = blockIdx.y, RP = split_rows(D), R0 = 32 * blockIdx.x;
+    unsigned* out = packed + (long)p * RP * 64;
+    const bool vec = D % 4 == 0 && reinterpret_cast<uintptr_t>(sino) % 16 == 0;
+    for (int i = threadIdx.x; i < kSplitSlices * 16; i += 256) {
+        const int s = i / 16, r = 2 * (i % 16), k = 2 * (R0 + r);
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (s < slices) {
+            const float* row = sino + ((long)s * P + p) * D;
+            if (vec && k + 3 < D) {
+                const float4 f = *reinterpret_cast<const float4*>(row + k);
+                v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (k + j < D) v[j] = row[k + j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            split_pair(v[2 * j] * scale, v[2 * j + 1] * scale, tile[r + j][s], tile[r + j][32 + s]);
+    }
+    __syncthreads();
+    // row R of the sinogram is packed row R + 1
+    for (int i = threadIdx.x; i < 32 * 16; i += 256) {
+        const int r = i / 16, c = 4 * (i % 16);
+        if (R0 + r < RP - 2)
+            reinterpret_cast<uint4*>(out)[(R0 + r + 1) * 16 + i % 16] =
+                make_uint4(tile[r][c], tile[r][c + 1], tile[r][c + 2], tile[r][c + 3]);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 32)
+        reinterpret_cast<uint4*>(out)[(threadIdx.x < 16 ? 0 : (RP - 1) * 16) + threadIdx.x % 16] =
+            make_uint4(0u, 0u, 0u, 0u);
+}
+
+// Test values for timing: zero mean, about a filtered sinogram's size.
+__global__ void tune_fill_kernel(float* out, long n)
+{
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
+        out[i] = (float)((int)((unsigned)i * 2654435761u) >> 8) * 0x1p-26f;
+}
+
+// Workgroup x: a TX x TY tile of the (up to) 32 slices; each wave an 8 x 8
+// pixel block as 2 x 2 blocks of 4 x 4.
+template <int TX, int TY, int WPE>
+__global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* __restrict__ packed,
+                                                               float* __restrict__ img,
+                                                               const float* __restrict__ cosT,
+                                                               const float* __restrict__ sinT, int slices, BpParams p)
+{
+    constexpr int NT = TX * TY, NW = NT / 64;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int AE = p.AE, RW = split_staged(p.W), bufsz = split_buffer(AE, p.W), RP = split_rows(p.D);
+    uint4* tab = reinterpret_cast<uint4*>(smem);
+    char* rows = smem + 256;
+    float4* info = reinterpret_cast<float4*>(rows + 2 * bufsz);   // (cos, sin, -T, LDS address of sample k = 0)
+    // (offset to a block's smallest t, selector table, packed row of the first staged row, -)
+    float4* info2 = info + kSplitInfo;
+
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    int2 txy;
+    bp_work(p, txy);
+    const int x0 = txy.x * TX, y0 = txy.y * TY;
+    const int bx = x0 + (wave % (TX / 8)) * 8, by = y0 + (wave / (TX / 8)) * 8;   // the wave's block
+    const int m = lane & 15, g = lane >> 4;
+    float xp[2], yp[2];
+    bool use = false;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        xp[i] = ((float)(bx + 4 * i + (m & 3)) - p.center) * p.scale;
+        yp[i] = ((float)(by + 4 * i + (m >> 2)) - p.center) * p.scale;
+    }
+#pragma unroll
+    for (int sb = 0; sb < 4; sb++) {
+        const int x = bx + 4 * (sb & 1) + (m & 3), y = by + 4 * (sb >> 1) + (m >> 2);
+        use |= x < p.N && y < p.N && !(p.mask && bp_outside(x, y, p.N, p.center));
+    }
+    const bool active = __any(use);
+    const int nch = __syncthreads_or(use) ? (p.P + AE - 1) / AE : 0;
+
+    f4_t acc[4][2];
+#pragma unroll
+    for (int sb = 0; sb < 4; sb++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) acc[sb][u] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    const unsigned rbase = lds_address(rows), tbase = lds_address(tab);
+    // records of angles 64 b .. 64 b + 63 (AE divides 64), slot angle % 128, by
+    // one wave, another one each time; those past the last angle repeat it
+    // with the all-zero selector table
+    auto make_info = [&](int b) {
+        if (wave != b % NW) return;
+        const int pa = 64 * b + lane, pc = min(pa, p.P - 1), r = pa % kSplitInfo;
+        const int ch = pc / AE, a = pc - ch * AE;
+        const float xa = ((float)x0 - p.center) * p.scale, xb = ((float)(x0 + TX - 1) - p.center) * p.scale;
+        const float ya = ((float)y0 - p.center) * p.scale, yb = ((float)(y0 + TY - 1) - p.center) * p.scale;
+        const AngleWin w = angle_window(cosT[pc], sinT[pc], xa, xb, ya, yb, p.cI);
+        // the origin is moved down to an even detector
+        const int odd = ((int)-w.negT + p.cI) & 1, first = (w.kmin + odd - 2) & ~1;
+        info[r] = make_float4(w.c, w.s, w.negT + (float)odd,
+                              __uint_as_float(rbase + (unsigned)((ch & 1) * bufsz + a * RW * kSplitRow + (a & 1) * 64 -
+                                                                 first * (kSplitRow / 2))));
+        info2[r] = make_float4(3.0f * p.scale * (fminf(w.c, 0.0f) + fminf(w.s, 0.0f)) - 0.01f,
+                               __uint_as_float(tbase + (pa < p.P ? 0u : 128u)),
+                               __int_as_float((first + (int)-w.negT - odd + p.cI) / 2 + 1), 0.0f);
+    };
+    // chunk ch's rows into its buffer: a wave copies 4 rows (1 KB) at a time
+    const int units = AE * RW / 4;
+    auto stage = [&](int ch) {
+        const int p0 = ch * AE, na = min(AE, p.P - p0);
+        for (int i = wave; i < units; i += NW) {
+            const int a = i / (RW / 4), r = 4 * (i - a * (RW / 4));
+            if (a >= na) break;
+            const int R = __float_as_int(info2[(p0 + a) % kSplitInfo].z) + r + lane / 16;
+            const unsigned* src = packed + ((long)(p0 + a) * RP + clamp_index(R, RP - 1)) * 64 + (lane & 15) * 4;
+            char* dst = rows + (ch & 1) * bufsz + (a * RW + r) * kSplitRow + (a & 1) * 64;
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                             (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+        }
+    };
+    if (nch) {
+        for (int i = tid; i < 2 * bufsz / 16; i += NT) reinterpret_cast<uint4*>(rows)[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (tid < 16) {
+            // row q of the first table: byte selectors that move (w0, w1) to half q
+            unsigned sel[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int d = tid - 2 * j;
+                sel[j] = d == 0 ? 0x03020100u : (d == -1 ? 0x0c0c0302u : (d == 1 ? 0x01000c0cu : 0x0c0c0c0cu));
+                if (tid > 6) sel[j] = 0x0c0c0c0cu;
+            }
+            tab[tid] = make_uint4(sel[0], sel[1], sel[2], sel[3]);
+        }
+        make_info(0);
+        make_info(1);
+        __syncthreads();
+        stage(0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    for (int ch = 0; ch < nch; ch++) {
+        const int p0 = ch * AE, na = min(AE, p.P - p0);
+        // chunks ch and ch + 1 lie in blocks p0 / 64 and the next: the ring's
+        // other half is free for the block after
+        if (ch > 0 && p0 % 64 == 0 && p0 + 64 < p.P) make_info(p0 / 64 + 1);
+        if (ch + 1 < nch) stage(ch + 1);
+        if (active) {
+            const float4* inf = info + p0 % kSplitInfo + g;
+            for (int a = 0; a < na; a += 4) {
+                const float4 in = inf[a], in2 = inf[a + kSplitInfo];
+                const unsigned rb = __float_as_uint(in.w) + (unsigned)m * 4u, tb = __float_as_uint(in2.y);
+                const float xc[2] = {__builtin_fmaf(xp[0], in.x, in.z), __builtin_fmaf(xp[1], in.x, in.z)};
+#pragma unroll
+                for (int sb = 0; sb < 4; sb++) {
+                    const float t = __builtin_fmaf(yp[sb >> 1], in.y, xc[sb & 1]);
+                    const int kb = floor_to_int(row_first(t) + in2.x) & ~1;
+                    int k;
+                    float f;
+                    bp_split(t, k, f);
+                    const lds_u4 sel = lds_load<lds_u4>(tb + (unsigned)(k - kb) * 16u);
+                    unsigned at = rb + (unsigned)kb * (kSplitRow / 2);
+                    unsigned hi, lo;
+                    split_pair(1.0f - f, f, hi, lo);
+                    lds_u4 bh[2], bl[2];
+#pragma unroll
+                    for (int u = 0; u < 2; u++) {
+                        // opaque bases: each two-address read then fills two
+                        // adjacent registers of one operand
+                        asm("" : "+v"(at));
+#pragma unroll
+                        for (int j = 0; j < 4; j++) bh[u][j] = lds_load<unsigned>(at + kSplitRow * j);
+                        at += 128;
+                        asm("" : "+v"(at));
+#pragma unroll
+                        for (int j = 0; j < 4; j++) bl[u][j] = lds_load<unsigned>(at + kSplitRow * j);
+                        at -= 64;
+                    }
+                    lds_u4 ah, al;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        ah[j] = __builtin_amdgcn_perm(0u, hi, sel[j]);
+                        al[j] = __builtin_amdgcn_perm(0u, lo, sel[j]);
+                    }
+                    auto mma = [](f4_t& c, lds_u4 a, lds_u4 b) {
+                        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, a),
+                                                                   __builtin_bit_cast(h8_t, b), c, 0, 0, 0);
+                    };
+#pragma unroll
+                    for (int u = 0; u < 2; u++) mma(acc[sb][u], al, bh[u]);
+#pragma unroll
+                    for (int u = 0; u < 2; u++) mma(acc[sb][u], ah, bl[u]);
+#pragma unroll
+                    for (int u = 0; u < 2; u++) mma(acc[sb][u], ah, bh[u]);
+                }
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's part of chunk ch + 1 is in LDS
+        __syncthreads();
+    }
+    // lane (n = m, g): pixels 4 g .. 4 g + 3 of a block (its row g), slice 16 u + n
+#pragma unroll
+    for (int sb = 0; sb < 4; sb++) {
+        const int x = bx + 4 * (sb & 1), y = by + 4 * (sb >> 1) + g;
+        if (y >= p.N || x >= p.N) continue;
+        bool in[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) in[v] = !(p.mask && bp_outside(x + v, y, p.N, p.center));
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            if (16 * u + m >= slices) continue;
+            float* o = img + (long)(16 * u + m) * p.N * p.N + (long)y * p.N + x;
+            f4_t r;
+#pragma unroll
+            for (int v = 0; v < 4; v++) r[v] = in[v] ? acc[sb][u][v] * p.norm * p.out_scale : p.maskingValue;
+            if (x + 4 <= p.N && reinterpret_cast<uintptr_t>(o) % 16 == 0) {
+                *reinterpret_cast<f4_t*>(o) = r;
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (x + v < p.N) o[v] = r[v];
+            }
+        }
+    }
+}
+
 // [slices][P][D] FP16 -> the x4 layout (zero-filled past the last slice).
 __global__ void f16_to_x4_kernel(const uint16_t* __restrict__ in, uint2* __restrict__ out, int slices, long plane)
 {
@@ -1891,6 +2208,114 @@ extern "C" int risa_hip_bp_run_f16(risa_bp_t h, const uint16_t* sino, float in_s
             launch_f16x4(h, h->variant_f16, h->x4.ptr, in_scale, n, img + (size_t)s0 * h->g.numberOfPixels *
                          h->g.numberOfPixels, s);
         }
+    });
+}
+
+// ------------------------------------------ FP32 split backprojection --
+// Used by the chain for groups of many frames (chain.hip); its sums are
+// rounded otherwise than bp_linear_kernel's, at the same accuracy.
+struct SplitShape {
+    int tx, ty, amax, variant;   // variant: an FP32 variant of the same tile shape (its dispatch order)
+    void (*fn)(const unsigned*, float*, const float*, const float*, int, BpParams);
+};
+static const SplitShape kSplitShapes[] = {
+    {32, 32, 8, 0, bp_split_kernel<32, 32, 4>},
+    {32, 16, 4, 1, bp_split_kernel<32, 16, 6>},
+    {16, 16, 4, 2, bp_split_kernel<16, 16, 8>},
+};
+constexpr int kNumSplitShapes = sizeof(kSplitShapes) / sizeof(kSplitShapes[0]);
+constexpr int kMaxSplitLds = 160 * 1024;   // a gfx950 workgroup's LDS
+
+// Bytes of the packed sinograms of one launch (32 slices); 0 where the
+// geometry is outside what the kernel takes.
+extern "C" size_t risa_bp_split_bytes(risa_bp_t h)
+{
+    const risa_geom& g = h->g;
+    if (g.useTextureMemory || g.interpolationType == 1 || h->lut.scale > kSplitMaxScale) return 0;
+    return (size_t)g.numberOfParallelProjections * split_rows(g.numberOfParallelDetectors) * kSplitRow;
+}
+
+// Up to 32 sinograms [slices][P][D] -> images [slices][N][N] with tile shape
+// `shape`; |value * scale| must stay within the FP16 range.  `packed`:
+// risa_bp_split_bytes of scratch, 16-byte aligned.
+extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, float scale, int slices, void* packed, float* img,
+                      hipStream_t s)
+{
+    return guarded("risa_bp_run_split", [&] {
+        if (shape < 0 || shape >= kNumSplitShapes || slices < 1 || slices > kSplitSlices || !(scale > 0.0f))
+            fail(RISA_ERR_ARG, "bad argument");
+        if (risa_bp_split_bytes(h) == 0) fail(RISA_ERR_UNSUPPORTED, "geometry outside the split backprojector's range");
+        const SplitShape& v = kSplitShapes[shape];
+        BpParams p = make_params(h, v.tx, v.ty);
+        p.out_scale = 1.0f / scale;
+        p.AE = v.amax;
+        while (p.AE > 4 && split_lds(p.AE, p.W) > kMaxSplitLds) p.AE /= 2;
+        const int lds = split_lds(p.AE, p.W);
+        if (lds > kMaxSplitLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %d B of LDS", lds);
+        dim3 grid(p.tilesX * ceil_div(p.N, v.ty), 1);
+        p.xg = xcd_groups(grid.x, 1);
+        const long off = h->order_off[(size_t)v.variant];
+        p.order = p.xg && off >= 0 ? h->tile_order.ptr + off : nullptr;
+        unsigned* pk = reinterpret_cast<unsigned*>(packed);
+        hipLaunchKernelGGL(split_pack_kernel, dim3(ceil_div(split_rows(p.D) - 2, 32), p.P), dim3(256), 0, s, sino,
+                           slices, p.P, p.D, scale, pk);
+        check_launch("split_pack_kernel");
+        hipLaunchKernelGGL(v.fn, grid, dim3(v.tx * v.ty), lds, s, pk, img, h->cosT.ptr, h->sinT.ptr, slices, p);
+        check_launch("bp_split_kernel");
+    });
+}
+
+// Times the split shapes at 32 slices against the handle's FP32 variant on
+// the same launch: `shape` gets the fastest one and `min_slices` the batch
+// from which it beats the variant (its cost does not depend on the slices up
+// to 32, the variant's is about proportional), or more than 32 if never.
+extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, int* min_slices)
+{
+    return guarded("risa_bp_tune_split", [&] {
+        DeviceGuard dg(h->device);
+        const size_t ns = (size_t)h->g.numberOfParallelProjections * h->g.numberOfParallelDetectors;
+        const size_t ni = (size_t)h->g.numberOfPixels * h->g.numberOfPixels;
+        DeviceBuffer<float> sino(ns * kSplitSlices), img(ni * kSplitSlices);
+        DeviceBuffer<char> packed(risa_bp_split_bytes(h));
+        // values that toggle the multipliers as real ones do
+        hipLaunchKernelGGL(tune_fill_kernel, dim3(1024), dim3(256), 0, s, sino.ptr, (long)sino.count);
+        check_launch("tune_fill_kernel");
+        struct Events {
+            hipEvent_t a = nullptr, b = nullptr;
+            ~Events()
+            {
+                if (a) (void)hipEventDestroy(a);
+                if (b) (void)hipEventDestroy(b);
+            }
+        } ev;
+        RISA_HIP_CHECK(hipEventCreate(&ev.a));
+        RISA_HIP_CHECK(hipEventCreate(&ev.b));
+        auto time_it = [&](auto&& launch) {
+            launch();
+            RISA_HIP_CHECK(hipEventRecord(ev.a, s));
+            for (int it = 0; it < 5; it++) launch();
+            RISA_HIP_CHECK(hipEventRecord(ev.b, s));
+            RISA_HIP_CHECK(hipEventSynchronize(ev.b));
+            float ms = 0;
+            RISA_HIP_CHECK(hipEventElapsedTime(&ms, ev.a, ev.b));
+            return ms;
+        };
+        float plain = 1e30f, best = 1e30f;
+        *shape = 0;
+        for (int round = 0; round < 2; round++) {
+            plain = std::min(plain, time_it([&] { launch_linear(h, h->variant, sino.ptr, img.ptr, kSplitSlices, s); }));
+            for (int v = 0; v < kNumSplitShapes; v++) {
+                const float ms = time_it([&] {
+                    if (risa_bp_run_split(h, v, sino.ptr, 1024.0f, kSplitSlices, packed.ptr, img.ptr, s) != RISA_OK)
+                        fail(RISA_ERR_HIP, "%s", risa_last_error());
+                });
+                if (ms < best) {
+                    best = ms;
+                    *shape = v;
+                }
+            }
+        }
+        *min_slices = 1 + (int)(kSplitSlices * best / plain);
     });
 }
 

@@ -10,7 +10,12 @@
 //        per group) are dealt round-robin to `lanes` streams (own scratch
 //        buffers each) forked from and joined back into the caller's stream,
 //        so lanes x per frames are in flight -- the way the reference
-//        overlaps frames across its per-stage threads.
+//        overlaps frames across its per-stage threads.  Chains of at least 64
+//        frames take groups of 32 and backproject those of at least split_min
+//        frames on the matrix cores (bp_split_kernel), where timing both at
+//        creation finds that the faster way: 256 frames of 512^2 x 1000 angles
+//        4.40 ms a call, 6.75 with bp_linear_kernel; 256^2 x 500 stays with
+//        the latter (158 us per 32 slices against 208).
 // MIXED: groups of `per` consecutive frames (a multiple of 4, up to 32) dealt
 //        to `lanes` streams the same way; per group the DFT-GEMM filter on
 //        MFMA writes the FP16 sinogram in the 4-slice interleaved layout and
@@ -19,16 +24,24 @@
 //        backprojection.
 #include "device_common.h"
 
+#include <cmath>
 #include <map>
 #include <tuple>
 #include <vector>
 
 int risa_filter_run_oop(risa_filter_t h, const float* in, float* out, long rows, hipStream_t s);
+double risa_filter_l1(risa_filter_t h);
+int risa_fan2para_gain(risa_fan2para_t h, double* gain);
+extern "C" size_t risa_bp_split_bytes(risa_bp_t h);
+extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, int* min_slices);
+extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, float scale, int slices, void* packed, float* img,
+                      hipStream_t s);
 
 namespace {
 constexpr float kF16SinoScale = 256.0f;   // FP16 filtered sinogram stores 256 * value
 constexpr int kPlainLanes = 2;            // streams in PLAIN mode
 constexpr int kPlainMaxPer = 16;          // frames per lane step in PLAIN mode, at most
+constexpr int kSplitPer = 32;             // frames per lane step of a PLAIN chain with the split backprojector
 constexpr int kMixedLanes = 2;            // streams in MIXED mode
 constexpr int kMixedMaxPer = 32;          // frames per lane step in MIXED mode, at most (a multiple of 4)
 }  // namespace
@@ -55,6 +68,13 @@ struct risa_chain_s {
     risa_bp_t bp = nullptr;
     risa::DeviceBuffer<float> att_buf, par_buf, filt_buf;   // `per` frame slots per lane
     risa::DeviceBuffer<uint16_t> f16_buf;                   // MIXED: `per` slots per lane, x4 layout
+    // PLAIN, per = kSplitPer: groups of at least split_min frames go through
+    // the FP32 backprojector on the matrix cores (tile shape split_shape, -1:
+    // off), whose FP16 hi + lo operands hold filtered sample * split_scale
+    int split_shape = -1, split_min = 0;
+    float split_scale = 0.0f;
+    risa::DeviceBuffer<char> split_buf;                     // packed sinograms, one launch per lane
+    size_t split_bytes = 0;
     std::vector<hipStream_t> lane_streams;
     std::vector<hipEvent_t> lane_events;   // [0] fork, [1..lanes] joins
     std::map<std::tuple<const void*, const void*, int, std::vector<int32_t>>, ChainGraph> graphs;
@@ -97,6 +117,32 @@ static void ok(int rc)
     if (rc != RISA_OK) fail(rc, "%s", risa_last_error());
 }
 
+// The power of two that brings every filtered sample of the chain into the
+// FP16 range, from what the stages can produce: counts of 0 .. 65535 over the
+// given references, the rebinning's weights and the filter's absolute sum.
+// 0 when there is none (references that are not finite).
+static float split_scale(risa_chain_t h, const float* avg_ref, const float* avg_dark)
+{
+    const risa_geom& g = h->g;
+    const long Df = g.numberOfFanDetectors, n = Df * g.numberOfFanProjections;
+    const float tiny = 1.0e-5f;
+    float lo = INFINITY, hi = 0.0f, num = tiny;   // the denominators' range, the largest numerator
+    for (int k = 0; k < g.numberOfPlanes; k++)
+        for (long e = 0; e < n; e++) {
+            const float dark = avg_dark[k * Df + e % Df], den = std::max(avg_ref[k * n + e] - dark, tiny);
+            if (!(std::fabs(dark) <= 1e30f) || !(den <= 1e30f) || std::isnan(avg_ref[k * n + e])) return 0.0f;
+            lo = std::min(lo, den);
+            hi = std::max(hi, den);
+            num = std::max(num, 65535.0f - dark);
+        }
+    double gain = 0.0;
+    ok(risa_fan2para_gain(h->f2p, &gain));
+    const double att = std::max(std::fabs(std::log((double)num / lo)), std::fabs(std::log((double)tiny / hi)));
+    const double bound = 1.001 * att * gain * risa_filter_l1(h->filt);
+    if (!(bound > 0.0) || !(bound < 1e6)) return 0.0f;
+    return (float)std::exp2(std::floor(std::log2(65000.0 / bound)));
+}
+
 extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, const float* avg_dark, int device,
                                      int mode, int max_frames, risa_chain_t* out)
 {
@@ -120,6 +166,18 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
             if (mode == RISA_CHAIN_PLAIN) {
                 h->lanes = std::min(kPlainLanes, max_frames);
                 h->per = std::max(1, std::min(kPlainMaxPer, max_frames / h->lanes));
+                if (max_frames >= kPlainLanes * kSplitPer && (h->split_bytes = risa_bp_split_bytes(h->bp)) > 0 &&
+                    (h->split_scale = split_scale(h, avg_ref, avg_dark)) > 0.0f) {
+                    ok(risa_hip_bp_autotune_batch(h->bp, kPlainLanes * kPlainMaxPer, nullptr));
+                    ok(risa_bp_tune_split(h->bp, nullptr, &h->split_shape, &h->split_min));
+                    if (h->split_min <= kSplitPer) {
+                        h->per = kSplitPer;
+                        h->split_bytes = (h->split_bytes + 255) / 256 * 256;
+                        h->split_buf.resize(h->split_bytes * h->lanes);
+                    } else {
+                        h->split_shape = -1;
+                    }
+                }
                 const size_t slots = (size_t)h->lanes * h->per;
                 h->att_buf.resize(fan * slots);
                 h->par_buf.resize(par * slots);
@@ -150,7 +208,9 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
             // itself per variant, eagerly, proved too noisy to rank the closest
             // shapes
             if (mode == RISA_CHAIN_PLAIN) {
-                if (h->per > 1) ok(risa_hip_bp_autotune_batch(h->bp, h->lanes * h->per, nullptr));
+                if (h->split_min > 0) {
+                    // tuned above
+                } else if (h->per > 1) ok(risa_hip_bp_autotune_batch(h->bp, h->lanes * h->per, nullptr));
                 else ok(risa_hip_bp_autotune_slices(h->bp, h->lanes, nullptr));
             } else {
                 ok(risa_hip_bp_autotune_f16(h->bp, h->per, nullptr));
@@ -191,7 +251,11 @@ static void enqueue(risa_chain_t h, const uint16_t* raw, const int32_t* planes, 
                 ok(risa_hip_attenuation_run_batch(h->att, raw + f * fan, planes + f, n, att, ls));
                 ok(risa_hip_fan2para_run_batch(h->f2p, att, planes + f, n, pb, ls));
                 ok(risa_filter_run_oop(h->filt, pb, fb, (long)n * g.numberOfParallelProjections, ls));
-                ok(risa_hip_bp_run_batch(h->bp, fb, n, img + f * out, ls));
+                if (h->split_shape >= 0 && n >= h->split_min)
+                    ok(risa_bp_run_split(h->bp, h->split_shape, fb, h->split_scale, n, h->split_buf.ptr + k * h->split_bytes,
+                                         img + f * out, ls));
+                else
+                    ok(risa_hip_bp_run_batch(h->bp, fb, n, img + f * out, ls));
             }
         } else {
             uint16_t* hb = h->f16_buf.ptr + (size_t)k * per * par;
@@ -296,6 +360,7 @@ extern "C" int risa_hip_chain_set_variant(risa_chain_t h, int variant)
         h->drain();
         h->release_graphs();
         ok(risa_hip_bp_set_variant(h->bp, variant));
+        h->split_shape = -1;   // every group with the given variant
     });
 }
 

@@ -17,6 +17,7 @@
 #include "device_common.h"
 
 #include <algorithm>
+#include <cstring>
 
 #include "../host/tables.h"
 
@@ -299,6 +300,23 @@ __global__ void rebin_weights_f64_kernel(uint32_t* __restrict__ q, RebinGeo g, i
     w[8 + slot] = __float_as_uint((float)fg);
 }
 
+// Largest factor by which the table's bilinear weights can raise a sample
+// ((|1 - ft| + |ft|) (|1 - fg| + |fg|); 1 inside a cell), as float bits.
+__global__ void __launch_bounds__(256) rebin_gain_kernel(const uint32_t* __restrict__ table, long entries,
+                                                         unsigned* __restrict__ gain)
+{
+    float g = 0.0f;
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < entries * 4; i += (long)gridDim.x * blockDim.x) {
+        const uint32_t* q = table + (i / 4) * 12;
+        const int sl = (int)(i % 4);
+        if (!(q[sl] >> 31)) continue;
+        const float ft = __uint_as_float(q[4 + sl]), fg = __uint_as_float(q[8 + sl]);
+        const float v = (fabsf(1.0f - ft) + fabsf(ft)) * (fabsf(1.0f - fg) + fabsf(fg));
+        g = v <= 1e30f ? fmaxf(g, v) : INFINITY;   // NaN counts as unbounded
+    }
+    atomicMax(gain, __float_as_uint(g));
+}
+
 }  // namespace risa
 
 struct risa_fan2para_s {
@@ -436,6 +454,30 @@ extern "C" int risa_hip_fan2para_create_ex(const risa_geom* g, int device, int w
 extern "C" int risa_hip_fan2para_create(const risa_geom* g, int device, risa_fan2para_t* out)
 {
     return risa_hip_fan2para_create_ex(g, device, RISA_REBIN_WEIGHTS_FP64, out);
+}
+
+// An upper bound of |rebinned sample| / max |fan sample| (an output is a mean
+// of rays, plus half a sample more at an odd D's doubled column).
+int risa_fan2para_gain(risa_fan2para_t h, double* gain)
+{
+    return guarded("risa_fan2para_gain", [&] {
+        DeviceGuard dg(h->device);
+        DeviceBuffer<unsigned> g(1);
+        g.upload({0u});
+        hipLaunchKernelGGL(rebin_gain_kernel, dim3(1024), dim3(256), 0, nullptr, h->table.ptr, (long)(h->table.count / 12),
+                           g.ptr);
+        check_launch("rebin_gain_kernel");
+        if (h->extra.count) {
+            hipLaunchKernelGGL(rebin_gain_kernel, dim3(16), dim3(256), 0, nullptr, h->extra.ptr,
+                               (long)(h->extra.count / 12), g.ptr);
+            check_launch("rebin_gain_kernel");
+        }
+        unsigned bits = 0;
+        RISA_HIP_CHECK(hipMemcpy(&bits, g.ptr, sizeof(bits), hipMemcpyDeviceToHost));
+        float v;
+        std::memcpy(&v, &bits, sizeof(v));
+        *gain = 1.5 * (double)v;
+    });
 }
 
 // Frame f of the call reads fan(f) and writes par(f).

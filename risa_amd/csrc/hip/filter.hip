@@ -1382,6 +1382,14 @@ int risa_filter_run_oop(risa_filter_t h, const float* in, float* out, long rows,
     });
 }
 
+// Sum of |c| over the circulant: |filtered| <= this times max |row|.
+double risa_filter_l1(risa_filter_t h)
+{
+    double sum = 0.0;
+    for (double v : circulant(h->taps, h->g.numberOfParallelDetectors)) sum += std::fabs(v);
+    return sum;
+}
+
 extern "C" int risa_hip_filter_adjoint_run(risa_filter_t h, float* grad, int slices, void* stream)
 {
     // C is symmetric (c[d] = c[-d]), so the adjoint is the same filter.
