@@ -580,52 +580,84 @@ __global__ void __launch_bounds__(256) fft_xspec_kernel(const float* __restrict_
         }
 }
 
-// Bin k of the summed spectrum: the partials in block order, in double.
-__global__ void xspec_reduce_kernel(const float2* __restrict__ partial, int nblocks, int K, double2* __restrict__ sum)
+// The tail of the padded tap gradient: three short sums, each bound by the
+// latency of its serial chain, so each is spread over a workgroup and added up
+// in a fixed order (one thread per output took 112, 154 and 75 us at D = 303,
+// M = 625, 453 partials; now 7, 5 and 5).
+
+// sum of v over the workgroup's 256 threads by a fixed tree, in thread 0
+__device__ __forceinline__ double block_sum(double v, double* red)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= K) return;
-    double sx = 0.0, sy = 0.0;
-    for (int b = 0; b < nblocks; b++) {
-        const float2 v = partial[(long)b * K + k];
-        sx += v.x;
-        sy += v.y;
+    red[threadIdx.x] = v;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+        __syncthreads();
     }
-    sum[k] = make_double2(sx, sy);
+    return red[0];
+}
+
+// Bins 8 blockIdx.x + 0..7 of the summed spectrum, in double: thread
+// (32 chains, 8 bins) takes partials chain, chain + 32, ... in order (a row of
+// 8 bins is one 64-byte segment), then a fixed tree over the chains.
+__global__ void __launch_bounds__(256) xspec_reduce_kernel(const float2* __restrict__ partial, int nblocks, int K,
+                                                           double2* __restrict__ sum)
+{
+    __shared__ double2 red[256];
+    const int k = blockIdx.x * 8 + threadIdx.x % 8;
+    double2 acc = make_double2(0.0, 0.0);
+    if (k < K)
+        for (int b = threadIdx.x / 8; b < nblocks; b += 32) {
+            const float2 v = partial[(long)b * K + k];
+            acc.x += v.x;
+            acc.y += v.y;
+        }
+    red[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = 128; w >= 8; w >>= 1) {
+        if ((int)threadIdx.x < w) {
+            red[threadIdx.x].x += red[threadIdx.x + w].x;
+            red[threadIdx.x].y += red[threadIdx.x + w].y;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x < 8 && k < K) sum[k] = red[threadIdx.x];
 }
 
 // R[d] = r_lin[d] + r_lin[d - D], r_lin[j] = (1/M) sum_k S(k) e^{2 pi i j k / M}
-// over the Hermitian spectrum S (S(M - k) = conj S(k)).
-__global__ void xcorr_wrap_kernel(const double2* __restrict__ S, int M, int D, double* __restrict__ R)
+// over the Hermitian spectrum S (S(M - k) = conj S(k)); workgroup d, its
+// threads over the bins.
+__global__ void __launch_bounds__(256) xcorr_wrap_kernel(const double2* __restrict__ S, int M, int D,
+                                                         double* __restrict__ R)
 {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    if (d >= D) return;
-    double acc = 0.0;
-    for (int w = 0; w < 2; w++) {
-        const long j = w == 0 ? d : (long)d - D + M;   // r_lin[d - D] sits at index d - D + M
-        double v = S[0].x;
-        const int kmax = (M % 2 == 0) ? M / 2 - 1 : M / 2;
-        for (int k = 1; k <= kmax; k++) {
-            double sn, cs;
-            sincospi(2.0 * (double)((j * k) % M) / M, &sn, &cs);
-            v += 2.0 * (S[k].x * cs - S[k].y * sn);
-        }
-        if (M % 2 == 0) v += S[M / 2].x * ((j % 2) ? -1.0 : 1.0);
-        acc += v;
+    __shared__ double red[256];
+    const int d = blockIdx.x;
+    const int j0 = d, j1 = d - D + M;   // r_lin[d - D] sits at index d - D + M
+    double v = 0.0;
+    for (int k = threadIdx.x; k <= M / 2; k += 256) {
+        double s0, c0, s1, c1;
+        sincospi(2.0 * (double)((unsigned)(j0 * k) % (unsigned)M) / M, &s0, &c0);
+        sincospi(2.0 * (double)((unsigned)(j1 * k) % (unsigned)M) / M, &s1, &c1);
+        // bins 0 and M / 2 (even M) are their own mirror images
+        const double2 z = S[k];
+        v += (k == 0 || 2 * k == M ? 1.0 : 2.0) * (z.x * (c0 + c1) - z.y * (s0 + s1));
     }
-    R[d] = acc / M;
+    v = block_sum(v, red);
+    if (threadIdx.x == 0) R[d] = v / M;
 }
 
-// dtaps[k] = w_k sum_d R[d] cos(2 pi k d / D).
-__global__ void xcorr_taps_kernel(const double* __restrict__ R, int D, float* __restrict__ dtaps)
+// dtaps[k] = w_k sum_d R[d] cos(2 pi k d / D), workgroup k.
+__global__ void __launch_bounds__(256) xcorr_taps_kernel(const double* __restrict__ R, int D,
+                                                         float* __restrict__ dtaps)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int K = D / 2 + 1;
-    if (k >= K) return;
+    __shared__ double red[256];
+    const int k = blockIdx.x;
     double acc = 0.0;
-    for (int d = 0; d < D; d++) acc += R[d] * cospi(2.0 * (double)(((long)k * d) % D) / D);
+    for (int d = threadIdx.x; d < D; d += 256)
+        acc += R[d] * cospi(2.0 * (double)((unsigned)(k * d) % (unsigned)D) / D);
+    acc = block_sum(acc, red);
     const double wk = (k == 0 || (D % 2 == 0 && k == D / 2)) ? 1.0 : 2.0;
-    dtaps[k] = (float)(wk * acc);
+    if (threadIdx.x == 0) dtaps[k] = (float)(wk * acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1419,11 +1451,11 @@ static void launch_grad_taps_padded(risa_filter_t h, const float* x, const float
     hipLaunchKernelGGL(fft_xspec_kernel, dim3(grid), dim3(128 * slots), lds, s, x, g, h->tw.ptr, h->plan, D, rows,
                        sc.xpart);
     check_launch("fft_xspec_kernel");
-    hipLaunchKernelGGL(xspec_reduce_kernel, dim3(ceil_div(KM, 256)), dim3(256), 0, s, sc.xpart, grid, KM, sc.xsum);
+    hipLaunchKernelGGL(xspec_reduce_kernel, dim3(ceil_div(KM, 8)), dim3(256), 0, s, sc.xpart, grid, KM, sc.xsum);
     check_launch("xspec_reduce_kernel");
-    hipLaunchKernelGGL(xcorr_wrap_kernel, dim3(ceil_div(D, 64)), dim3(64), 0, s, sc.xsum, M, D, sc.xcorr);
+    hipLaunchKernelGGL(xcorr_wrap_kernel, dim3(D), dim3(256), 0, s, sc.xsum, M, D, sc.xcorr);
     check_launch("xcorr_wrap_kernel");
-    hipLaunchKernelGGL(xcorr_taps_kernel, dim3(ceil_div(D / 2 + 1, 64)), dim3(64), 0, s, sc.xcorr, D, dtaps);
+    hipLaunchKernelGGL(xcorr_taps_kernel, dim3(D / 2 + 1), dim3(256), 0, s, sc.xcorr, D, dtaps);
     check_launch("xcorr_taps_kernel");
 }
 
