@@ -6,7 +6,7 @@
 // (:231-241), cuFFT C2R, with taps from designFilter (:169-191).
 //
 // Two implementations:
-//  * FFT32: a batched Stockham FFT written here (radices 4, 2, 3, 5) that
+//  * FFT32: a batched Stockham FFT written here (radices 5, 3, 8, 4, 2) that
 //    keeps a row pair in LDS: two real rows x_a, x_b are transformed as one
 //    complex row z = x_a + i x_b; since H is real and symmetric,
 //    IDFT(H . DFT(z)) = y_a + i y_b.  One HBM read and one write per element.
@@ -28,6 +28,7 @@ struct FftPlan {
     int D;
     int nst;
     int radix[24];
+    float inv[24];   // 1 / (product of the earlier passes' radices)
 };
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
@@ -103,34 +104,92 @@ __device__ __forceinline__ void dft8(float2* a)
     a[7] = csub(e[3], o3);
 }
 
-// Butterfly b (0 <= b < m = D / r) of one radix-r Stockham pass over a row of
-// length D (src -> dst; Ns = product of the earlier passes' radices,
-// stride = D / (Ns r)).
-template <int S>
-__device__ __forceinline__ void stockham_butterfly(const float2* src, float2* dst, int r, int Ns, int m, int stride,
-                                                   const float2* __restrict__ tw, int b)
+// Row entry i in LDS.  PAD: one spare entry after every 8, for plans whose
+// passes are all powers of two: without it the first passes' writes (stride R)
+// and the second's (blocks of R at stride R^2) hit few banks.  A plan that
+// begins with 5 or 3 spreads them by itself.
+template <bool PAD>
+__host__ __device__ constexpr int row_index(int i)
 {
-    const int k = b % Ns;
-    float2 a[5];
-    a[0] = src[b];
-    for (int q = 1; q < r; q++) {
-        float2 w = tw[q * k * stride];
-        if (S > 0) w.y = -w.y;
-        a[q] = cmul(src[b + q * m], w);
-    }
-    butterfly<S>(a, r);
-    const int base = (b - k) * r + k;
-    for (int q = 0; q < r; q++) dst[base + q * Ns] = a[q];
+    return PAD ? i + (i >> 3) : i;
 }
 
-// One Stockham pass over a row held in LDS (src -> dst), threads t0..T-1.
-template <int S>
-__device__ __forceinline__ void stockham_pass(const float2* src, float2* dst, int D, int r, int Ns,
-                                              const float2* __restrict__ tw, int t0, int T)
+// Butterfly b (0 <= b < m = M / R) of one radix-R Stockham pass over a row of
+// length M (src -> dst; Ns = product of the earlier passes' radices, inv =
+// 1 / Ns, stride = M / (Ns R)).  The radix is a template argument, so the
+// elements stay in registers.
+template <int S, int R, bool PAD, class Tw>
+__device__ __forceinline__ void stockham_butterfly(const float2* src, float2* dst, int Ns, float inv, int m, int stride,
+                                                   Tw tw, int b)
 {
-    const int m = D / r;
-    const int stride = D / (Ns * r);
-    for (int b = t0; b < m; b += T) stockham_butterfly<S>(src, dst, r, Ns, m, stride, tw, b);
+    // b mod Ns; b < 2^20: (b + 1/2) / Ns is at least 1 / (2 Ns) from the next
+    // integer, its rounding error below 2^-2 / Ns
+    const int k = b - (int)(((float)b + 0.5f) * inv) * Ns;
+    float2 a[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) a[q] = src[row_index<PAD>(b + q * m)];
+    if (Ns > 1) {
+#pragma unroll
+        for (int q = 1; q < R; q++) {
+            float2 w = tw[q * k * stride];
+            if (S > 0) w.y = -w.y;
+            a[q] = cmul(a[q], w);
+        }
+    }
+    if constexpr (R == 8) dft8<S>(a);
+    else butterfly<S>(a, R);
+    const int base = (b - k) * R + k;
+#pragma unroll
+    for (int q = 0; q < R; q++) dst[row_index<PAD>(base + q * Ns)] = a[q];
+}
+
+template <int R, bool PAD, class Tw>
+__device__ __forceinline__ void stockham_pass(const float2* src, float2* dst, int M, int Ns, float inv, Tw tw, int t0,
+                                              int T)
+{
+    const int m = M / R, stride = m / Ns;
+    for (int b = t0; b < m; b += T) stockham_butterfly<-1, R, PAD>(src, dst, Ns, inv, m, stride, tw, b);
+}
+
+// Forward transform of the workgroup's rows, threads t0 .. T-1 of each row;
+// the result is in src afterwards.  Contains the barriers.
+template <bool PAD, class Tw>
+__device__ __forceinline__ void row_dft(float2*& src, float2*& dst, const FftPlan& plan, Tw tw, int t0, int T,
+                                        bool active)
+{
+    const int M = plan.D;
+    int Ns = 1;
+    for (int s = 0; s < plan.nst; s++) {
+        const int r = plan.radix[s];
+        const float inv = plan.inv[s];
+        if (active) {
+            if (r == 8) stockham_pass<8, PAD>(src, dst, M, Ns, inv, tw, t0, T);
+            else if (r == 4) stockham_pass<4, PAD>(src, dst, M, Ns, inv, tw, t0, T);
+            else if (r == 2) stockham_pass<2, PAD>(src, dst, M, Ns, inv, tw, t0, T);
+            else if constexpr (!PAD) {   // 5 and 3 come first in a plan, which is then not padded
+                if (r == 5) stockham_pass<5, PAD>(src, dst, M, Ns, inv, tw, t0, T);
+                else stockham_pass<3, PAD>(src, dst, M, Ns, inv, tw, t0, T);
+            }
+        }
+        Ns *= r;
+        float2* t = src; src = dst; dst = t;
+        __syncthreads();
+    }
+}
+
+// Threads that share a row of the LDS kernels, one radix-5 or radix-8
+// butterfly each or a few, and whether the twiddles are copied to LDS (a
+// gather from LDS costs less than one through the vector caches; beyond 1024
+// entries the space is worth more).
+template <int T>
+constexpr bool kTwInLds = T <= 128;
+__host__ inline int row_threads(int M) { return M <= 256 ? 64 : (M <= 1024 ? 128 : 256); }
+inline bool row_padded(const FftPlan& p) { return p.nst > 0 && p.radix[0] != 5 && p.radix[0] != 3; }
+// LDS of `slots` rows (two buffers each) and the twiddles.
+inline size_t row_lds(const FftPlan& p, int slots)
+{
+    const int M = p.D, rp = row_padded(p) ? row_index<true>(M) : M;
+    return ((size_t)slots * 2 * rp + (row_threads(M) <= 128 ? M : 0)) * sizeof(float2);
 }
 
 // The rows of one FFT-filter launch: row r is row r % per of frame r / per,
@@ -148,62 +207,56 @@ struct RowFrames {
 // The transform length M = plan.D is D itself, or (for lengths the radices
 // do not factor) an M >= 2D - 1 over which the length-D circular convolution
 // is exact: the row is zero-padded to M, H is the response of the wrapped
-// circulant on M points, and the first D outputs are kept.  A workgroup of
-// blockDim.x / 128 slots holds one row pair per slot.
-__global__ void __launch_bounds__(256) fft_filter_kernel(RowFrames fr, uint16_t* __restrict__ out16, float out_scale,
-                                                         const float2* __restrict__ tw, const float* __restrict__ H,
-                                                         FftPlan plan, int D, long rows)
+// circulant on M points, and the first D outputs are kept.
+// One workgroup of T threads per row pair: latency bound (a chain of
+// 2 x 3 or 4 LDS passes), so as many workgroups as there are pairs.  The
+// inverse transform runs the forward passes with real and imaginary parts
+// exchanged, which halves the code.  2160 rows of 500: 11.9 us, 34.9 with
+// radices up to 5 chosen at run time and pairs of rows per workgroup; 8000
+// rows of 256: 27.3 us, 62 (beside another lane's backprojection).
+template <int T, bool PAD>
+__global__ void __launch_bounds__(T) fft_filter_kernel(RowFrames fr, uint16_t* __restrict__ out16, float out_scale,
+                                                       const float2* __restrict__ tw, const float* __restrict__ H,
+                                                       FftPlan plan, int D, long rows)
 {
     extern __shared__ float2 lds[];
-    const int M = plan.D;
-    const int T = 128;
-    const int slots = blockDim.x / T;
-    const int slot = threadIdx.x / T;
-    const int t0 = threadIdx.x % T;
-    const long pair = (long)blockIdx.x * slots + slot;
-    const long ra = pair * 2, rb = pair * 2 + 1;
-    float2* b0 = lds + (size_t)slot * 2 * M;
-    float2* b1 = b0 + M;
-    const bool active = ra < rows;
+    const int M = plan.D, t0 = threadIdx.x;
+    const long ra = (long)blockIdx.x * 2, rb = ra + 1;
+    float2* b0 = lds;
+    float2* b1 = b0 + row_index<PAD>(M);
+    float2* twl = b1 + row_index<PAD>(M);
     const bool hasb = rb < rows;
     const int fa = (int)(ra / fr.per), fb = hasb ? (int)(rb / fr.per) : fa;
     const long qa = ra - (long)fa * fr.per, qb = rb - (long)fb * fr.per;
-    if (active) {
-        const float* xa = fr.in[fa] + qa * D;
-        const float* xb = fr.in[fb] + qb * D;
-        for (int n = t0; n < D; n += T) b0[n] = make_float2(xa[n], hasb ? xb[n] : 0.0f);
-        for (int n = D + t0; n < M; n += T) b0[n] = make_float2(0.0f, 0.0f);
-    }
+    const float* xa = fr.in[fa] + qa * D;
+    const float* xb = fr.in[fb] + qb * D;
+    if (kTwInLds<T>)
+        for (int n = t0; n < M; n += T) twl[n] = tw[n];
+    for (int n = t0; n < D; n += T) b0[row_index<PAD>(n)] = make_float2(xa[n], hasb ? xb[n] : 0.0f);
+    for (int n = D + t0; n < M; n += T) b0[row_index<PAD>(n)] = make_float2(0.0f, 0.0f);
     __syncthreads();
     float2* src = b0;
     float2* dst = b1;
-    int Ns = 1;
-    for (int s = 0; s < plan.nst; s++) {
-        if (active) stockham_pass<-1>(src, dst, M, plan.radix[s], Ns, tw, t0, T);
-        Ns *= plan.radix[s];
-        float2* t = src; src = dst; dst = t;
-        __syncthreads();
+    for (int dir = 0; dir < 2; dir++) {
+        if constexpr (kTwInLds<T>) row_dft<PAD>(src, dst, plan, (const float2*)twl, t0, T, true);
+        else row_dft<PAD>(src, dst, plan, tw, t0, T, true);
+        if (dir == 0) {
+            for (int k = t0; k < M; k += T) {
+                const float2 z = src[row_index<PAD>(k)];
+                src[row_index<PAD>(k)] = make_float2(z.y * H[k], z.x * H[k]);
+            }
+            __syncthreads();
+        }
     }
-    if (active)
-        for (int k = t0; k < M; k += T) src[k] = cscale(src[k], H[k]);
-    __syncthreads();
-    Ns = 1;
-    for (int s = 0; s < plan.nst; s++) {
-        if (active) stockham_pass<+1>(src, dst, M, plan.radix[s], Ns, tw, t0, T);
-        Ns *= plan.radix[s];
-        float2* t = src; src = dst; dst = t;
-        __syncthreads();
-    }
-    if (!active) return;
     for (int n = t0; n < D; n += T) {
-        const float2 v = src[n];
+        const float2 v = src[row_index<PAD>(n)];   // (imaginary, real)
         if (fr.has_out) {
-            fr.out[fa][qa * D + n] = v.x;
-            if (hasb) fr.out[fb][qb * D + n] = v.y;
+            fr.out[fa][qa * D + n] = v.y;
+            if (hasb) fr.out[fb][qb * D + n] = v.x;
         }
         if (out16) {
-            out16[ra * D + n] = float_to_half_bits(v.x * out_scale);
-            if (hasb) out16[rb * D + n] = float_to_half_bits(v.y * out_scale);
+            out16[ra * D + n] = float_to_half_bits(v.y * out_scale);
+            if (hasb) out16[rb * D + n] = float_to_half_bits(v.x * out_scale);
         }
     }
 }
@@ -212,7 +265,7 @@ __global__ void __launch_bounds__(256) fft_filter_kernel(RowFrames fr, uint16_t*
 // filter with each Stockham pass a launch over a chunk of row pairs held in
 // global memory, buf[y][0..M) for pair pair0 + y (grid y = pairs in the
 // chunk, every one of them < (rows + 1) / 2).  Same butterflies, twiddles and
-// response as fft_filter_kernel, so both paths give the same values.
+// response as fft_filter_kernel.
 struct PairRows {
     long ra, rb;
     int fa, fb;
@@ -248,11 +301,18 @@ template <int S>
 __global__ void __launch_bounds__(256) fftg_pass_kernel(const float2* __restrict__ src, float2* __restrict__ dst,
                                                         int M, int r, int Ns, const float2* __restrict__ tw)
 {
-    const int m = M / r;
+    const int m = M / r, stride = m / Ns;
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= m) return;
     const size_t off = (size_t)blockIdx.y * M;
-    stockham_butterfly<S>(src + off, dst + off, r, Ns, m, M / (Ns * r), tw, b);
+    const float inv = 1.0f / (float)Ns;
+    src += off;
+    dst += off;
+    if (r == 8) stockham_butterfly<S, 8, false>(src, dst, Ns, inv, m, stride, tw, b);
+    else if (r == 5) stockham_butterfly<S, 5, false>(src, dst, Ns, inv, m, stride, tw, b);
+    else if (r == 4) stockham_butterfly<S, 4, false>(src, dst, Ns, inv, m, stride, tw, b);
+    else if (r == 3) stockham_butterfly<S, 3, false>(src, dst, Ns, inv, m, stride, tw, b);
+    else stockham_butterfly<S, 2, false>(src, dst, Ns, inv, m, stride, tw, b);
 }
 
 __global__ void __launch_bounds__(256) fftg_scale_kernel(float2* __restrict__ buf, const float* __restrict__ H, int M)
@@ -286,6 +346,14 @@ __global__ void __launch_bounds__(256) fftg_store_kernel(RowFrames fr, const flo
 // leave the spectrum in the same lane / register distribution as the input,
 // so H multiplies in place and the inverse runs the same stages with
 // conjugate twiddles.  tw[n] = e^{-2 pi i n / 512}.
+// buf belongs to the wave, whose LDS accesses complete in order: the syncs only
+// keep the compiler from moving them.
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 template <int S>
 __device__ __forceinline__ void fft512_pass(float2 (&v)[8], float2* buf, const float2 (&w1)[8],
                                             const float2 (&w2)[8], int L)
@@ -296,7 +364,7 @@ __device__ __forceinline__ void fft512_pass(float2 (&v)[8], float2* buf, const f
     for (int k = 1; k < 8; k++) v[k] = cmul(v[k], S < 0 ? w1[k] : make_float2(w1[k].x, -w1[k].y));
 #pragma unroll
     for (int k = 0; k < 8; k++) buf[k * 65 + L] = v[k];
-    __syncthreads();
+    wave_sync();
     {
         // stage 2 (lane a + 8 k0): DFT over b, times w64^{a k1}
         const int a = L & 7, k0 = L >> 3;
@@ -305,11 +373,11 @@ __device__ __forceinline__ void fft512_pass(float2 (&v)[8], float2* buf, const f
         dft8<S>(v);
 #pragma unroll
         for (int k = 1; k < 8; k++) v[k] = cmul(v[k], S < 0 ? w2[k] : make_float2(w2[k].x, -w2[k].y));
-        __syncthreads();
+        wave_sync();
 #pragma unroll
         for (int k = 0; k < 8; k++) buf[(k0 * 8 + k) * 9 + a] = v[k];
     }
-    __syncthreads();
+    wave_sync();
     {
         // stage 3 (lane k0 + 8 k1): DFT over a -> X[L + 64 k2]
         const int k0 = L & 7, k1 = L >> 3;
@@ -317,7 +385,7 @@ __device__ __forceinline__ void fft512_pass(float2 (&v)[8], float2* buf, const f
         for (int a = 0; a < 8; a++) v[a] = buf[(k0 * 8 + k1) * 9 + a];
         dft8<S>(v);
     }
-    __syncthreads();
+    wave_sync();
 }
 
 __global__ void __launch_bounds__(64) fft512_filter_kernel(RowFrames fr, uint16_t* __restrict__ out16, float out_scale,
@@ -365,102 +433,185 @@ __global__ void __launch_bounds__(64) fft512_filter_kernel(RowFrames fr, uint16_
 // Gradient w.r.t. the taps: for each row slot the complex row is
 // z = x + i sigma g (one row); X[k] = (Z[k] + conj Z[D-k]) / 2,
 // G[k] = (Z[k] - conj Z[D-k]) / 2i, contribution Re(conj(G[k]) X[k]).
+// x and g can differ in magnitude by many orders (g is a loss gradient): g is
+// scaled by a power of two sigma = 2^e that brings its row maximum to x's, or
+// the rounding of X would swamp G in the shared complex transform.
 // A fixed grid walks the rows (workgroup b takes rows b*slots + slot,
 // advancing by grid*slots, in order) and keeps its sums in registers:
 // partial[blockIdx.x][k], so the partial buffer is sized once, not per call.
-// D = plan.D <= 2048.
 constexpr int kTapBlocks = 512;
-constexpr int kTapPer = 9;   // taps per thread: ceil((2048 / 2 + 1) / 128)
-__global__ void __launch_bounds__(256) fft_grad_taps_kernel(const float* __restrict__ x, const float* __restrict__ g,
-                                                            const float2* __restrict__ tw, FftPlan plan, long rows,
-                                                            float* __restrict__ partial)
+constexpr int kTapThreads = 512;   // at most, per workgroup
+
+__device__ __forceinline__ int grad_exponent(float ax, float ag)
 {
+    return ax > 0.0f && ag > 0.0f ? max(-100, min(100, ilogbf(ax) - ilogbf(ag))) : 0;
+}
+
+// Loads row r (slot's rows x, g) zero-padded to M into b0 with g scaled, and
+// transforms it; src is the spectrum.  Contains the barriers.
+template <int T, bool PAD>
+__device__ __forceinline__ int grad_row(const float* __restrict__ x, const float* __restrict__ g,
+                                        const float2* __restrict__ tw, const float2* twl, const FftPlan& plan, int D,
+                                        long r, bool active, unsigned (*amax)[2], int slot, int t0, float2*& src,
+                                        float2*& dst)
+{
+    const int M = plan.D;
+    if (t0 < 2) amax[slot][t0] = 0u;
+    __syncthreads();
+    float mx = 0.0f, mg = 0.0f;
+    if (active) {
+        for (int n = t0; n < D; n += T) {
+            const float xv = x[r * D + n], gv = g[r * D + n];
+            src[row_index<PAD>(n)] = make_float2(xv, gv);
+            mx = fmaxf(mx, fabsf(xv));
+            mg = fmaxf(mg, fabsf(gv));
+        }
+        for (int n = D + t0; n < M; n += T) src[row_index<PAD>(n)] = make_float2(0.0f, 0.0f);
+    }
+    atomicMax(&amax[slot][0], __float_as_uint(mx));
+    atomicMax(&amax[slot][1], __float_as_uint(mg));
+    __syncthreads();
+    const int e = grad_exponent(__uint_as_float(amax[slot][0]), __uint_as_float(amax[slot][1]));
+    if (active && e != 0)
+        for (int n = t0; n < D; n += T) src[row_index<PAD>(n)].y = ldexpf(src[row_index<PAD>(n)].y, e);
+    __syncthreads();
+    if constexpr (kTwInLds<T>) row_dft<PAD>(src, dst, plan, twl, t0, T, active);
+    else row_dft<PAD>(src, dst, plan, tw, t0, T, active);
+    return e;
+}
+
+// D = plan.D <= 2048, T threads per row.
+template <int T, bool PAD>
+__global__ void __launch_bounds__(kTapThreads) fft_grad_taps_kernel(const float* __restrict__ x,
+                                                                    const float* __restrict__ g,
+                                                                    const float2* __restrict__ tw, FftPlan plan,
+                                                                    long rows, float* __restrict__ partial)
+{
+    constexpr int PER = (T == 64 ? 256 : T == 128 ? 1024 : 2048) / 2 / T + 1;   // taps per thread
     extern __shared__ float2 lds[];
-    const int D = plan.D, K = D / 2 + 1;
-    const int T = 128;
-    const int slots = blockDim.x / T;
-    const int slot = threadIdx.x / T;
-    const int t0 = threadIdx.x % T;
-    float2* b0 = lds + (size_t)slot * 2 * D;
-    float2* b1 = b0 + D;
-    __shared__ unsigned int amax[2][2];
-    float acc[kTapPer];
+    __shared__ unsigned int amax[kTapThreads / T][2];
+    const int D = plan.D, K = D / 2 + 1, slots = blockDim.x / T, slot = threadIdx.x / T, t0 = threadIdx.x % T;
+    float2* b0 = lds + (size_t)slot * 2 * row_index<PAD>(D);
+    float2* b1 = b0 + row_index<PAD>(D);
+    float2* twl = lds + (size_t)slots * 2 * row_index<PAD>(D);
+    if (kTwInLds<T>)
+        for (int n = threadIdx.x; n < D; n += blockDim.x) twl[n] = tw[n];
+    float acc[PER];
 #pragma unroll
-    for (int u = 0; u < kTapPer; u++) acc[u] = 0.0f;
+    for (int u = 0; u < PER; u++) acc[u] = 0.0f;
     for (long r0 = (long)blockIdx.x * slots; r0 < rows; r0 += (long)gridDim.x * slots) {
         const long r = r0 + slot;
         const bool active = r < rows;
-        // x and g can differ in magnitude by many orders (g is a loss
-        // gradient): g is scaled by a power of two sigma that brings its row
-        // maximum to x's, or the rounding of X would swamp G in the shared
-        // complex transform
-        if (threadIdx.x < 4) amax[threadIdx.x / 2][threadIdx.x % 2] = 0u;
-        __syncthreads();
-        float mx = 0.0f, mg = 0.0f;
-        if (active)
-            for (int n = t0; n < D; n += T) {
-                const float xv = x[r * D + n], gv = g[r * D + n];
-                b0[n] = make_float2(xv, gv);
-                mx = fmaxf(mx, fabsf(xv));
-                mg = fmaxf(mg, fabsf(gv));
-            }
-        atomicMax(&amax[slot][0], __float_as_uint(mx));
-        atomicMax(&amax[slot][1], __float_as_uint(mg));
-        __syncthreads();
-        int e = 0;
-        {
-            const float ax = __uint_as_float(amax[slot][0]), ag = __uint_as_float(amax[slot][1]);
-            if (ax > 0.0f && ag > 0.0f) e = max(-100, min(100, ilogbf(ax) - ilogbf(ag)));
-        }
-        if (active && e != 0)
-            for (int n = t0; n < D; n += T) b0[n].y = ldexpf(b0[n].y, e);
-        __syncthreads();
         float2* src = b0;
         float2* dst = b1;
-        int Ns = 1;
-        for (int s = 0; s < plan.nst; s++) {
-            if (active) stockham_pass<-1>(src, dst, D, plan.radix[s], Ns, tw, t0, T);
-            Ns *= plan.radix[s];
-            float2* t = src; src = dst; dst = t;
-            __syncthreads();
-        }
+        const int e = grad_row<T, PAD>(x, g, tw, twl, plan, D, r, active, amax, slot, t0, src, dst);
         if (active) {
 #pragma unroll
-            for (int u = 0; u < kTapPer; u++) {
+            for (int u = 0; u < PER; u++) {
                 const int k = t0 + u * T;
                 if (k >= K) break;
-                const float2 zk = src[k];
-                const float2 zm = src[(D - k) % D];
+                const float2 zk = src[row_index<PAD>(k)];
+                const float2 zm = src[row_index<PAD>(k == 0 ? 0 : D - k)];
                 const float2 X = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
                 const float2 G = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
                 acc[u] += ldexpf(G.x * X.x + G.y * X.y, -e);
             }
         }
-        __syncthreads();   // the next pair overwrites b0 / b1
+        __syncthreads();   // the next row overwrites b0 / b1
     }
-    // two slots' sums through LDS (slot 1 writes, slot 0 adds)
+    // the slots' sums through LDS, added in slot order
     float* red = reinterpret_cast<float*>(lds);
-    if (slots == 2) {
-        if (slot == 1)
 #pragma unroll
-            for (int u = 0; u < kTapPer; u++) {
-                const int k = t0 + u * T;
-                if (k < K) red[k] = acc[u];
-            }
-        __syncthreads();
+    for (int u = 0; u < PER; u++) {
+        const int k = t0 + u * T;
+        if (k < K) red[slot * K + k] = acc[u];
     }
-    if (slot == 0)
-#pragma unroll
-        for (int u = 0; u < kTapPer; u++) {
-            const int k = t0 + u * T;
-            if (k < K) partial[(long)blockIdx.x * K + k] = slots == 2 ? acc[u] + red[k] : acc[u];
-        }
+    __syncthreads();
+    for (int k = threadIdx.x; k < K; k += blockDim.x) {
+        float v = red[k];
+        for (int q = 1; q < slots; q++) v += red[q * K + k];
+        partial[(long)blockIdx.x * K + k] = v;
+    }
 }
 
-// Row slots per workgroup of the FFT kernels: two while their buffers (two
-// per slot, M complex entries each) and a little static LDS fit 64 KB, else
-// one (gfx950 gives a workgroup up to 160 KB).
-inline int fft_slots(int M) { return (size_t)2 * 2 * M * sizeof(float2) + 64 <= 64 * 1024 ? 2 : 1; }
+// The same for D = 512, one row per wave in registers (fft512_pass): lane L
+// holds bins L + 64 c, whose mirror images 512 - k lie in lane 64 - L, element
+// 7 - c.  No barriers and three LDS transposes per row: 11520 rows 14 us, 167
+// with the passes above at radices up to 4.
+constexpr int kTap512Waves = 8;
+__global__ void __launch_bounds__(64 * kTap512Waves) fft512_grad_taps_kernel(const float* __restrict__ x,
+                                                                            const float* __restrict__ g,
+                                                                            const float2* __restrict__ tw, long rows,
+                                                                            float* __restrict__ partial)
+{
+    __shared__ float2 bufs[kTap512Waves][576];
+    const int L = threadIdx.x % 64, wave = threadIdx.x / 64;
+    float2* buf = bufs[wave];
+    float2 w1[8], w2[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        w1[k] = tw[L * k];
+        w2[k] = tw[(8 * (L & 7) * k) & 511];
+    }
+    float acc[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};   // taps L + 64 u; tap 256 in lane 0
+    for (long r = (long)blockIdx.x * kTap512Waves + wave; r < rows; r += (long)gridDim.x * kTap512Waves) {
+        float2 v[8];
+        float mx = 0.0f, mg = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            v[c] = make_float2(x[r * 512 + L + 64 * c], g[r * 512 + L + 64 * c]);
+            mx = fmaxf(mx, fabsf(v[c].x));
+            mg = fmaxf(mg, fabsf(v[c].y));
+        }
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) {
+            mx = fmaxf(mx, __shfl_xor(mx, w));
+            mg = fmaxf(mg, __shfl_xor(mg, w));
+        }
+        const int e = grad_exponent(mx, mg);
+#pragma unroll
+        for (int c = 0; c < 8; c++) v[c].y = ldexpf(v[c].y, e);
+        fft512_pass<-1>(v, buf, w1, w2, L);
+#pragma unroll
+        for (int u = 0; u < 5; u++) {
+            float2 zm;   // bin (512 - (L + 64 u)) mod 512
+            if (u < 4) {
+                zm.x = __shfl(v[7 - u].x, (64 - L) & 63);
+                zm.y = __shfl(v[7 - u].y, (64 - L) & 63);
+                if (L == 0) zm = v[(8 - u) & 7];
+            } else {
+                zm = v[4];   // lane 0: bin 256 is its own mirror image
+            }
+            const float2 zk = v[u];
+            const float2 X = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
+            const float2 G = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
+            acc[u] += ldexpf(G.x * X.x + G.y * X.y, -e);
+        }
+    }
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(&bufs[0][0]);   // [wave][257]
+#pragma unroll
+    for (int u = 0; u < 5; u++)
+        if (u < 4 || L == 0) red[wave * 257 + L + 64 * u] = acc[u];
+    __syncthreads();
+    for (int k = threadIdx.x; k < 257; k += 64 * kTap512Waves) {
+        float s = red[k];
+#pragma unroll
+        for (int w = 1; w < kTap512Waves; w++) s += red[w * 257 + k];
+        partial[(long)blockIdx.x * 257 + k] = s;
+    }
+}
+
+// Row slots per workgroup of the gradient kernels: up to kTapThreads threads
+// within 64 KB, fewer where kTapBlocks workgroups already cover the rows.
+inline int grad_slots(const FftPlan& p, long rows)
+{
+    const int T = row_threads(p.D);
+    int slots = 1;
+    while (slots * 2 * T <= kTapThreads && row_lds(p, slots * 2) <= 64 * 1024 && (long)slots * kTapBlocks < rows)
+        slots *= 2;
+    return slots;
+}
 
 // One workgroup per tap k: thread t sums partials t, t + 256, ... in order,
 // then a fixed LDS tree -- deterministic, and no thread walks all partials.
@@ -491,65 +642,38 @@ __global__ void __launch_bounds__(256) reduce_taps_kernel(const float* __restric
 // (|j| < D) has the spectrum G(k) conj(X(k)); the spectra are summed over rows
 // (fixed grid, registers, then a fixed-order reduction), transformed back
 // once, wrapped to R[d] = r_lin[d] + r_lin[d - D], and cosine-transformed.
-constexpr int kXspecPer = 17;   // bins per thread: ceil((4096 / 2 + 1) / 128)
-__global__ void __launch_bounds__(256) fft_xspec_kernel(const float* __restrict__ x, const float* __restrict__ g,
-                                                        const float2* __restrict__ tw, FftPlan plan, int D, long rows,
-                                                        float2* __restrict__ partial)
+// M = plan.D <= 4096, T threads per row.
+template <int T, bool PAD>
+__global__ void __launch_bounds__(kTapThreads) fft_xspec_kernel(const float* __restrict__ x,
+                                                                const float* __restrict__ g,
+                                                                const float2* __restrict__ tw, FftPlan plan, int D,
+                                                                long rows, float2* __restrict__ partial)
 {
+    constexpr int PER = (T == 64 ? 256 : T == 128 ? 1024 : 4096) / 2 / T + 1;   // bins per thread
     extern __shared__ float2 lds[];
-    const int M = plan.D, K = M / 2 + 1;
-    const int T = 128;
-    const int slots = blockDim.x / T;
-    const int slot = threadIdx.x / T;
-    const int t0 = threadIdx.x % T;
-    float2* b0 = lds + (size_t)slot * 2 * M;
-    float2* b1 = b0 + M;
-    __shared__ unsigned int amax[2][2];
-    float2 acc[kXspecPer];
+    __shared__ unsigned int amax[kTapThreads / T][2];
+    const int M = plan.D, K = M / 2 + 1, slots = blockDim.x / T, slot = threadIdx.x / T, t0 = threadIdx.x % T;
+    float2* b0 = lds + (size_t)slot * 2 * row_index<PAD>(M);
+    float2* b1 = b0 + row_index<PAD>(M);
+    float2* twl = lds + (size_t)slots * 2 * row_index<PAD>(M);
+    if (kTwInLds<T>)
+        for (int n = threadIdx.x; n < M; n += blockDim.x) twl[n] = tw[n];
+    float2 acc[PER];
 #pragma unroll
-    for (int u = 0; u < kXspecPer; u++) acc[u] = make_float2(0.0f, 0.0f);
+    for (int u = 0; u < PER; u++) acc[u] = make_float2(0.0f, 0.0f);
     for (long r0 = (long)blockIdx.x * slots; r0 < rows; r0 += (long)gridDim.x * slots) {
         const long r = r0 + slot;
         const bool active = r < rows;
-        if (threadIdx.x < 4) amax[threadIdx.x / 2][threadIdx.x % 2] = 0u;
-        __syncthreads();
-        float mx = 0.0f, mg = 0.0f;
-        if (active) {
-            for (int n = t0; n < D; n += T) {
-                const float xv = x[r * D + n], gv = g[r * D + n];
-                b0[n] = make_float2(xv, gv);
-                mx = fmaxf(mx, fabsf(xv));
-                mg = fmaxf(mg, fabsf(gv));
-            }
-            for (int n = D + t0; n < M; n += T) b0[n] = make_float2(0.0f, 0.0f);
-        }
-        atomicMax(&amax[slot][0], __float_as_uint(mx));
-        atomicMax(&amax[slot][1], __float_as_uint(mg));
-        __syncthreads();
-        int e = 0;
-        {
-            const float ax = __uint_as_float(amax[slot][0]), ag = __uint_as_float(amax[slot][1]);
-            if (ax > 0.0f && ag > 0.0f) e = max(-100, min(100, ilogbf(ax) - ilogbf(ag)));
-        }
-        if (active && e != 0)
-            for (int n = t0; n < D; n += T) b0[n].y = ldexpf(b0[n].y, e);
-        __syncthreads();
         float2* src = b0;
         float2* dst = b1;
-        int Ns = 1;
-        for (int s = 0; s < plan.nst; s++) {
-            if (active) stockham_pass<-1>(src, dst, M, plan.radix[s], Ns, tw, t0, T);
-            Ns *= plan.radix[s];
-            float2* t = src; src = dst; dst = t;
-            __syncthreads();
-        }
+        const int e = grad_row<T, PAD>(x, g, tw, twl, plan, D, r, active, amax, slot, t0, src, dst);
         if (active) {
 #pragma unroll
-            for (int u = 0; u < kXspecPer; u++) {
+            for (int u = 0; u < PER; u++) {
                 const int k = t0 + u * T;
                 if (k >= K) break;
-                const float2 zk = src[k];
-                const float2 zm = src[(M - k) % M];
+                const float2 zk = src[row_index<PAD>(k)];
+                const float2 zm = src[row_index<PAD>(k == 0 ? 0 : M - k)];
                 const float2 X = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
                 const float2 G = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
                 // G conj(X), G carrying sigma = 2^e
@@ -560,25 +684,27 @@ __global__ void __launch_bounds__(256) fft_xspec_kernel(const float* __restrict_
         __syncthreads();
     }
     float2* red = lds;
-    if (slots == 2) {
-        if (slot == 1)
 #pragma unroll
-            for (int u = 0; u < kXspecPer; u++) {
-                const int k = t0 + u * T;
-                if (k < K) red[k] = acc[u];
-            }
-        __syncthreads();
+    for (int u = 0; u < PER; u++) {
+        const int k = t0 + u * T;
+        if (k < K) red[slot * K + k] = acc[u];
     }
-    if (slot == 0)
-#pragma unroll
-        for (int u = 0; u < kXspecPer; u++) {
-            const int k = t0 + u * T;
-            if (k >= K) break;
-            float2 v = acc[u];
-            if (slots == 2) v = make_float2(v.x + red[k].x, v.y + red[k].y);
-            partial[(long)blockIdx.x * K + k] = v;
-        }
+    __syncthreads();
+    for (int k = threadIdx.x; k < K; k += blockDim.x) {
+        float2 v = red[k];
+        for (int q = 1; q < slots; q++) v = cadd(v, red[q * K + k]);
+        partial[(long)blockIdx.x * K + k] = v;
+    }
 }
+
+// fn<T, PAD> of a row kernel for the plan.
+#define RISA_ROW_KERNEL(fn, p)                                              \
+    (row_padded(p) ? (row_threads((p).D) == 64    ? fn<64, true>            \
+                      : row_threads((p).D) == 128 ? fn<128, true>           \
+                                                  : fn<256, true>)          \
+                   : (row_threads((p).D) == 64    ? fn<64, false>           \
+                      : row_threads((p).D) == 128 ? fn<128, false>          \
+                                                  : fn<256, false>))
 
 // The tail of the padded tap gradient: three short sums, each bound by the
 // latency of its serial chain, so each is spread over a workgroup and added up
@@ -1037,10 +1163,18 @@ static bool make_plan(int D, FftPlan& p)
     p.D = D;
     p.nst = 0;
     int n = D;
+    // odd radices first (their strides spread over the LDS banks), then as few
+    // passes as the powers of two allow: 8s, and 4 4 rather than 8 2
+    while (n % 5 == 0 && p.nst < 24) { p.radix[p.nst++] = 5; n /= 5; }
+    while (n % 3 == 0 && p.nst < 24) { p.radix[p.nst++] = 3; n /= 3; }
+    while (n % 8 == 0 && n != 16 && p.nst < 24) { p.radix[p.nst++] = 8; n /= 8; }
     while (n % 4 == 0 && p.nst < 24) { p.radix[p.nst++] = 4; n /= 4; }
     while (n % 2 == 0 && p.nst < 24) { p.radix[p.nst++] = 2; n /= 2; }
-    while (n % 3 == 0 && p.nst < 24) { p.radix[p.nst++] = 3; n /= 3; }
-    while (n % 5 == 0 && p.nst < 24) { p.radix[p.nst++] = 5; n /= 5; }
+    int Ns = 1;
+    for (int s = 0; s < p.nst; s++) {
+        p.inv[s] = 1.0f / (float)Ns;
+        Ns *= p.radix[s];
+    }
     return n == 1;
 }
 
@@ -1279,11 +1413,8 @@ static void launch_fft(risa_filter_t h, const RowFrames& fr, uint16_t* out16, fl
         check_launch("fft512_filter_kernel");
         return;
     }
-    const int slots = fft_slots(M);
-    const int grid = ceil_div(pairs, slots);
-    const size_t lds = (size_t)slots * 2 * M * sizeof(float2);
-    hipLaunchKernelGGL(fft_filter_kernel, dim3(grid), dim3(128 * slots), lds, s, fr, out16, out_scale, h->tw.ptr,
-                       h->H.ptr, h->plan, D, rows);
+    hipLaunchKernelGGL(RISA_ROW_KERNEL(fft_filter_kernel, h->plan), dim3((unsigned)pairs), dim3(row_threads(M)),
+                       row_lds(h->plan, 1), s, fr, out16, out_scale, h->tw.ptr, h->H.ptr, h->plan, D, rows);
     check_launch("fft_filter_kernel");
 }
 // `rows` consecutive rows in -> out (out null: FP16 output only).
@@ -1445,11 +1576,10 @@ static void launch_grad_taps_padded(risa_filter_t h, const float* x, const float
                                     float* dtaps, const GradScratch& sc, hipStream_t s)
 {
     const int D = h->g.numberOfParallelDetectors, M = h->M, KM = M / 2 + 1;
-    const int slots = fft_slots(M);
-    const size_t lds = (size_t)slots * 2 * M * sizeof(float2);
+    const int slots = grad_slots(h->plan, rows);
     const int grid = (int)std::max(1L, std::min<long>(nblocks, (rows + slots - 1) / slots));
-    hipLaunchKernelGGL(fft_xspec_kernel, dim3(grid), dim3(128 * slots), lds, s, x, g, h->tw.ptr, h->plan, D, rows,
-                       sc.xpart);
+    hipLaunchKernelGGL(RISA_ROW_KERNEL(fft_xspec_kernel, h->plan), dim3(grid), dim3(row_threads(M) * slots),
+                       row_lds(h->plan, slots), s, x, g, h->tw.ptr, h->plan, D, rows, sc.xpart);
     check_launch("fft_xspec_kernel");
     hipLaunchKernelGGL(xspec_reduce_kernel, dim3(ceil_div(KM, 8)), dim3(256), 0, s, sc.xpart, grid, KM, sc.xsum);
     check_launch("xspec_reduce_kernel");
@@ -1471,11 +1601,14 @@ static void grad_taps(risa_filter_t h, const float* x, const float* g, int slice
         launch_grad_taps_padded(h, x, g, rows, kTapBlocks, dtaps, sc, s);
         return;
     }
-    const int slots = fft_slots(D);
+    const int slots = D == 512 ? kTap512Waves : grad_slots(h->plan, rows);
     const int nblocks = (int)std::max(1L, std::min<long>(kTapBlocks, (rows + slots - 1) / slots));
-    const size_t lds = (size_t)slots * 2 * D * sizeof(float2);
-    hipLaunchKernelGGL(fft_grad_taps_kernel, dim3(nblocks), dim3(128 * slots), lds, s, x, g, h->tw.ptr, h->plan, rows,
-                       sc.partial);
+    if (D == 512)
+        hipLaunchKernelGGL(fft512_grad_taps_kernel, dim3(nblocks), dim3(64 * kTap512Waves), 0, s, x, g, h->tw.ptr,
+                           rows, sc.partial);
+    else
+        hipLaunchKernelGGL(RISA_ROW_KERNEL(fft_grad_taps_kernel, h->plan), dim3(nblocks), dim3(row_threads(D) * slots),
+                           row_lds(h->plan, slots), s, x, g, h->tw.ptr, h->plan, rows, sc.partial);
     check_launch("fft_grad_taps_kernel");
     hipLaunchKernelGGL(reduce_taps_kernel, dim3(K), dim3(256), 0, s, sc.partial, nblocks, K, D, dtaps);
     check_launch("reduce_taps_kernel");

@@ -1,5 +1,6 @@
-"""Tap gradient: the short sums after the row transforms, at the edges of
-their workgroups."""
+"""Row transforms of the filter and of the tap gradient at each radix, row
+width and layout, and the tap gradient's short sums at the edges of their
+workgroups."""
 from __future__ import annotations
 
 import numpy as np
@@ -38,4 +39,57 @@ def test_padded_tap_gradient_tail(risa, orc, geom_c0, cuda, D, P, S):
     flt.grad_taps(torch.from_numpy(x).to(cuda), torch.from_numpy(gr).to(cuda), 0, dt)   # no rows: zero
     torch.cuda.synchronize()
     assert float(dt.abs().max()) == 0.0
+    flt.close()
+
+
+@pytest.mark.parametrize("D", [1, 2, 3, 30, 16, 128, 250, 256, 500, 1024, 1280, 2048, 4000, 4096, 4608])
+def test_filter_row_kernels(risa, orc, geom_c0, cuda, D):
+    """The row transform at each radix, row width and LDS layout, and one
+    length beyond LDS (4608), with an odd number of rows, against numpy in
+    double.  Bound 2e-6 in the 2-norm: two transforms of at most 9 passes, each
+    rounding to a few 6e-8 (twiddle, product, sums) of the RMS, added in
+    quadrature: 3 x 6e-8 x sqrt(18) < 1e-6."""
+    import torch
+    from risa_amd import device
+
+    print(f"case: filter rows D={D}", flush=True)
+    P, S = 7, 3
+    g = geom_c0.replace(numberOfParallelDetectors=D, numberOfParallelProjections=P)
+    rng = np.random.default_rng(D)
+    x = rng.standard_normal((S, P, D)).astype(np.float32)
+    taps = (1.0 + rng.random(D // 2 + 1)).astype(np.float32)
+    flt = device.Filter(g)
+    flt.set_taps(taps)
+    t = torch.from_numpy(x.copy()).to(cuda)
+    flt(t, S)
+    torch.cuda.synchronize()
+    h = taps.astype(np.float64)
+    ref = np.fft.irfft(np.fft.rfft(x.astype(np.float64)) * h, n=D) * D if D > 1 else x.astype(np.float64) * h[0]
+    err = float(np.linalg.norm(t.cpu().numpy() - ref) / np.linalg.norm(ref))
+    print(f"  rel L2 {err:.2e}", flush=True)
+    assert err < 2e-6
+    flt.close()
+
+
+@pytest.mark.parametrize("D,rows", [(4, 3), (128, 5000), (256, 515), (500, 1100), (512, 1), (512, 5003), (1024, 700),
+                                    (2048, 9)])
+def test_tap_gradient_row_kernels(risa, orc, geom_c0, cuda, D, rows):
+    """Lengths the transform takes unpadded: each row width, one to several rows
+    per workgroup and pass, the register transform of 512; bound as above."""
+    import torch
+    from risa_amd import device
+
+    print(f"case: tap gradient D={D} rows={rows}", flush=True)
+    g = geom_c0.replace(numberOfParallelDetectors=D, numberOfParallelProjections=rows)
+    rng = np.random.default_rng(D + rows)
+    x = rng.standard_normal((1, rows, D)).astype(np.float32)
+    gr = ((rng.standard_normal((1, rows, D)) + 0.5 * x) * 1e-5).astype(np.float32)
+    flt = device.Filter(g)
+    dt = torch.full((D // 2 + 1,), float("nan"), dtype=torch.float32, device=cuda)
+    flt.grad_taps(torch.from_numpy(x).to(cuda), torch.from_numpy(gr).to(cuda), 1, dt)
+    torch.cuda.synchronize()
+    ref = orc.grad_taps_f64(x.astype(np.float64), gr.astype(np.float64))
+    err = float(np.linalg.norm(dt.cpu().numpy() - ref) / np.linalg.norm(ref))
+    print(f"  rel L2 vs FP64 oracle {err:.2e}", flush=True)
+    assert err < 1e-5
     flt.close()
