@@ -1409,6 +1409,8 @@ constexpr int kAdjWin = 72;                 // bins per band window (64 |cA| + 3
 constexpr int kAdjRec = kAdjWin + 1;        // record: kstart, then the window
 constexpr int kAdjPad = 80;                 // zero columns either side of a padded image row
 constexpr int kAdjWavesPerGroup = 8;        // angles per workgroup (one wave each), one band
+constexpr int kAdjSlices = 16;              // images per pass through the buffers, in groups of 4 and a last 2 or 1
+constexpr int kAdjPlaces = kAdjSlices + 3;  // padded copies: the groups of 4, one group of 2, one of 1
 constexpr int kAdjTab = 192;                // segment table entries per wave (64 + 64 + 1 used at most)
 
 struct AdjAngle {
@@ -1428,6 +1430,7 @@ struct AdjParams {
     double c0;            // (N - 1) / 2
     float outmul;         // norm * out_scale
     long img_stride;      // elements per padded image
+    int quads, tail;      // groups of four images of the pass, and the images of the group behind them (0 .. 2)
     int lgTX, lgTY;       // log2 of the forward tile's width / height
     int tilesX, tilesY;   // the forward's tile grid
 };
@@ -1451,33 +1454,51 @@ __global__ void adj_tile_origin_kernel(const float* __restrict__ cosT, const flo
     T[i] = -w.negT;
 }
 
-// Zero-padded, masked copies of `slices` images [N][N]: A [r][kAdjPad + x] =
-// img[r][x], B [r][kAdjPad + x] = img[x][r] (transposed), zero outside the
-// mask.  The padding columns are zeroed once at set-up and never written.
-__global__ void __launch_bounds__(256) adj_pad_kernel(const float* __restrict__ img, float* __restrict__ A,
-                                                      float* __restrict__ B, int N, int PW, int mask, float center,
-                                                      long img_stride)
+// A group of W images (4, or the pass's last 2 or 1) is stored pixel by pixel,
+// the W values side by side, so that one load fetches a pixel of all of them.
+// Groups of 4 start at kAdjSlices / 4 places of 4 image_strides; a group of 2
+// and one of 1 have places of their own behind them, since the padding columns
+// (zero from set-up) lie elsewhere for every W.
+__host__ __device__ inline long adj_group_offset(int group, int W, long img_stride)
 {
-    __shared__ float tile[32][33];
-    const int s = blockIdx.z;
-    const float* I = img + (long)s * N * N;
-    float* As = A + s * img_stride;
-    float* Bs = B + s * img_stride;
+    return (W == 4 ? 4L * group : W == 2 ? (long)kAdjSlices : (long)kAdjSlices + 2) * img_stride;
+}
+
+// Zero-padded, masked copies of a pass's images [N][N], in groups: A [r]
+// [kAdjPad + x] = img[r][x], B [r][kAdjPad + x] = img[x][r] (transposed), zero
+// outside the mask.  The padding columns are zeroed once at set-up and never
+// written.
+__global__ void __launch_bounds__(256) adj_pad_kernel(const float* __restrict__ img, int slices,
+                                                      float* __restrict__ A, float* __restrict__ B, int N, int PW,
+                                                      int mask, float center, long img_stride, int quads, int tail)
+{
+    __shared__ float4 tile[32][33];
+    const int z = blockIdx.z, W = z < quads ? 4 : tail, s0 = 4 * z;
+    const float* I = img + (long)s0 * N * N;
+    float* As = A + adj_group_offset(z, W, img_stride);
+    float* Bs = B + adj_group_offset(z, W, img_stride);
     const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
+    auto put = [&](float* out, long at, float4 v) {
+        if (W == 4) reinterpret_cast<float4*>(out)[at] = v;
+        else if (W == 2) reinterpret_cast<float2*>(out)[at] = make_float2(v.x, v.y);
+        else out[at] = v.x;
+    };
     for (int r = threadIdx.y; r < 32; r += 8) {
         const int y = by + r, x = bx + threadIdx.x;
-        float v = 0.0f;
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         if (y < N && x < N) {
-            v = I[(long)y * N + x];
-            if (mask && bp_outside(x, y, N, center)) v = 0.0f;
-            As[(long)y * PW + kAdjPad + x] = v;
+            if (!(mask && bp_outside(x, y, N, center)))
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (s0 + k < slices) v[k] = I[(long)k * N * N + (long)y * N + x];
+            put(As, (long)y * PW + kAdjPad + x, make_float4(v[0], v[1], v[2], v[3]));
         }
-        tile[r][threadIdx.x] = v;
+        tile[r][threadIdx.x] = make_float4(v[0], v[1], v[2], v[3]);
     }
     __syncthreads();
     for (int r = threadIdx.y; r < 32; r += 8) {
         const int x = bx + r, y = by + threadIdx.x;   // B row x, column y
-        if (y < N && x < N) Bs[(long)x * PW + kAdjPad + y] = tile[threadIdx.x][r];
+        if (y < N && x < N) put(Bs, (long)x * PW + kAdjPad + y, tile[threadIdx.x][r]);
     }
 }
 
@@ -1488,24 +1509,24 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// One lane's path over rows [r0, r1] of angle p (class CLS) through AS
-// images at once (rsrc[i]); returns each image's three sums.  The path, its
-// table entries, the pixel coordinate and the fraction are shared; each
-// image adds one buffer load and three accumulations per row, with the same
+// One lane's path over rows [r0, r1] of angle p (class CLS) through the AS
+// images of a group at once (rsrc); returns each image's three sums.  The
+// path, its load, table entries, the pixel coordinate and the fraction are
+// shared; each image adds three accumulations per row, with the same
 // operations as a one-image path.  tab: this wave's segment table.  rt[r] =
-// {byte offset of the path's row-r pixel of lane 0 in the padded image,
-// minus J0 * 4; delta(r) * 8}.  Rows go in blocks of 16 / AS (8 / AS where a
-// segment has fewer rows left; a partial block's spare rows add zero),
-// loads first.
+// {4 x index of the path's row-r pixel of lane 0 in the padded image, minus
+// J0 * 4; delta(r) * 8}.  Rows go in blocks of 8 (16 for one image), loads
+// first; half of that where a segment has fewer rows left (a partial block's
+// spare rows add zero).
 template <int CLS, int AS>
-__device__ __forceinline__ void adj_path(const __amdgpu_buffer_rsrc_t (&rsrc)[AS], const int2* __restrict__ rt,
+__device__ __forceinline__ void adj_path(__amdgpu_buffer_rsrc_t rsrc, const int2* __restrict__ rt,
                                          const float* __restrict__ coord, const float* __restrict__ Tp,
                                          const AdjParams& q, float2* tab, int J0, int lane, int r0, int r1, float c,
                                          float s, float A1, float (&g0)[AS], float (&gm)[AS], float (&ga)[AS])
 {
     // the segment: rows of one forward tile row (class A) or column (class B)
     const int sh = CLS ? q.lgTX : q.lgTY;
-    const int voff = lane * 4, J04 = J0 * 4;
+    const int voff = lane * 4 * AS, J04 = J0 * 4;
     const unsigned lane8 = lds_address(tab) + (unsigned)lane * 8u;
     unsigned lbase = lane8;   // lane8 - 8 * (the segment's smallest delta)
     // the row's table entry: one VALU add on a scalar byte offset (left to
@@ -1516,8 +1537,19 @@ __device__ __forceinline__ void adj_path(const __amdgpu_buffer_rsrc_t (&rsrc)[AS
         const lds_f2 w = lds_load<lds_f2>(a);
         return make_float2(w.x, w.y);
     };
-    auto load = [&](int k, int off) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc[k], voff, off + J04, 0));
+    auto load = [&](float (&v)[AS], int off) {
+        const int o = (int)((unsigned)(off + J04) * AS);
+        if constexpr (AS == 4) {
+            const f4_t w = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, o, 0));
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = w[k];
+        } else if constexpr (AS == 2) {
+            const lds_f2 w = __builtin_bit_cast(lds_f2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, voff, o, 0));
+            v[0] = w.x;
+            v[1] = w.y;
+        } else {
+            v[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff, o, 0));
+        }
     };
     auto row = [&](const float (&v)[AS], float2 e, float rc) {
         float tp, rm;
@@ -1546,11 +1578,10 @@ __device__ __forceinline__ void adj_path(const __amdgpu_buffer_rsrc_t (&rsrc)[AS
         for (int i = 0; i < NB; i++) {
             const int ri = r + min(i, live - 1);
             const int2 t = rt[ri];
+            load(v[i], t.x);
 #pragma unroll
-            for (int k = 0; k < AS; k++) {
-                v[i][k] = load(k, t.x);
+            for (int k = 0; k < AS; k++)
                 if (i >= live) v[i][k] = 0.0f;
-            }
             e[i] = entry(t.y);
             rc[i] = coord[ri];
         }
@@ -1584,7 +1615,7 @@ __device__ __forceinline__ void adj_path(const __amdgpu_buffer_rsrc_t (&rsrc)[AS
         }
         // rows left in this segment (segments are whole tile rows / columns)
         const int lim = min(r1, segend) - r + 1;
-        constexpr int BIG = 16 / AS > 4 ? 16 / AS : 4, SMALL = BIG / 2;
+        constexpr int BIG = AS == 1 ? 16 : 8, SMALL = BIG / 2;
         if (lim >= BIG) {
             block(std::integral_constant<int, BIG>{}, r, BIG);
             r += BIG;
@@ -1595,9 +1626,65 @@ __device__ __forceinline__ void adj_path(const __amdgpu_buffer_rsrc_t (&rsrc)[AS
     }
 }
 
+// The path of angle p's band b through group z's W images, and the band's
+// window of each of the first nv of them.
+template <int W>
+__device__ __forceinline__ void adj_band(const float* __restrict__ A, const float* __restrict__ B,
+                                         float* __restrict__ partial, const int2* __restrict__ rowtab, int2 rr,
+                                         const float* __restrict__ coord, const float* __restrict__ Ttab, float c,
+                                         float s, const AdjAngle& an, const AdjParams& q, int b, int z, int nv,
+                                         float2* tab, float* w, int lane)
+{
+    const int p = an.p, J0 = an.J0base + 64 * b;
+    // this lane's bins a_lo .. a_lo + 2
+    const double cAd = (double)an.cA * (double)q.scale;
+    const double base = ((double)(J0 + lane) - q.c0) * cAd;
+    const int a_lo = (int)floor(base - 0.5 * fabs(cAd));
+    const float* img = (an.cls ? B : A) + adj_group_offset(z, W, q.img_stride);
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(img), (short)0, (int)(unsigned)(q.img_stride * 4 * W), 0x00020000);
+    const int2* rt = rowtab + (long)p * q.N;
+    const float* Tp = Ttab + (long)p * q.tilesX * q.tilesY;
+    const float A1 = (float)(a_lo + 1);
+    float g0[W], gm[W], ga[W];
+#pragma unroll
+    for (int k = 0; k < W; k++) g0[k] = gm[k] = ga[k] = 0.0f;
+    if (an.cls) adj_path<1, W>(rsrc, rt, coord, Tp, q, tab, J0, lane, rr.x, rr.y, c, s, A1, g0, gm, ga);
+    else adj_path<0, W>(rsrc, rt, coord, Tp, q, tab, J0, lane, rr.x, rr.y, c, s, A1, g0, gm, ga);
+    // window of the band: the lanes' a_lo are monotone in the lane index
+    const int kstart = min(__builtin_amdgcn_readfirstlane(a_lo), __builtin_amdgcn_readlane(a_lo, 63));
+    const int wi = min(max(a_lo - kstart, 0), kAdjWin - 3);
+#pragma unroll
+    for (int k = 0; k < W; k++) {
+        if (k >= nv) break;
+        // the path's three contributions (t-bins a_lo, a_lo + 1, a_lo + 2):
+        // max(-m, 0) = (|m| - m) / 2, 1 - |m|, max(m, 0) = (|m| + m) / 2
+        const float c0v = 0.5f * (ga[k] - gm[k]), c1v = g0[k] - ga[k], c2v = 0.5f * (ga[k] + gm[k]);
+        float* rec = partial + (((long)(4 * z + k) * q.P + p) * q.nbmax + b) * kAdjRec;
+        for (int j = lane; j < kAdjWin; j += 64) w[j] = 0.0f;
+        wave_lds_sync();
+        atomicAdd(&w[wi], c0v);
+        atomicAdd(&w[wi + 1], c1v);
+        atomicAdd(&w[wi + 2], c2v);
+        wave_lds_sync();
+        if (lane == 0) rec[0] = __int_as_float(kstart);
+        for (int j = lane; j < kAdjWin; j += 64) rec[1 + j] = w[j];
+        wave_lds_sync();   // the window is read before the next image clears it
+    }
+}
+
 // Workgroup (x, y, z): kAdjWavesPerGroup angles of the sorted list, band y,
-// images AS z .. AS z + AS - 1 of the pass (those below `slices`).
-template <int AS>
+// group z of the pass: four images for z < q.quads (QUADS), the last TAIL ones
+// behind them.
+//
+// Bound by vector issue (one operation in 5.1 clocks per SIMD) and by the L1's
+// accesses (in 86% of the clocks): a row of a wave costs 4 (class A) or 5
+// operations, one load and one LDS read for the path and three operations per
+// image.  Hence four images at once (16 operations for 256 image values; two
+// at once 10 for 128), and the images stored side by side: one 16-byte load a
+// lane instead of four.  16 images of 512^2 x 720 angles: 545 us, 741 with two
+// images from separate planes; 5 images of 320^2 x 181 angles: 59 us, 76.
+template <bool QUADS, int TAIL>
 __global__ void __launch_bounds__(64 * kAdjWavesPerGroup) bp_adjoint_path_kernel(
     const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ partial,
     const AdjAngle* __restrict__ angles, const int2* __restrict__ bands, const int2* __restrict__ rowtab,
@@ -1609,7 +1696,6 @@ __global__ void __launch_bounds__(64 * kAdjWavesPerGroup) bp_adjoint_path_kernel
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int lane = threadIdx.x % 64;
     const int pos = blockIdx.x * kAdjWavesPerGroup + wave;
-    const int sl0 = blockIdx.z * AS, nv = min(AS, slices - sl0);
     if (pos >= q.npos) return;
     const AdjAngle an = angles[pos];
     if (an.p < 0 || (int)blockIdx.y >= an.nb) return;
@@ -1617,52 +1703,14 @@ __global__ void __launch_bounds__(64 * kAdjWavesPerGroup) bp_adjoint_path_kernel
     // dispatched first, the short edge bands fill in behind them
     const int i = blockIdx.y, mid = (an.nb - 1) / 2;
     const int b = (i & 1) ? mid + (i + 1) / 2 : mid - i / 2;
-    const int p = an.p;
-    const int J0 = an.J0base + 64 * b;
-    // this lane's bins a_lo .. a_lo + 2
-    const double cAd = (double)an.cA * (double)q.scale;
-    const double base = ((double)(J0 + lane) - q.c0) * cAd;
-    const int a_lo = (int)floor(base - 0.5 * fabs(cAd));
-    const int2 rr = bands[p * q.nbmax + b];
-    // images past the pass's last read the last one again and write nothing
-    __amdgpu_buffer_rsrc_t rsrc[AS];
-#pragma unroll
-    for (int k = 0; k < AS; k++) {
-        const float* img = (an.cls ? B : A) + (long)(sl0 + min(k, nv - 1)) * q.img_stride;
-        rsrc[k] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(img), (short)0, (int)(q.img_stride * 4),
-                                                    0x00020000);
-    }
-    const int2* rt = rowtab + (long)p * q.N;
-    const float* Tp = Ttab + (long)p * q.tilesX * q.tilesY;
-    const float c = cosT[p], s = sinT[p], A1 = (float)(a_lo + 1);
-    float g0[AS], gm[AS], ga[AS];
-#pragma unroll
-    for (int k = 0; k < AS; k++) g0[k] = gm[k] = ga[k] = 0.0f;
-    if (an.cls)
-        adj_path<1, AS>(rsrc, rt, coord, Tp, q, tabs[wave], J0, lane, rr.x, rr.y, c, s, A1, g0, gm, ga);
-    else
-        adj_path<0, AS>(rsrc, rt, coord, Tp, q, tabs[wave], J0, lane, rr.x, rr.y, c, s, A1, g0, gm, ga);
-    // window of the band: the lanes' a_lo are monotone in the lane index
-    const int kstart = min(__builtin_amdgcn_readfirstlane(a_lo), __builtin_amdgcn_readlane(a_lo, 63));
-    const int wi = min(max(a_lo - kstart, 0), kAdjWin - 3);
-    float* w = win[wave];
-#pragma unroll
-    for (int k = 0; k < AS; k++) {
-        if (k >= nv) break;
-        // the path's three contributions (t-bins a_lo, a_lo + 1, a_lo + 2):
-        // max(-m, 0) = (|m| - m) / 2, 1 - |m|, max(m, 0) = (|m| + m) / 2
-        const float c0v = 0.5f * (ga[k] - gm[k]), c1v = g0[k] - ga[k], c2v = 0.5f * (ga[k] + gm[k]);
-        float* rec = partial + (((long)(sl0 + k) * q.P + p) * q.nbmax + b) * kAdjRec;
-        for (int j = lane; j < kAdjWin; j += 64) w[j] = 0.0f;
-        wave_lds_sync();
-        atomicAdd(&w[wi], c0v);
-        atomicAdd(&w[wi + 1], c1v);
-        atomicAdd(&w[wi + 2], c2v);
-        wave_lds_sync();
-        if (lane == 0) rec[0] = __int_as_float(kstart);
-        for (int j = lane; j < kAdjWin; j += 64) rec[1 + j] = w[j];
-        wave_lds_sync();   // the window is read before the next image clears it
-    }
+    const int2 rr = bands[an.p * q.nbmax + b];
+    const float c = cosT[an.p], s = sinT[an.p];
+    const int z = blockIdx.z;
+    if (QUADS && z < q.quads)
+        adj_band<4>(A, B, partial, rowtab, rr, coord, Ttab, c, s, an, q, b, z, min(4, slices - 4 * z), tabs[wave],
+                    win[wave], lane);
+    else if constexpr (TAIL != 0)
+        adj_band<TAIL>(A, B, partial, rowtab, rr, coord, Ttab, c, s, an, q, b, z, TAIL, tabs[wave], win[wave], lane);
 }
 
 // sino[s][a][k] = outmul * sum over the angle's bands (in band order) of the
@@ -1832,7 +1880,7 @@ struct risa_bp_s {
     risa::DeviceBuffer<int2> adj_rows;       // [P][N] {(r * PW + pad + delta(r)) * 4, delta(r) * 8}
     risa::DeviceBuffer<int2> adj_bands;      // [P][nbmax] {first row, last row}
     risa::DeviceBuffer<int> adj_nb;          // [P]
-    risa::DeviceBuffer<float> adj_imgA, adj_imgB;   // [kAdjSlices][N][PW] padded, masked copies
+    risa::DeviceBuffer<float> adj_imgA, adj_imgB;   // [kAdjPlaces][N][PW] padded, masked copies, in groups
     risa::DeviceBuffer<float> adj_partial;   // [kAdjSlices][P][nbmax][kAdjRec]
     risa::DeviceBuffer<float> adj_T;         // [P][tilesY][tilesX] the forward's tile origins (variant in use)
     risa::DeviceBuffer<float> adj_coord;     // [N] the forward's pixel coordinates
@@ -1841,12 +1889,6 @@ struct risa_bp_s {
     risa::DeviceBuffer<int> tile_order;
     std::vector<long> order_off;
 };
-
-namespace risa {
-// slices per pass of the sheared-path adjoint through its buffers
-constexpr int kAdjSlices = 16;
-constexpr int kAdjPathSlices = 2;   // images per wave of the path kernel (a divisor of kAdjSlices)
-}  // namespace risa
 
 namespace risa {
 // risa_hip_bp_run_f16 converts and backprojects up to this many groups of 4
@@ -2031,8 +2073,8 @@ static void setup_adjoint(risa_bp_s* h)
     h->adj_bands.upload(bands);
     h->adj_nb.resize(nb.size());
     h->adj_nb.upload(nb);
-    h->adj_imgA.resize((size_t)kAdjSlices * q.img_stride);
-    h->adj_imgB.resize((size_t)kAdjSlices * q.img_stride);
+    h->adj_imgA.resize((size_t)kAdjPlaces * q.img_stride);
+    h->adj_imgB.resize((size_t)kAdjPlaces * q.img_stride);
     // the padding columns stay zero: pad kernels write only the N x N interior
     RISA_HIP_CHECK(hipMemset(h->adj_imgA.ptr, 0, h->adj_imgA.count * sizeof(float)));
     RISA_HIP_CHECK(hipMemset(h->adj_imgB.ptr, 0, h->adj_imgB.count * sizeof(float)));
@@ -2385,17 +2427,24 @@ static void adjoint_run(risa_bp_t h, const float* img, int slices, float* sino, 
     hipLaunchKernelGGL(adj_tile_origin_kernel, dim3((unsigned)ceil_div(work, 256L)), dim3(256), 0, s, h->cosT.ptr,
                        h->sinT.ptr, q, h->adj_T.ptr, h->adj_coord.ptr);
     check_launch("adj_tile_origin_kernel");
-    for (int s0 = 0; s0 < slices; s0 += kAdjSlices) {
-        const int n = std::min(kAdjSlices, slices - s0);
-        hipLaunchKernelGGL(adj_pad_kernel, dim3(ceil_div(N, 32), ceil_div(N, 32), n), dim3(32, 8), 0, s,
-                           img + (size_t)s0 * N * N, h->adj_imgA.ptr, h->adj_imgB.ptr, N, q.PW, h->fuse_mask ? 1 : 0,
-                           h->lut.center, q.img_stride);
+    // a group of 4 is read with 32-bit byte offsets
+    const int per = (unsigned long)q.img_stride * 16 >> 32 ? 2 : kAdjSlices;
+    for (int s0 = 0; s0 < slices; s0 += per) {
+        const int n = std::min(per, slices - s0);
+        // 3 left over run as a group of 4
+        q.quads = (n + 1) / 4;
+        q.tail = n % 4 == 3 ? 0 : n % 4;
+        const unsigned groups = (unsigned)(q.quads + (q.tail ? 1 : 0));
+        hipLaunchKernelGGL(adj_pad_kernel, dim3(ceil_div(N, 32), ceil_div(N, 32), groups), dim3(32, 8), 0, s,
+                           img + (size_t)s0 * N * N, n, h->adj_imgA.ptr, h->adj_imgB.ptr, N, q.PW,
+                           h->fuse_mask ? 1 : 0, h->lut.center, q.img_stride, q.quads, q.tail);
         check_launch("adj_pad_kernel");
-        hipLaunchKernelGGL(bp_adjoint_path_kernel<kAdjPathSlices>,
-                           dim3(h->adj_groups, q.nbmax, ceil_div(n, kAdjPathSlices)), dim3(64 * kAdjWavesPerGroup), 0,
-                           s, h->adj_imgA.ptr, h->adj_imgB.ptr, h->adj_partial.ptr, h->adj_angles.ptr,
-                           h->adj_bands.ptr, h->adj_rows.ptr, h->adj_coord.ptr, h->adj_T.ptr, h->cosT.ptr, h->sinT.ptr,
-                           n, q);
+        const auto path = q.tail == 0   ? bp_adjoint_path_kernel<true, 0>
+                          : q.tail == 1 ? (q.quads ? bp_adjoint_path_kernel<true, 1> : bp_adjoint_path_kernel<false, 1>)
+                                        : (q.quads ? bp_adjoint_path_kernel<true, 2> : bp_adjoint_path_kernel<false, 2>);
+        hipLaunchKernelGGL(path, dim3(h->adj_groups, q.nbmax, groups), dim3(64 * kAdjWavesPerGroup), 0, s,
+                           h->adj_imgA.ptr, h->adj_imgB.ptr, h->adj_partial.ptr, h->adj_angles.ptr, h->adj_bands.ptr,
+                           h->adj_rows.ptr, h->adj_coord.ptr, h->adj_T.ptr, h->cosT.ptr, h->sinT.ptr, n, q);
         check_launch("bp_adjoint_path_kernel");
         hipLaunchKernelGGL(adj_reduce_kernel, dim3(P, n), dim3(256), (size_t)q.nbmax * kAdjRec * sizeof(float), s,
                            h->adj_partial.ptr, h->adj_nb.ptr, sino + (size_t)s0 * P * D, q);

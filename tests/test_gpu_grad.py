@@ -1,6 +1,6 @@
-"""Row transforms of the filter and of the tap gradient at each radix, row
-width and layout, and the tap gradient's short sums at the edges of their
-workgroups."""
+"""The backward path and its transforms: rows of the filter and of the tap
+gradient at each radix, row width and layout, the tap gradient's short sums at
+the edges of their workgroups, and the adjoint projector's groups of images."""
 from __future__ import annotations
 
 import numpy as np
@@ -93,3 +93,31 @@ def test_tap_gradient_row_kernels(risa, orc, geom_c0, cuda, D, rows):
     print(f"  rel L2 vs FP64 oracle {err:.2e}", flush=True)
     assert err < 1e-5
     flt.close()
+
+
+@pytest.mark.parametrize("N,P,mask", [(37, 5, True), (96, 18, False)])
+def test_adjoint_image_groups(risa, geom_c0, cuda, N, P, mask):
+    """The adjoint projector takes images in groups of four and a last two or
+    one, and 16 per pass: every image's sinogram is the one it has alone, bit
+    for bit (the same operations per image), also after a call that left other
+    values, NaN among them, in the groups' buffers."""
+    import torch
+    from risa_amd import device
+
+    g = geom_c0.replace(numberOfPixels=N, numberOfParallelProjections=P, numberOfParallelDetectors=N,
+                        fusedMasking=int(mask))
+    bp = device.Backprojection(g)
+    x = torch.from_numpy(np.random.default_rng(N).standard_normal((19, N, N)).astype(np.float32)).to(cuda)
+    alone = torch.empty((19, P, N), dtype=torch.float32, device=cuda)
+    for i in range(19):
+        bp.adjoint(x[i], alone[i])
+    assert float(alone.abs().max()) > 0.0
+    for S in (1, 2, 3, 4, 5, 6, 7, 16, 17, 19):
+        print(f"case: adjoint groups N={N} slices={S}", flush=True)
+        bad = torch.full((4, N, N), float("nan"), dtype=torch.float32, device=cuda)
+        bp.adjoint_batch(bad, 4, torch.empty((4, P, N), dtype=torch.float32, device=cuda))
+        got = torch.full((S, P, N), float("nan"), dtype=torch.float32, device=cuda)
+        bp.adjoint_batch(x[:S].contiguous(), S, got)
+        torch.cuda.synchronize()
+        assert torch.equal(got, alone[:S])
+    bp.close()
