@@ -230,6 +230,12 @@ __host__ __device__ constexpr int bp_row_buffers(int sb) { return sb == 4 ? 1 : 
 // adjacent lanes' 16-byte reads 32 bytes apart) and both halves share one
 // address, the second read taking the plane offset as its immediate.
 constexpr unsigned kQuadPlane = 16384;
+// LDS of one group of threads, a multiple of 16 B.
+__host__ __device__ constexpr size_t tile_lds(int AE, int W, int sb)
+{
+    const size_t rows = sb == 4 ? (size_t)2 * kQuadPlane : (size_t)2 * AE * W * 8 * sb;
+    return (rows + (size_t)3 * AE * 24 + 15) / 16 * 16;
+}
 template <int SB>
 struct LdsEnt {
     float v[2 * SB];
@@ -252,7 +258,11 @@ __device__ __forceinline__ LdsEnt<SB> lds_entry(unsigned addr)
     }
     return e;
 }
-template <int TX, int TY, int PPT, int E, int U, int SB = 1>
+//
+// Q > 1: Q groups of TX TY / PPT threads, group g over the angles
+// [P g / Q, P (g + 1) / Q) with rows and windows of its own (LDS region g), the
+// groups' sums added in order at the end.
+template <int TX, int TY, int PPT, int E, int U, int SB = 1, int Q = 1>
 __device__ __forceinline__ void bp_tile(const void* __restrict__ sino_v, float* __restrict__ I,
                                         const float* __restrict__ cosT, const float* __restrict__ sinT,
                                         const BpParams& p, int x0, int y0, int in_f16, char* smem,
@@ -267,14 +277,17 @@ __device__ __forceinline__ void bp_tile(const void* __restrict__ sino_v, float* 
     constexpr int NT = TX * TY / PPT;
     constexpr int RS = TY / PPT;
     constexpr unsigned EB = SB == 4 ? 16u : 8u * SB;   // entry stride in a row (a plane for SB = 4)
-    const int tid = threadIdx.x;
+    static_assert(Q == 1 || NT % 64 == 0, "a wave works on one group's angles");
+    const int grp = Q == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    const int tid = Q == 1 ? (int)threadIdx.x : (int)threadIdx.x - grp * NT;
     const int tx = tid % TX, ty = tid / TX;
+    const int pa = Q == 1 ? 0 : (int)((long)p.P * grp / Q), pb = Q == 1 ? p.P : (int)((long)p.P * (grp + 1) / Q);
     const float* S = reinterpret_cast<const float*>(sino_v);
     const uint16_t* S16 = reinterpret_cast<const uint16_t*>(sino_v);
     const int W = p.W, AE = p.AE;
-    char* rows = smem;
+    char* rows = Q == 1 ? smem : smem + grp * tile_lds(AE, W, SB);
     const unsigned rbase = lds_address(rows);
-    float4* info = reinterpret_cast<float4*>(smem + (SB == 4 ? (size_t)2 * kQuadPlane : (size_t)NB * AE * W * EB));
+    float4* info = reinterpret_cast<float4*>(rows + (SB == 4 ? (size_t)2 * kQuadPlane : (size_t)NB * AE * W * EB));
     int2* kinfo = reinterpret_cast<int2*>(info + 3 * AE);
 
     const int x = x0 + tx;
@@ -291,6 +304,7 @@ __device__ __forceinline__ void bp_tile(const void* __restrict__ sino_v, float* 
         any |= use[r] ? 1 : 0;
     }
     if (!__syncthreads_or(any)) {
+        if (Q > 1 && grp > 0) return;
 #pragma unroll
         for (int r = 0; r < PPT; r++) {
             const int y = y0 + ty + r * RS;
@@ -311,30 +325,36 @@ __device__ __forceinline__ void bp_tile(const void* __restrict__ sino_v, float* 
 
     const float xa = ((float)x0 - p.center) * p.scale, xb = ((float)(x0 + TX - 1) - p.center) * p.scale;
     const float ya = ((float)y0 - p.center) * p.scale, yb = ((float)(y0 + TY - 1) - p.center) * p.scale;
-    const int nch = (p.P + AE - 1) / AE;
+    // the same number of chunks for every group: they share the barriers
+    const int nch = ((p.P + Q - 1) / Q + AE - 1) / AE;
     // the windows of chunk ch go to ring slot ch % 3: chunk ch is computed
     // while ch + 1 is fetched and ch + 2 is prepared, one barrier per chunk
-    auto make_info = [&](int ch) {
-        if (ch >= nch) return;
-        const int p0 = ch * AE, na = min(AE, p.P - p0);
-        float4* inf = info + (ch % 3) * AE;
-        int2* kin = kinfo + (ch % 3) * AE;
-        for (int a = tid; a < na; a += NT) {
-            const AngleWin w = angle_window(cosT[p0 + a], sinT[p0 + a], xa, xb, ya, yb, p.cI);
-            const int row = (ch % NB) * AE * W + a * W;
-            inf[a] = make_float4(w.c, w.s, w.negT, __uint_as_float(rbase + (unsigned)(row - w.kmin) * EB));
-            kin[a] = make_int2(w.kmin, w.kabs);
-        }
+    // One thread per angle (AE <= 64 <= NT); its (cos, sin) is loaded well
+    // before the window is computed.
+    static_assert(NT >= 64, "a thread per angle of a chunk");
+    auto load_angle = [&](int ch) {
+        const int a = pa + ch * AE + tid;
+        return tid < AE && a < pb ? make_float2(cosT[a], sinT[a]) : make_float2(0.0f, 0.0f);
     };
-    make_info(0);
-    make_info(1);
+    auto make_info = [&](int ch, float2 cs) {
+        if (tid >= min(AE, pb - pa - ch * AE)) return;
+        const AngleWin w = angle_window(cs.x, cs.y, xa, xb, ya, yb, p.cI);
+        const int row = (ch % NB) * AE * W + tid * W;
+        info[(ch % 3) * AE + tid] = make_float4(w.c, w.s, w.negT, __uint_as_float(rbase + (unsigned)(row - w.kmin) * EB));
+        kinfo[(ch % 3) * AE + tid] = make_int2(w.kmin, w.kabs);
+    };
+    {
+        const float2 cs0 = load_angle(0), cs1 = load_angle(1);
+        make_info(0, cs0);
+        make_info(1, cs1);
+    }
     __syncthreads();
 
     float s0r[E][SB], s1r[E][SB];
     bool in0r[E], in1r[E];
     int kr[E];
     auto fetch = [&](int ch) {
-        const int p0 = ch * AE, nae = min(AE, p.P - p0) * W;
+        const int p0 = pa + ch * AE, nae = min(AE, pb - p0) * W;
         const int2* kin = kinfo + (ch % 3) * AE;
 #pragma unroll
         for (int q = 0; q < E; q++) {
@@ -375,7 +395,7 @@ __device__ __forceinline__ void bp_tile(const void* __restrict__ sino_v, float* 
         }
     };
     auto commit = [&](int ch) {
-        const int nae = min(AE, p.P - ch * AE) * W;
+        const int nae = min(AE, pb - pa - ch * AE) * W;
         char* buf = rows + (size_t)(ch % NB) * AE * W * EB;
 #pragma unroll
         for (int q = 0; q < E; q++) {
@@ -410,8 +430,9 @@ __device__ __forceinline__ void bp_tile(const void* __restrict__ sino_v, float* 
     commit(0);
     __syncthreads();
     for (int ch = 0; ch < nch; ch++) {
-        const int p0 = ch * AE, na = min(AE, p.P - p0);
+        const int na = min(AE, pb - pa - ch * AE);
         const float4* inf = info + (ch % 3) * AE;
+        const float2 cs = load_angle(ch + 2);
         if (ch + 1 < nch) fetch(ch + 1);
         if (wave_active) {
             // U angles per step: all U*PPT LDS reads are issued before the
@@ -455,8 +476,25 @@ __device__ __forceinline__ void bp_tile(const void* __restrict__ sino_v, float* 
         }
         if constexpr (NB == 1) __syncthreads();   // the single row buffer is read
         if (ch + 1 < nch) commit(ch + 1);
-        make_info(ch + 2);
+        make_info(ch + 2, cs);
         __syncthreads();
+    }
+    if constexpr (Q > 1) {
+        // the rows are read: the groups' sums go through their space
+        float* red = reinterpret_cast<float*>(smem);
+#pragma unroll
+        for (int r = 0; r < PPT; r++)
+#pragma unroll
+            for (int b = 0; b < SB; b++)
+                if (grp > 0) red[(((grp - 1) * PPT + r) * SB + b) * NT + tid] = acc[r][b];
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 0; g < Q - 1; g++)
+#pragma unroll
+            for (int r = 0; r < PPT; r++)
+#pragma unroll
+                for (int b = 0; b < SB; b++) acc[r][b] += red[((g * PPT + r) * SB + b) * NT + tid];
     }
 #pragma unroll
     for (int r = 0; r < PPT; r++) {
@@ -480,8 +518,8 @@ struct BpSlices {
     float* img[kBpSlices];
 };
 
-template <int TX, int TY, int PPT, int E, int U, int SB>
-__global__ void __launch_bounds__(TX* TY / PPT) bp_linear_kernel(BpSlices L, const float* __restrict__ cosT,
+template <int TX, int TY, int PPT, int E, int U, int SB, int Q = 1>
+__global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_kernel(BpSlices L, const float* __restrict__ cosT,
                                                                  const float* __restrict__ sinT, int slices,
                                                                  BpParams p)
 {
@@ -490,7 +528,7 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_kernel(BpSlices L, con
     const int first = bp_work(p, txy) * SB;
     const int x0 = txy.x * TX, y0 = txy.y * TY;
     if constexpr (SB == 1) {
-        bp_tile<TX, TY, PPT, E, U, 1>(L.sino[first], L.img[first], cosT, sinT, p, x0, y0, 0, smem);
+        bp_tile<TX, TY, PPT, E, U, 1, Q>(L.sino[first], L.img[first], cosT, sinT, p, x0, y0, 0, smem);
     } else {
         const int nv = min(SB, slices - first);
         const float* sp[SB];
@@ -500,7 +538,7 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_kernel(BpSlices L, con
             sp[b] = L.sino[b < nv ? first + b : first];
             ip[b] = L.img[b < nv ? first + b : first];
         }
-        bp_tile<TX, TY, PPT, E, U, SB>(sp[0], ip[0], cosT, sinT, p, x0, y0, 0, smem, sp, ip, nv);
+        bp_tile<TX, TY, PPT, E, U, SB, Q>(sp[0], ip[0], cosT, sinT, p, x0, y0, 0, smem, sp, ip, nv);
     }
 }
 
@@ -1790,11 +1828,15 @@ namespace risa {
 // and the cap on angles per chunk.  The chunk holds AE = min(amax,
 // E * threads / W) angles so one thread stages at most E entries.
 struct BpVariant {
-    int tx, ty, ppt, e, u, sb, amax;   // sb: slices per workgroup (1 or 2)
+    int tx, ty, ppt, e, u, sb, amax;   // sb: slices per workgroup (1, 2 or 4)
     void (*fn)(BpSlices, const float*, const float*, int, BpParams);
+    int q = 1;                         // groups of threads that share the angles
+    int threads() const { return tx * ty / ppt; }   // of one group
 };
 
 #define RISA_BPV(TX, TY, PPT, E, U, SB, AMAX) {TX, TY, PPT, E, U, SB, AMAX, bp_linear_kernel<TX, TY, PPT, E, U, SB>}
+#define RISA_BPQ(TX, TY, PPT, E, U, SB, AMAX, Q) \
+    {TX, TY, PPT, E, U, SB, AMAX, bp_linear_kernel<TX, TY, PPT, E, U, SB, Q>, Q}
 static const BpVariant kVariants[] = {
     RISA_BPV(32, 32, 4, 8, 4, 1, 64), RISA_BPV(32, 16, 2, 8, 4, 1, 64), RISA_BPV(16, 16, 1, 4, 4, 1, 64),
     RISA_BPV(32, 32, 8, 16, 2, 1, 64), RISA_BPV(64, 16, 4, 16, 4, 1, 64), RISA_BPV(32, 16, 4, 16, 4, 1, 64),
@@ -1807,8 +1849,18 @@ static const BpVariant kVariants[] = {
     // four slices per workgroup: two planes of 16-byte half entries, one staged row buffer
     RISA_BPV(32, 32, 4, 4, 1, 4, 64), RISA_BPV(32, 32, 4, 4, 2, 4, 64), RISA_BPV(32, 16, 2, 4, 2, 4, 64),
     RISA_BPV(16, 16, 1, 2, 4, 4, 64),
+    // The angles shared by q groups of threads: where one or a few slices leave
+    // each SIMD with one wave or a few, whose chain of LDS reads then sets the
+    // time (one wave takes about 100 clocks per angle, of which it issues for
+    // 40).  More waves at the same tiles: 256^2 x 500 angles, one slice 32.5 ->
+    // 14.3 us; 512^2 x 1000 one slice 80 -> 53, four 145 -> 133; 384^2 x 360
+    // six slices 67 -> 60.  Full launches stay with the variants above
+    // (512^2 x 720, 16 slices: 314 us, 321 at best with groups).
+    RISA_BPQ(16, 16, 2, 4, 4, 1, 64, 4), RISA_BPQ(16, 16, 2, 4, 4, 1, 64, 8), RISA_BPQ(32, 32, 4, 4, 2, 1, 64, 4),
+    RISA_BPQ(16, 16, 2, 4, 4, 2, 64, 4), RISA_BPQ(16, 16, 1, 2, 4, 2, 64, 2), RISA_BPQ(32, 32, 4, 4, 2, 2, 64, 2),
 };
 #undef RISA_BPV
+#undef RISA_BPQ
 static constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
 struct BpF16Variant {
@@ -1845,17 +1897,12 @@ static int window_entries(int tx, int ty, float scale)
 // buffer of two kQuadPlane-byte planes of 16-byte half entries) + a ring of
 // 3 chunks of per-angle windows (16 B + 8 B per angle).
 constexpr size_t kMaxLds = 64 * 1024;
-static size_t tile_lds(int AE, int W, int sb)
-{
-    const size_t rows = sb == 4 ? (size_t)2 * kQuadPlane : (size_t)2 * AE * W * 8 * sb;
-    return rows + (size_t)3 * AE * 24;
-}
 // AE also shrinks so the tile fits the LDS budget (sb = 4: a plane).
-static int chunk_angles(int threads, int e, int amax, int W, int sb = 1)
+static int chunk_angles(int threads, int e, int amax, int W, int sb = 1, int q = 1)
 {
     int ae = std::min(amax, e * threads / W);
     if (sb == 4) ae = std::min<long>(ae, (long)kQuadPlane / (16L * W));
-    else ae = std::min<long>(ae, (long)kMaxLds / (2L * W * 8 * sb + 72));
+    else ae = std::min<long>(ae, (long)kMaxLds / q / (2L * W * 8 * sb + 88));
     return std::max(1, ae);
 }
 
@@ -2137,9 +2184,13 @@ static void launch_linear_at(risa_bp_t h, int variant, SinoAt sino, ImgAt img, i
 {
     const BpVariant& v = kVariants[variant];
     BpParams p = make_params(h, v.tx, v.ty);
-    const int threads = v.tx * v.ty / v.ppt;
-    p.AE = chunk_angles(threads, v.e, v.amax, p.W, v.sb);
-    const size_t lds = tile_lds(p.AE, p.W, v.sb);
+    p.AE = chunk_angles(v.threads(), v.e, v.amax, p.W, v.sb, v.q);
+    if (v.q > 1) {   // a group's chunks of about the same length
+        const int len = ceil_div(p.P, v.q);
+        p.AE = ceil_div(len, ceil_div(len, p.AE));
+    }
+    const size_t lds = std::max(v.q * tile_lds(p.AE, p.W, v.sb),
+                                sizeof(float) * (v.q - 1) * v.ppt * v.sb * v.threads());
     if (lds > kMaxLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %zu B of LDS", lds);
     static_assert(kBpSlices % 4 == 0, "launch chunks hold whole slice groups");
     for (int k0 = 0; k0 < slices; k0 += kBpSlices) {
@@ -2153,7 +2204,7 @@ static void launch_linear_at(risa_bp_t h, int variant, SinoAt sino, ImgAt img, i
         dim3 grid(p.tilesX * ceil_div(p.N, v.ty), ceil_div(n, v.sb));
         p.xg = xcd_groups(grid.x, grid.y);
         p.order = p.xg && h->order_off[(size_t)variant] >= 0 ? h->tile_order.ptr + h->order_off[(size_t)variant] : nullptr;
-        hipLaunchKernelGGL(v.fn, grid, dim3(threads), lds, s, L, h->cosT.ptr, h->sinT.ptr, n, p);
+        hipLaunchKernelGGL(v.fn, grid, dim3(v.q * v.threads()), lds, s, L, h->cosT.ptr, h->sinT.ptr, n, p);
         check_launch("bp_linear_kernel");
     }
 }

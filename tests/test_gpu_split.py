@@ -111,3 +111,27 @@ def test_chain_plain_large_groups(risa, geom_c1, cuda):
         assert torch.equal(again, img)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("N,P,S", [(33, 1, 1), (33, 3, 2), (40, 7, 3), (17, 13, 1), (64, 131, 5)])
+def test_angle_groups(risa, geom_c0, cuda, N, P, S):
+    """Variants whose angles are shared by groups of threads, with fewer angles
+    than groups and uneven shares, against the first variant: every variant sums
+    the same terms.  Bound 1e-5 of the image's norm: coordinates below 64 round
+    to 4e-6, the sample differences they multiply are about 1.4 of a sample."""
+    import torch
+    from risa_amd import device
+
+    g = geom_c0.replace(numberOfPixels=N, numberOfParallelProjections=P, numberOfParallelDetectors=N + 5)
+    bp = device.Backprojection(g)
+    x = torch.from_numpy(np.random.default_rng(N + P).standard_normal((S, P, N + 5)).astype(np.float32)).to(cuda)
+    ref = None
+    for v in range(device.bp_num_variants()):
+        print(f"case: angle groups N={N} P={P} S={S} variant {v}", flush=True)
+        bp.variant = v
+        img = torch.full((S, N, N), float("nan"), dtype=torch.float32, device=cuda)
+        bp.batch(x, S, img)
+        torch.cuda.synchronize()
+        ref = img if ref is None else ref
+        assert float((img - ref).norm() / ref.norm()) < 1e-5
+    bp.close()
