@@ -63,6 +63,14 @@ __device__ __attribute__((noinline)) float rebin_ray(const float* __restrict__ f
 // e.g. the alpha_0 = 0 row) gathers from global memory instead.
 constexpr int kRebinBlock = 16;
 constexpr int kPatchMax = 512;
+// Workgroups a launch aims at before a plane's frames share one.  A workgroup
+// walks its frames one after another, each a load, two barriers and the rays:
+// 2 us a frame whatever the block count, so few blocks need more workgroups;
+// each further one reads the block's table entries again.  32 frames of
+// 256 x 500 (512 blocks): 57 us in one group, 25 / 22 / 28 aiming at 2048 /
+// 4096 / 16384; 8 frames of 512 x 1000 in two planes (2 x 2016 blocks): 25 /
+// 29 / 33, so the line lies between.
+constexpr long kRebinFill = 3072;
 
 // Ray of one slot from its LDS patch (no wrap inside a patch).
 __device__ __forceinline__ float patch_ray(const float* __restrict__ pt, int4 box, uint32_t idx, float ft, float fg)
@@ -135,11 +143,13 @@ __global__ void __launch_bounds__(256) rebin_kernel(const uint4* __restrict__ ta
     for (int sl = 0; sl < 4; sl++) {
         const int4 b = box[sl];
         const int cnt = b.z > 0 ? b.z * b.w : 0;
+        const float inv = 1.0f / (float)max(b.w, 1);
 #pragma unroll
         for (int j = 0; j < kPer; j++) {
             const int t = threadIdx.x + j * 256;
             have[sl][j] = t < cnt;
-            const int r = have[sl][j] ? t / b.w : 0;
+            // t / b.w: t < 512, so (t + 1/2) / b.w is further from an integer than its rounding
+            const int r = have[sl][j] ? (int)(((float)t + 0.5f) * inv) : 0;
             goff[sl][j] = have[sl][j] ? (b.x + r) * Df + b.y + (t - r * b.w) : 0;
         }
     }
@@ -489,6 +499,10 @@ static void launch_rebin_at(risa_fan2para_t h, FanAt fan, const int32_t* planes,
     for (int f0 = 0; f0 < frames; f0 += kMaxFramesPerLaunch) {
         const int nf = std::min(kMaxFramesPerLaunch, frames - f0);
         FrameGroups fg{};
+        // frames per workgroup: all of a plane's while the planes' blocks fill
+        // the chip, else fewer
+        const int blocks = ceil_div(D, kRebinBlock) * ceil_div(P, kRebinBlock);
+        const int cap = std::max(1, (int)((long)nf * blocks / kRebinFill));
         int groups = 0, pos = 0;
         for (int k = 0; k < h->g.numberOfPlanes; k++) {
             int cnt = 0;
@@ -502,15 +516,16 @@ static void launch_rebin_at(risa_fan2para_t h, FanAt fan, const int32_t* planes,
                     cnt++;
                 }
             }
-            if (cnt) {
+            const int parts = ceil_div(cnt, cap);
+            for (int q = 0; q < parts; q++) {
                 fg.plane[groups] = k;
-                fg.start[groups] = pos;
-                fg.count[groups] = cnt;
+                fg.start[groups] = pos + cnt * q / parts;
+                fg.count[groups] = cnt * (q + 1) / parts - cnt * q / parts;
                 groups++;
-                pos += cnt;
             }
+            pos += cnt;
         }
-        dim3 grid(ceil_div(D, kRebinBlock) * ceil_div(P, kRebinBlock), groups);
+        dim3 grid(blocks, groups);
         hipLaunchKernelGGL(rebin_kernel, grid, dim3(256), 0, s, reinterpret_cast<const uint4*>(h->table.ptr),
                            h->boxes.ptr, h->order.ptr, Df, Pf, D, P, (long)(h->plane_words / 4), h->box_plane, fg);
         check_launch("rebin_kernel");
