@@ -624,10 +624,17 @@ struct HRowG {
     HRow h[G];
 };
 
+// LDS of one group of threads: G planes of two chunks of E * threads 16-byte
+// entries, and the ring of angle windows; a multiple of 16 B.
+__host__ __device__ constexpr size_t f16_lds(int G, int E, int threads, int AE)
+{
+    return ((size_t)G * 2 * E * threads * 16 + (size_t)3 * AE * 24 + 15) / 16 * 16;
+}
+
 // G groups of 4 slices per workgroup: the per-pixel t, index and weight are
-// shared by 4G slices.
-template <int TX, int TY, int PPT, int E, int U, int G>
-__global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2* __restrict__ sino,
+// shared by 4G slices.  Q groups of threads share the angles as in bp_tile.
+template <int TX, int TY, int PPT, int E, int U, int G, int Q = 1>
+__global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_kernel(const uint2* __restrict__ sino,
                                                                      float* __restrict__ img,
                                                                      const float* __restrict__ cosT,
                                                                      const float* __restrict__ sinT, int slices,
@@ -643,12 +650,16 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2
     constexpr int PLANE = 2 * E * NT;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int W = p.W, AE = p.AE;
-    HRow* rows = reinterpret_cast<HRow*>(smem);
+    static_assert(NT % 64 == 0, "a wave works on one group's angles");
+    const int grp = Q == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    const int pa = Q == 1 ? 0 : (int)((long)p.P * grp / Q), pb = Q == 1 ? p.P : (int)((long)p.P * (grp + 1) / Q);
+    char* region = Q == 1 ? smem : smem + grp * f16_lds(G, E, NT, AE);
+    HRow* rows = reinterpret_cast<HRow*>(region);
     const unsigned rbase = lds_address(rows);
-    float4* info = reinterpret_cast<float4*>(smem + (size_t)G * PLANE * sizeof(HRow));
+    float4* info = reinterpret_cast<float4*>(region + (size_t)G * PLANE * sizeof(HRow));
     int2* kinfo = reinterpret_cast<int2*>(info + 3 * AE);
 
-    const int tid = threadIdx.x;
+    const int tid = (int)threadIdx.x - grp * NT;
     const int tx = tid % TX, ty = tid / TX;
     int2 txy;
     const int g0 = bp_work(p, txy) * G;
@@ -674,6 +685,7 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2
         any |= use[r] ? 1 : 0;
     }
     if (!__syncthreads_or(any)) {
+        if (Q > 1 && grp > 0) return;
         for (int b = 0; b < nb; b++)
 #pragma unroll
             for (int r = 0; r < PPT; r++) {
@@ -691,28 +703,32 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2
 
     const float xa = ((float)x0 - p.center) * p.scale, xb = ((float)(x0 + TX - 1) - p.center) * p.scale;
     const float ya = ((float)y0 - p.center) * p.scale, yb = ((float)(y0 + TY - 1) - p.center) * p.scale;
-    const int nch = (p.P + AE - 1) / AE;
-    auto make_info = [&](int ch) {
-        if (ch >= nch) return;
-        const int p0 = ch * AE, na = min(AE, p.P - p0);
-        float4* inf = info + (ch % 3) * AE;
-        int2* kin = kinfo + (ch % 3) * AE;
-        for (int a = tid; a < na; a += NT) {
-            const AngleWin w = angle_window(cosT[p0 + a], sinT[p0 + a], xa, xb, ya, yb, p.cI);
-            const int row = (ch & 1) * AE * W + a * W;
-            inf[a] = make_float4(w.c, w.s, w.negT,
-                                 __uint_as_float(rbase + (unsigned)((row - w.kmin) * (int)sizeof(HRow))));
-            kin[a] = make_int2(w.kmin, w.kabs);
-        }
+    // the same number of chunks for every group: they share the barriers
+    const int nch = ((p.P + Q - 1) / Q + AE - 1) / AE;
+    // one thread per angle (AE <= 64 <= NT), loaded well before its window
+    auto load_angle = [&](int ch) {
+        const int a = pa + ch * AE + tid;
+        return tid < AE && a < pb ? make_float2(cosT[a], sinT[a]) : make_float2(0.0f, 0.0f);
     };
-    make_info(0);
-    make_info(1);
+    auto make_info = [&](int ch, float2 cs) {
+        if (tid >= min(AE, pb - pa - ch * AE)) return;
+        const AngleWin w = angle_window(cs.x, cs.y, xa, xb, ya, yb, p.cI);
+        const int row = (ch & 1) * AE * W + tid * W;
+        info[(ch % 3) * AE + tid] = make_float4(
+            w.c, w.s, w.negT, __uint_as_float(rbase + (unsigned)((row - w.kmin) * (int)sizeof(HRow))));
+        kinfo[(ch % 3) * AE + tid] = make_int2(w.kmin, w.kabs);
+    };
+    {
+        const float2 cs0 = load_angle(0), cs1 = load_angle(1);
+        make_info(0, cs0);
+        make_info(1, cs1);
+    }
     __syncthreads();
 
     uint2 q0r[E][G], q1r[E][G];
     bool in0r[E], in1r[E];
     auto fetch = [&](int ch) {
-        const int p0 = ch * AE, nae = min(AE, p.P - p0) * W;
+        const int p0 = pa + ch * AE, nae = min(AE, pb - p0) * W;
         const int2* kin = kinfo + (ch % 3) * AE;
 #pragma unroll
         for (int q = 0; q < E; q++) {
@@ -746,7 +762,7 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2
         }
     };
     auto commit = [&](int ch) {
-        const int nae = min(AE, p.P - ch * AE) * W;
+        const int nae = min(AE, pb - pa - ch * AE) * W;
         HRow* buf = rows + (ch & 1) * AE * W;
 #pragma unroll
         for (int q = 0; q < E; q++) {
@@ -764,8 +780,9 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2
     commit(0);
     __syncthreads();
     for (int ch = 0; ch < nch; ch++) {
-        const int p0 = ch * AE, na = min(AE, p.P - p0);
+        const int na = min(AE, pb - pa - ch * AE);
         const float4* inf = info + (ch % 3) * AE;
+        const float2 cs = load_angle(ch + 2);
         if (ch + 1 < nch) fetch(ch + 1);
         if (wave_active) {
             int a = 0;
@@ -825,8 +842,24 @@ __global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2
             }
         }
         if (ch + 1 < nch) commit(ch + 1);
-        make_info(ch + 2);
+        make_info(ch + 2, cs);
         __syncthreads();
+    }
+    if constexpr (Q > 1) {
+        float* red = reinterpret_cast<float*>(smem);   // the rows are read
+#pragma unroll
+        for (int r = 0; r < PPT; r++)
+#pragma unroll
+            for (int b = 0; b < B; b++)
+                if (grp > 0) red[(((grp - 1) * PPT + r) * B + b) * NT + tid] = acc[r][b];
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 0; g < Q - 1; g++)
+#pragma unroll
+            for (int r = 0; r < PPT; r++)
+#pragma unroll
+                for (int b = 0; b < B; b++) acc[r][b] += red[((g * PPT + r) * B + b) * NT + tid];
     }
     for (int b = 0; b < nb; b++)
 #pragma unroll
@@ -1866,9 +1899,12 @@ static constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 struct BpF16Variant {
     int tx, ty, ppt, e, u, g, amax;
     void (*fn)(const uint2*, float*, const float*, const float*, int, BpParams);
+    int q = 1;   // groups of threads that share the angles
 };
 #define RISA_BPH(TX, TY, PPT, E, U, G, AMAX) \
     {TX, TY, PPT, E, U, G, AMAX, bp_linear_f16_kernel<TX, TY, PPT, E, U, G>}
+#define RISA_BPG(TX, TY, PPT, E, U, G, AMAX, Q) \
+    {TX, TY, PPT, E, U, G, AMAX, bp_linear_f16_kernel<TX, TY, PPT, E, U, G, Q>, Q}
 // 16-pixel-wide tiles: the 16-byte LDS entries of a half-wave row then
 // stay clear of bank conflicts; G groups of 4 slices share each pixel's
 // weight.  The LDS planes take G * 2 * E * threads * 16 B, at most 32 KB
@@ -1878,8 +1914,15 @@ static const BpF16Variant kF16Variants[] = {
     RISA_BPH(16, 16, 1, 2, 4, 2, 64), RISA_BPH(16, 32, 2, 2, 2, 2, 64), RISA_BPH(16, 32, 4, 4, 2, 2, 64),
     RISA_BPH(16, 32, 4, 2, 2, 2, 64), RISA_BPH(16, 16, 1, 2, 2, 2, 64), RISA_BPH(16, 16, 1, 1, 2, 4, 64),
     RISA_BPH(16, 8, 1, 1, 2, 8, 64),
+    // The angles shared by q groups of threads, for launches that leave a SIMD
+    // few waves (as in the FP32 table): 512^2 x 1000 angles, 4 slices 148 ->
+    // 102 us, 8 slices 178 -> 162; 256^2 x 500, 4 slices 59 -> 26, 16 slices
+    // 67 -> 49.  From 16 slices of 512^2 the variants above are at least as fast.
+    RISA_BPG(16, 32, 2, 2, 2, 1, 64, 4), RISA_BPG(16, 16, 1, 1, 4, 1, 64, 4), RISA_BPG(16, 16, 1, 2, 4, 2, 64, 2),
+    RISA_BPG(16, 32, 2, 2, 2, 2, 64, 2), RISA_BPG(16, 16, 1, 1, 2, 2, 64, 4),
 };
 #undef RISA_BPH
+#undef RISA_BPG
 static constexpr int kNumF16Variants = sizeof(kF16Variants) / sizeof(kF16Variants[0]);
 
 // Largest window a tx x ty tile needs for detector scale `scale`: the span of
@@ -2268,13 +2311,18 @@ static void launch_f16x4(risa_bp_t h, int variant, const uint2* sino, float in_s
     // per group an LDS plane of two chunks of E * threads entries
     if (p.W > v.e * threads) fail(RISA_ERR_UNSUPPORTED, "backprojection window exceeds the tile's staging");
     p.AE = std::max(1, std::min(v.amax, v.e * threads / p.W));
-    const size_t lds = (size_t)v.g * 2 * v.e * threads * sizeof(HRow) + (size_t)3 * p.AE * 24;
-    if (lds > kMaxLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %zu B of LDS", lds);
+    if (v.q > 1) {   // a group's chunks of about the same length
+        const int len = ceil_div(p.P, v.q);
+        p.AE = ceil_div(len, ceil_div(len, p.AE));
+    }
+    const size_t lds = std::max(v.q * f16_lds(v.g, v.e, threads, p.AE),
+                                sizeof(float) * (v.q - 1) * v.ppt * kF16Group * v.g * threads);
+    if (lds > (v.q > 1 ? kMaxLds / 64 * 80 : kMaxLds)) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %zu B of LDS", lds);
     dim3 grid(p.tilesX * ceil_div(p.N, v.ty), ceil_div(ceil_div(slices, kF16Group), v.g));
     p.xg = xcd_groups(grid.x, grid.y);
     const long off = h->order_off[(size_t)(kNumVariants + variant)];
     p.order = p.xg && off >= 0 ? h->tile_order.ptr + off : nullptr;
-    hipLaunchKernelGGL(v.fn, grid, dim3(threads), lds, s, sino, img, h->cosT.ptr, h->sinT.ptr, slices, p);
+    hipLaunchKernelGGL(v.fn, grid, dim3(v.q * threads), lds, s, sino, img, h->cosT.ptr, h->sinT.ptr, slices, p);
     check_launch("bp_linear_f16_kernel");
 }
 
