@@ -6,8 +6,8 @@
 // stream-ordered, and a captured hipGraph replays the launch sequence.
 //
 // PLAIN: frame by frame, FP32 throughout (FFT filter, FP32 backprojector).
-//        Groups of `per` consecutive frames (up to 16; each stage runs once
-//        per group) are dealt round-robin to `lanes` streams (own scratch
+//        Groups of `per` consecutive frames (up to 16, or 32; each stage runs
+//        once per group) are dealt round-robin to `lanes` streams (own scratch
 //        buffers each) forked from and joined back into the caller's stream,
 //        so lanes x per frames are in flight -- the way the reference
 //        overlaps frames across its per-stage threads.  Chains of at least 64
@@ -40,8 +40,8 @@ extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, floa
 namespace {
 constexpr float kF16SinoScale = 256.0f;   // FP16 filtered sinogram stores 256 * value
 constexpr int kPlainLanes = 2;            // streams in PLAIN mode
-constexpr int kPlainMaxPer = 16;          // frames per lane step in PLAIN mode, at most
-constexpr int kSplitPer = 32;             // frames per lane step of a PLAIN chain with the split backprojector
+constexpr int kPlainMaxPer = 16;          // frames per lane step of a PLAIN chain below 64 frames, at most
+constexpr int kSplitPer = 32;             // and of 64 frames or more (also the split backprojector's slices)
 constexpr int kMixedLanes = 2;            // streams in MIXED mode
 constexpr int kMixedMaxPer = 32;          // frames per lane step in MIXED mode, at most (a multiple of 4)
 }  // namespace
@@ -164,8 +164,11 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
             const size_t fan = (size_t)g->numberOfFanDetectors * g->numberOfFanProjections;
             const size_t par = (size_t)g->numberOfParallelDetectors * g->numberOfParallelProjections;
             if (mode == RISA_CHAIN_PLAIN) {
-                h->lanes = std::min(kPlainLanes, max_frames);
-                h->per = std::max(1, std::min(kPlainMaxPer, max_frames / h->lanes));
+                // one group while it holds every frame (8 frames of 256^2 x 500:
+                // 97 us, 125 as two groups of 4 in two lanes), 32 to a group
+                // from 64 frames on (100 frames 539 us, 588 with 16)
+                h->lanes = max_frames > kPlainMaxPer ? kPlainLanes : 1;
+                h->per = std::min(max_frames >= kPlainLanes * kSplitPer ? kSplitPer : kPlainMaxPer, max_frames);
                 if (max_frames >= kPlainLanes * kSplitPer && (h->split_bytes = risa_bp_split_bytes(h->bp)) > 0 &&
                     (h->split_scale = split_scale(h, avg_ref, avg_dark)) > 0.0f) {
                     ok(risa_hip_bp_autotune_batch(h->bp, kPlainLanes * kPlainMaxPer, nullptr));
@@ -183,9 +186,11 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
                 h->par_buf.resize(par * slots);
                 h->filt_buf.resize(par * slots);
             } else {
-                // groups of a multiple of 4 frames: whole x4 slice groups per lane
-                const int half = (max_frames + kMixedLanes - 1) / kMixedLanes;
-                h->per = std::min(kMixedMaxPer, (half + 3) / 4 * 4);
+                // groups of a multiple of 4 frames: whole x4 slice groups per
+                // lane; as few as hold the frames (512^2 x 1000, 8 frames: one
+                // group 245 us, two of 4 in two lanes 292; 48 frames as 32 + 16
+                // 978, as 24 + 24 1160)
+                h->per = std::min(kMixedMaxPer, (max_frames + 3) / 4 * 4);
                 h->lanes = std::min(kMixedLanes, (max_frames + h->per - 1) / h->per);
                 const size_t slots = (size_t)h->lanes * h->per;
                 h->att_buf.resize(fan * slots);
@@ -210,7 +215,7 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
             if (mode == RISA_CHAIN_PLAIN) {
                 if (h->split_min > 0) {
                     // tuned above
-                } else if (h->per > 1) ok(risa_hip_bp_autotune_batch(h->bp, h->lanes * h->per, nullptr));
+                } else if (h->per > 1) ok(risa_hip_bp_autotune_batch(h->bp, std::min(kPlainLanes * kPlainMaxPer, h->lanes * h->per), nullptr));
                 else ok(risa_hip_bp_autotune_slices(h->bp, h->lanes, nullptr));
             } else {
                 ok(risa_hip_bp_autotune_f16(h->bp, h->per, nullptr));
