@@ -1005,6 +1005,13 @@ __global__ void tune_fill_kernel(float* out, long n)
         out[i] = (float)((int)((unsigned)i * 2654435761u) >> 8) * 0x1p-26f;
 }
 
+// The same in FP16, below 1/2 in magnitude.
+__global__ void tune_fill_f16_kernel(uint16_t* out, long n)
+{
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
+        out[i] = float_to_half_bits((float)((int)((unsigned)i * 2654435761u) >> 8) * 0x1p-24f);
+}
+
 // Workgroup x: a TX x TY tile of the (up to) 32 slices; each wave an 8 x 8
 // pixel block as 2 x 2 blocks of 4 x 4.
 using lds_bytes = __attribute__((address_space(3))) char;
@@ -1192,6 +1199,344 @@ __global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* _
                 for (int v = 0; v < 4; v++)
                     if (x + v < p.N) o[v] = r[v];
             }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// FP16-sinogram backprojection of 64 slices on the matrix cores, bit for bit
+// bp_linear_f16_kernel's of the 16 x 16 tiles: the same FP16 operands (1, f)
+// and (s0, s1 - s0), t from the same 16 x 16 tile origins, one product pair per
+// pixel, slice and angle, added in angle order (an MFMA adds the products of a
+// row into the FP32 sum as v_dot2_f32_f16 adds its two; the zeros add nothing).
+//
+// A block of 32 pixels (4 x 8 or 8 x 4) meets at most 8 floors of t at an
+// angle when its long side runs along the angle's iso-lines (near 45 degrees,
+// where it meets 9, a second product takes floors 8 to 15).  With K = 16 halves
+// = 8 (s, d) pairs, v_mfma_f32_32x32x16_f16 is
+//   A [32 pixels][8 pairs]: lane m + 32 h holds (1, f) of pixel m at pair
+//     floor(t) - kb - 4 h of four, zeros elsewhere,
+//   B [8 pairs][32 slices]: lane n + 32 h the pairs kb + 4 h .. + 3 of slice n.
+//
+// The block shape follows the angle's class (|cos| >= |sin|: 4 wide, 8 tall;
+// else 8 wide, 4 tall).  A wave holds an 8 x 8 square as two blocks; row m =
+// 16 e + 4 py + px of a block (px, py < 4, e the block's second 4 pixels along
+// its long side) makes the change of shape a change of registers: the
+// upper half of block 0's sums and the lower half of block 1's trade places.
+//
+// The pairs come packed by f16_pack_kernel, rows of one detector and 64
+// slices; a chunk's rows go from global memory straight to LDS (two buffers,
+// one barrier per chunk).  Rows are 288 bytes apart there, so that the rows
+// the two halves of a wave read, four apart, use different banks.  A block may
+// read rows past its angle's: their weights are zero and what they hold is
+// finite unless a sample is not.  A non-finite sample meets the zero weights
+// of its neighbours as NaN: a wave that ends with a non-finite sum evaluates
+// its pixels again one by one (bp_f16_pixel).
+//
+// Bound: LDS latency under load and instruction issue.  A wave spends about 65
+// instructions, 6.4 KB of LDS reads and 4 products per angle on 64 pixels of 64
+// slices (bp_linear_f16_kernel 1.4 vector operations and 4 bytes of LDS per
+// pixel and slice), so the 64 slices share what a pixel costs; the sums take
+// half of the registers, which leaves four waves per SIMD, and the rows one
+// workgroup per CU.  512^2 x 1000 angles, 64 slices: 705 us with the packing
+// (45), 895 with bp_linear_f16_kernel.  Weights placed by compares instead of
+// the selector table, and each wave copying rows of every angle: 784.
+// ---------------------------------------------------------------------------
+typedef float f16v_t __attribute__((ext_vector_type(16)));
+constexpr int kPackSlices = 64;
+constexpr int kPackInfo = 128;      // ring of angle records, per 16 x 16 part of the tile
+constexpr int kPackPitch = 288;     // bytes between staged rows (18 16-byte pieces, the last two spare)
+constexpr int kPackSlack = 5120;    // zeroed bytes after a buffer: 16 rows and more
+
+// Packed rows of an angle: a zero row, detectors -1 .. D - 1, a zero row.
+__host__ __device__ constexpr int pack_rows(int D) { return D + 3; }
+// Staged rows of an angle: its window and two before (a block's first floor
+// lies up to one below, and the parts' t round otherwise than the tile's).
+__host__ __device__ constexpr int pack_staged(int W) { return W + 3; }
+__host__ __device__ constexpr int pack_stride(int W) { return (pack_staged(W) * kPackPitch + 1023) / 1024 * 1024; }
+__host__ __device__ constexpr int pack_buffer(int AE, int W) { return AE * pack_stride(W) + kPackSlack; }
+__host__ __device__ constexpr int pack_lds(int AE, int W, int parts) { return 2 * pack_buffer(AE, W) + kPackInfo * 32 * parts + 28 * 16; }
+// Products per block and angle.
+__host__ __device__ inline int pack_steps(float c, float s, float scale)
+{
+    const float ac = fabsf(c), as = fabsf(s), span = scale * (3.0f * fmaxf(ac, as) + 7.0f * fminf(ac, as)) + 0.02f;
+    return ((int)span + 2 + 7) / 8;   // floors a span can meet, eight per product
+}
+
+// x4 sinograms -> packed[P][pack_rows(D)][64] dwords (s, d), zero outside
+// [0, D) and past the last group of 4 slices.  Bound by memory: 1000 x 512,
+// 64 slices read 66 MB and write 132.
+__global__ void __launch_bounds__(256) f16_pack_kernel(const uint2* __restrict__ sino, int groups, int P, int D,
+                                                       uint4* __restrict__ packed)
+{
+    __shared__ uint2 tile[16][66];
+    const int p = blockIdx.y, RP = pack_rows(D), R0 = 64 * blockIdx.x;
+    for (int i = threadIdx.x; i < 16 * 65; i += 256) {
+        const int g = i / 65, j = i - g * 65, k = R0 - 2 + j;
+        tile[g][j] = g < groups && (unsigned)k < (unsigned)D ? sino[((long)g * P + p) * D + k] : make_uint2(0u, 0u);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * 16; i += 256) {
+        const int r = i / 16, g = i % 16;
+        if (R0 + r < RP)
+            packed[((long)p * RP + R0 + r) * 16 + g] =
+                __builtin_bit_cast(uint4, stage_pairs(tile[g][r], tile[g][r + 1]));
+    }
+}
+
+// Pixel (x, y) of one slice, sample by sample: row[4 k] is the slice's sample
+// k of angle 0; xa .. yb the corners of its 16 x 16 tile.
+__device__ __forceinline__ float bp_f16_pixel(const uint16_t* __restrict__ row, const float* __restrict__ cosT,
+                                              const float* __restrict__ sinT, const BpParams& p, float xa, float xb,
+                                              float ya, float yb, int x, int y)
+{
+    const float xq = ((float)x - p.center) * p.scale, yq = ((float)y - p.center) * p.scale;
+    float acc = 0.0f;
+#pragma unroll 1
+    for (int a = 0; a < p.P; a++, row += (long)p.D * kF16Group) {
+        const AngleWin w = angle_window(cosT[a], sinT[a], xa, xb, ya, yb, p.cI);
+        int k;
+        float f;
+        bp_split(__builtin_fmaf(yq, w.s, __builtin_fmaf(xq, w.c, w.negT)), k, f);
+        k += w.kabs - w.kmin;
+        _Float16 h0 = (_Float16)0.0f, h1 = h0;
+        if ((unsigned)k < (unsigned)p.D) h0 = __builtin_bit_cast(_Float16, row[(long)k * kF16Group]);
+        if ((unsigned)(k + 1) < (unsigned)p.D) h1 = __builtin_bit_cast(_Float16, row[(long)(k + 1) * kF16Group]);
+        acc = __builtin_amdgcn_fdot2(weight_pair(f), h2_t{h0, (_Float16)(h1 - h0)}, acc, false);
+    }
+    return acc;
+}
+
+// Workgroup x: a TX x TY tile of (up to) 64 slices, from `packed` (and the x4
+// sinogram for non-finite pixels); each wave an 8 x 8 square.
+template <int TX, int TY, int WPE>
+__global__ void __launch_bounds__(TX* TY, WPE) bp_f16_mfma_kernel(const uint4* __restrict__ packed,
+                                                                  const uint2* __restrict__ sino,
+                                                                  float* __restrict__ img,
+                                                                  const float* __restrict__ cosT,
+                                                                  const float* __restrict__ sinT, int slices, BpParams p)
+{
+    constexpr int NT = TX * TY, NW = NT / 64, NB = 2, PX = TX / 16, PARTS = PX * (TY / 16), PITCH = kPackPitch;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int AE = p.AE, stride = pack_stride(p.W), bufsz = pack_buffer(AE, p.W), RP = pack_rows(p.D);
+    char* rows = smem;
+    float4* info = reinterpret_cast<float4*>(rows + 2 * bufsz);   // per part: (cos, sin, -T, LDS address of floor 0)
+    // (offset to a block's smallest t, steps (negative: class B), packed row of staged row 0, -)
+    int4* info2 = reinterpret_cast<int4*>(info + kPackInfo * PARTS);
+    uint4* tab = reinterpret_cast<uint4*>(info2 + kPackInfo * PARTS);   // byte selectors that move (1, f) to pair q - 12
+
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    int2 txy;
+    bp_work(p, txy);
+    const int x0 = txy.x * TX, y0 = txy.y * TY;
+    const int bx = x0 + (wave % (TX / 8)) * 8, by = y0 + (wave / (TX / 8)) * 8;   // the wave's square
+    const int part = (bx - x0) / 16 + PX * ((by - y0) / 16);
+    const int m = lane & 31, h = lane >> 5;
+    bool use = false;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {   // 32 of the square's pixels each
+        const int x = bx + (m & 7), y = by + 4 * i + (m >> 3);
+        use |= x < p.N && y < p.N && !(p.mask && bp_outside(x, y, p.N, p.center));
+    }
+    const bool active = __any(use);
+    const int nch = __syncthreads_or(use) ? (p.P + AE - 1) / AE : 0;
+
+    f16v_t acc[2][NB];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < NB; u++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][u][v] = 0.0f;
+    // the lane's pixel of the two blocks, for the current class
+    float X[2], Y[2];
+    int cls = 0;
+    auto set_class = [&](int c) {
+        const int px = m & 3, py = m >> 2 & 3, e = 4 * (m >> 4);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            X[i] = ((float)(bx + px + (c ? e : 4 * i)) - p.center) * p.scale;
+            Y[i] = ((float)(by + py + (c ? 4 * i : e)) - p.center) * p.scale;
+        }
+        if (c != cls)
+#pragma unroll
+            for (int u = 0; u < NB; u++)
+#pragma unroll
+                for (int v = 0; v < 8; v++) {
+                    const float t = acc[0][u][8 + v];
+                    acc[0][u][8 + v] = acc[1][u][v];
+                    acc[1][u][v] = t;
+                }
+        cls = c;
+    };
+    set_class(0);
+
+    auto coord = [&](int x) { return ((float)x - p.center) * p.scale; };
+    const unsigned rbase = lds_address(rows), tbase = lds_address(tab + 12), m4 = (unsigned)m * 4u;
+    // records of angles 64 b .. 64 b + 63 (AE divides 64), slot angle % 128, one
+    // part per wave, other waves each time
+    auto make_info = [&](int b) {
+        const int q = (wave + NW - PARTS * b % NW) % NW;
+        if (q >= PARTS) return;
+        const int pa = 64 * b + lane, pc = min(pa, p.P - 1), r = pa % kPackInfo;
+        const int ch = pc / AE, a = pc - ch * AE;
+        const int xs = x0 + 16 * (q % PX), ys = y0 + 16 * (q / PX);
+        const AngleWin t = angle_window(cosT[pc], sinT[pc], coord(x0), coord(x0 + TX - 1), coord(y0), coord(y0 + TY - 1), p.cI);
+        const AngleWin w = angle_window(cosT[pc], sinT[pc], coord(xs), coord(xs + 15), coord(ys), coord(ys + 15), p.cI);
+        const bool tall = fabsf(w.c) >= fabsf(w.s);
+        const float lc = fminf(w.c, 0.0f) * p.scale, ls = fminf(w.s, 0.0f) * p.scale;
+        const int steps = pack_steps(w.c, w.s, p.scale), row0 = w.kabs - w.kmin - t.kabs + 2;   // staged row of floor 0
+        info[q * kPackInfo + r] = make_float4(
+            w.c, w.s, w.negT, __uint_as_float(rbase + (unsigned)((ch & 1) * bufsz + a * stride + row0 * PITCH)));
+        info2[q * kPackInfo + r] = make_int4(
+            __float_as_int((tall ? 3.0f * lc + 7.0f * ls : 7.0f * lc + 3.0f * ls) - 0.01f), tall ? steps : -steps, t.kabs, 0);
+    };
+    // chunk ch's rows into its buffer (NW / AE waves per angle), 1 KB at a time
+    const int per = stride / 1024, wpa = NW / AE, sa = wave / wpa, sj = wave - sa * wpa;
+    auto stage = [&](int ch, lds_bytes* buf) {
+        const int pa = ch * AE + sa;
+        if (pa >= p.P) return;
+        const int row0 = __builtin_amdgcn_readfirstlane(info2[pa % kPackInfo].z);
+        const char* base = reinterpret_cast<const char*>(packed) + (long)pa * RP * 256;
+        unsigned o = (unsigned)(64 * sj + lane);   // 16-byte piece; o / 18 the row (o < 2000)
+        buf += sa * stride + sj * 1024;
+        for (int j = sj; j < per; j += wpa) {
+            const unsigned r = __umul24(o, 3641u) >> 16;
+            const unsigned at = ((unsigned)clamp_index(row0 + (int)r, RP - 1) * 16u + min(o - __umul24(r, 18u), 15u)) * 16u;
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + at), buf, 16, 0, 0);
+            o += 64u * (unsigned)wpa;
+            buf += wpa * 1024;
+        }
+    };
+    if (nch) {
+        for (int i = tid; i < 2 * bufsz / 16; i += NT) reinterpret_cast<uint4*>(rows)[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (tid < 28) {
+            unsigned sel[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) sel[j] = tid - 12 == j ? 0x03020100u : 0x0c0c0c0cu;
+            tab[tid] = make_uint4(sel[0], sel[1], sel[2], sel[3]);
+        }
+        make_info(0);
+        make_info(1);
+        __syncthreads();
+        stage(0, (lds_bytes*)rows);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    // next: the buffer of chunk ch + 1, which nothing else touches before the
+    // barrier (as in bp_split_kernel)
+    auto chunk = [&](int ch, lds_bytes* __restrict__ next) __attribute__((always_inline)) {
+        const int p0 = ch * AE, na = min(AE, p.P - p0);
+        if (ch + 1 < nch) stage(ch + 1, next);
+        if (!active) return;
+        const float4* inf = info + part * kPackInfo + p0 % kPackInfo;
+        const int4* inf2 = info2 + part * kPackInfo + p0 % kPackInfo;
+        float4 in = inf[0];
+        int2 in2 = *reinterpret_cast<const int2*>(inf2);
+        for (int a = 0; a < na; a++) {
+            const int st = __builtin_amdgcn_readfirstlane(in2.y);
+            if ((st < 0) != (cls != 0)) set_class(st < 0);
+            const int steps = st < 0 ? -st : st;
+            const float off = __int_as_float(in2.x);
+            unsigned at[2], w[2], tq[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const float t = __builtin_fmaf(Y[i], in.y, __builtin_fmaf(X[i], in.x, in.z));
+                // lane 0 holds the block's first pixel
+                const float t0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(t)));
+                const int kb = floor_to_int(t0 + off) + 4 * h;
+                int k;
+                float f;
+                bp_split(t, k, f);
+                w[i] = __builtin_bit_cast(unsigned, weight_pair(f));
+                tq[i] = tbase + (unsigned)(k - kb) * 16u;
+                at[i] = __float_as_uint(in.w) + m4 + (unsigned)__mul24(kb, PITCH);
+            }
+            const int an = min(a + 1, na - 1);   // the next angle's record, while this one is multiplied
+            in = inf[an];
+            in2 = *reinterpret_cast<const int2*>(inf2 + an);
+            for (int sp = 0;;) {
+                lds_u4 B[2][NB], sel[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    sel[i] = lds_load<lds_u4>(tq[i]);
+#pragma unroll
+                    for (int u = 0; u < NB; u++) {
+                        asm("" : "+v"(at[i]));   // two-address reads of one operand
+#pragma unroll
+                        for (int j = 0; j < 4; j++) B[i][u][j] = lds_load<unsigned>(at[i] + PITCH * j);
+                        at[i] += u + 1 < NB ? 128 : 8 * PITCH - 128 * (NB - 1);   // the next product's after the last
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);   // every read is under way before the first product
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    lds_u4 A;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) A[j] = __builtin_amdgcn_perm(0u, w[i], sel[i][j]);
+#pragma unroll
+                    for (int u = 0; u < NB; u++)
+                        acc[i][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            __builtin_bit_cast(h8_t, A), __builtin_bit_cast(h8_t, B[i][u]), acc[i][u], 0, 0, 0);
+                }
+                if (__builtin_expect(++sp >= steps, 1)) break;
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    tq[i] -= 8 * 16;
+                }
+            }
+        }
+    };
+    for (int ch = 0; ch < nch; ch++) {
+        // chunks ch and ch + 1 lie in blocks of 64 angles ch AE / 64 and the
+        // next: the ring's other half is free for the block after
+        if (ch > 0 && ch * AE % 64 == 0 && ch * AE + 64 < p.P) make_info(ch * AE / 64 + 1);
+        chunk(ch, (lds_bytes*)rows + ((ch + 1) & 1) * bufsz);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's part of chunk ch + 1 is in LDS
+        __syncthreads();
+    }
+    set_class(0);
+    // lane (n = m, h): register 8 e + 4 j + v of block i is pixel
+    // (4 i + v, 4 e + 2 j + h) of the square, slice 32 u + n
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            float z = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 16; v++) z = __builtin_fmaf(acc[i][u][v], 0.0f, z);
+            bad |= !(z == 0.0f);
+            if (32 * u + m >= slices) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int x = bx + 4 * i, y = by + 2 * r + h;
+                if (x >= p.N || y >= p.N) continue;
+                float* o = img + (long)(32 * u + m) * p.N * p.N + (long)y * p.N + x;
+                f4_t w;
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    w[v] = p.mask && bp_outside(x + v, y, p.N, p.center) ? p.maskingValue
+                                                                         : acc[i][u][4 * r + v] * p.norm * p.out_scale;
+                if (x + 4 <= p.N && reinterpret_cast<uintptr_t>(o) % 16 == 0) {
+                    *reinterpret_cast<f4_t*>(o) = w;
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        if (x + v < p.N) o[v] = w[v];
+                }
+            }
+        }
+    if (__any(bad)) {
+        const int xs = x0 + 16 * (part % PX), ys = y0 + 16 * (part / PX);
+#pragma unroll 1
+        for (int i = 0; i < 32 * NB; i++) {   // (pixel of the lane's rows, u)
+            const int x = bx + (i & 7), y = by + 2 * (i >> 3 & 3) + h, sl = 32 * (i >> 5) + m;
+            if (sl >= slices || x >= p.N || y >= p.N || (p.mask && bp_outside(x, y, p.N, p.center))) continue;
+            const uint16_t* row = reinterpret_cast<const uint16_t*>(sino + (long)(sl / kF16Group) * p.P * p.D) + sl % kF16Group;
+            img[(long)sl * p.N * p.N + (long)y * p.N + x] =
+                bp_f16_pixel(row, cosT, sinT, p, coord(xs), coord(xs + 15), coord(ys), coord(ys + 15), x, y) * p.norm *
+                p.out_scale;
         }
     }
 }
@@ -2465,6 +2810,102 @@ extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, int* m
             }
         }
         *min_slices = 1 + (int)(kSplitSlices * best / plain);
+    });
+}
+
+// -------------------------------- FP16 backprojection of 64 slices at once --
+// Used by the mixed chain for groups of many frames (chain.hip), in place of an
+// FP16 variant whose results it has bit for bit.
+// Bytes of packed samples for 64 slices, or 0 where the handle's geometry or
+// its FP16 variant (another tile than 16 x 16, or shared angles) has no
+// counterpart there.
+extern "C" size_t risa_bp_f16_pack_bytes(risa_bp_t h)
+{
+    const risa_geom& g = h->g;
+    const BpF16Variant& v = kF16Variants[h->variant_f16];
+    if (g.useTextureMemory || g.interpolationType == 1 || h->lut.scale > kSplitMaxScale || v.tx != 16 || v.ty != 16 || v.q != 1)
+        return 0;
+    return (size_t)g.numberOfParallelProjections * pack_rows(g.numberOfParallelDetectors) * kPackSlices * 4;
+}
+
+// Up to 64 slices of the x4 layout -> images; `packed`: risa_bp_f16_pack_bytes
+// of scratch, 16-byte aligned.
+extern "C" int risa_bp_run_f16_packed(risa_bp_t h, const uint16_t* sino_x4, float in_scale, int slices, void* packed,
+                                      float* img, hipStream_t s)
+{
+    return guarded("risa_bp_run_f16_packed", [&] {
+        if (slices < 1 || slices > kPackSlices || !(in_scale > 0)) fail(RISA_ERR_ARG, "bad argument");
+        if (risa_bp_f16_pack_bytes(h) == 0) fail(RISA_ERR_UNSUPPORTED, "no packed form of this FP16 variant");
+        constexpr int kTile = 32, kParts = 4;
+        BpParams p = make_params(h, kTile, kTile);
+        p.out_scale = 1.0f / in_scale;
+        p.AE = 4;
+        while (p.AE > 1 && pack_lds(p.AE, p.W, kParts) > kMaxSplitLds) p.AE /= 2;
+        const int lds = pack_lds(p.AE, p.W, kParts);
+        if (lds > kMaxSplitLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %d B of LDS", lds);
+        dim3 grid(p.tilesX * ceil_div(p.N, kTile), 1);
+        p.xg = xcd_groups(grid.x, 1);
+        const long off = h->order_off[0];   // the first FP32 variant has this tile
+        p.order = p.xg && off >= 0 ? h->tile_order.ptr + off : nullptr;
+        const uint2* x4 = reinterpret_cast<const uint2*>(sino_x4);
+        uint4* pk = reinterpret_cast<uint4*>(packed);
+        hipLaunchKernelGGL(f16_pack_kernel, dim3(ceil_div(pack_rows(p.D), 64), p.P), dim3(256), 0, s, x4,
+                           ceil_div(slices, kF16Group), p.P, p.D, pk);
+        check_launch("f16_pack_kernel");
+        hipLaunchKernelGGL((bp_f16_mfma_kernel<kTile, kTile, 4>), grid, dim3(kTile * kTile), lds, s, pk, x4, img, h->cosT.ptr, h->sinT.ptr, slices, p);
+        check_launch("bp_f16_mfma_kernel");
+    });
+}
+
+// Times it at 64 slices against the handle's FP16 variant: `min_slices` is the
+// batch from which it is the faster one (its cost does not depend on the
+// slices up to 64), or more than 64 if never.
+extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int* min_slices)
+{
+    return guarded("risa_bp_tune_f16_packed", [&] {
+        DeviceGuard dg(h->device);
+        const size_t ns = (size_t)h->g.numberOfParallelProjections * h->g.numberOfParallelDetectors;
+        const size_t ni = (size_t)h->g.numberOfPixels * h->g.numberOfPixels;
+        DeviceBuffer<uint16_t> sino(ns * kPackSlices);
+        DeviceBuffer<float> img(ni * kPackSlices);
+        DeviceBuffer<char> packed(risa_bp_f16_pack_bytes(h));
+        hipLaunchKernelGGL(tune_fill_f16_kernel, dim3(1024), dim3(256), 0, s, sino.ptr, (long)sino.count);
+        check_launch("tune_fill_f16_kernel");
+        hipEvent_t ev[2] = {};
+        auto destroy = [&] {
+            for (hipEvent_t e : ev)
+                if (e) (void)hipEventDestroy(e);
+        };
+        try {
+            for (hipEvent_t& e : ev) RISA_HIP_CHECK(hipEventCreate(&e));
+            auto time_it = [&](auto&& launch) {
+                launch();
+                RISA_HIP_CHECK(hipEventRecord(ev[0], s));
+                for (int it = 0; it < 5; it++) launch();
+                RISA_HIP_CHECK(hipEventRecord(ev[1], s));
+                RISA_HIP_CHECK(hipEventSynchronize(ev[1]));
+                float ms = 0;
+                RISA_HIP_CHECK(hipEventElapsedTime(&ms, ev[0], ev[1]));
+                return ms;
+            };
+            float plain = 1e30f, best = 1e30f;
+            for (int round = 0; round < 2; round++) {
+                plain = std::min(plain, time_it([&] {
+                                     launch_f16x4(h, h->variant_f16, reinterpret_cast<const uint2*>(sino.ptr), 1.0f,
+                                                  kPackSlices, img.ptr, s);
+                                 }));
+                best = std::min(best, time_it([&] {
+                                    if (risa_bp_run_f16_packed(h, sino.ptr, 1.0f, kPackSlices, packed.ptr, img.ptr, s) !=
+                                        RISA_OK)
+                                        fail(RISA_ERR_HIP, "%s", risa_last_error());
+                                }));
+            }
+            *min_slices = 1 + (int)(kPackSlices * best / plain);
+        } catch (...) {
+            destroy();
+            throw;
+        }
+        destroy();
     });
 }
 

@@ -21,7 +21,11 @@
 //        MFMA writes the FP16 sinogram in the 4-slice interleaved layout and
 //        the FP16-sinogram / FP32-accumulate backprojection runs the group in
 //        one launch, so one lane's front stages overlap the other's
-//        backprojection.
+//        backprojection.  Chains of at least 128 frames take groups of 64 and
+//        backproject those of at least split_min frames on the matrix cores
+//        (bp_f16_mfma_kernel, the same bits), where timing both at creation
+//        finds that the faster way: 512 frames of 512^2 x 1000 angles 8.00 ms
+//        a call, 8.95 with bp_linear_f16_kernel.
 #include "device_common.h"
 
 #include <cmath>
@@ -33,6 +37,10 @@ int risa_filter_run_oop(risa_filter_t h, const float* in, float* out, long rows,
 double risa_filter_l1(risa_filter_t h);
 int risa_fan2para_gain(risa_fan2para_t h, double* gain);
 extern "C" size_t risa_bp_split_bytes(risa_bp_t h);
+extern "C" size_t risa_bp_f16_pack_bytes(risa_bp_t h);
+extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int* min_slices);
+extern "C" int risa_bp_run_f16_packed(risa_bp_t h, const uint16_t* sino_x4, float in_scale, int slices, void* packed,
+                                      float* img, hipStream_t s);
 extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, int* min_slices);
 extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, float scale, int slices, void* packed, float* img,
                       hipStream_t s);
@@ -44,6 +52,7 @@ constexpr int kPlainMaxPer = 16;          // frames per lane step of a PLAIN cha
 constexpr int kSplitPer = 32;             // and of 64 frames or more (also the split backprojector's slices)
 constexpr int kMixedLanes = 2;            // streams in MIXED mode
 constexpr int kMixedMaxPer = 32;          // frames per lane step in MIXED mode, at most (a multiple of 4)
+constexpr int kPackPer = 64;              // and of a MIXED chain that backprojects groups on the matrix cores
 }  // namespace
 
 // Graph executables a chain keeps (one per buffer set and call shape); the
@@ -191,6 +200,16 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
                 // group 245 us, two of 4 in two lanes 292; 48 frames as 32 + 16
                 // 978, as 24 + 24 1160)
                 h->per = std::min(kMixedMaxPer, (max_frames + 3) / 4 * 4);
+                ok(risa_hip_bp_autotune_f16(h->bp, h->per, nullptr));
+                if (max_frames >= kMixedLanes * kPackPer && (h->split_bytes = risa_bp_f16_pack_bytes(h->bp)) > 0) {
+                    ok(risa_bp_tune_f16_packed(h->bp, nullptr, &h->split_min));
+                    if (h->split_min <= kPackPer) {
+                        h->per = kPackPer;
+                        h->split_shape = 0;
+                        h->split_bytes = (h->split_bytes + 255) / 256 * 256;
+                        h->split_buf.resize(h->split_bytes * kMixedLanes);
+                    }
+                }
                 h->lanes = std::min(kMixedLanes, (max_frames + h->per - 1) / h->per);
                 const size_t slots = (size_t)h->lanes * h->per;
                 h->att_buf.resize(fan * slots);
@@ -217,8 +236,6 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
                     // tuned above
                 } else if (h->per > 1) ok(risa_hip_bp_autotune_batch(h->bp, std::min(kPlainLanes * kPlainMaxPer, h->lanes * h->per), nullptr));
                 else ok(risa_hip_bp_autotune_slices(h->bp, h->lanes, nullptr));
-            } else {
-                ok(risa_hip_bp_autotune_f16(h->bp, h->per, nullptr));
             }
             RISA_HIP_CHECK(hipDeviceSynchronize());
         } catch (...) {
@@ -267,7 +284,11 @@ static void enqueue(risa_chain_t h, const uint16_t* raw, const int32_t* planes, 
             ok(risa_hip_attenuation_run_batch(h->att, raw + f * fan, planes + f, n, att, ls));
             ok(risa_hip_fan2para_run_batch(h->f2p, att, planes + f, n, pb, ls));
             ok(risa_hip_filter_run_f16x4(h->filt, pb, hb, n, kF16SinoScale, ls));
-            ok(risa_hip_bp_run_f16x4(h->bp, hb, kF16SinoScale, n, img + f * out, ls));
+            if (h->split_shape >= 0 && n >= h->split_min)
+                ok(risa_bp_run_f16_packed(h->bp, hb, kF16SinoScale, n, h->split_buf.ptr + k * h->split_bytes,
+                                          img + f * out, ls));
+            else
+                ok(risa_hip_bp_run_f16x4(h->bp, hb, kF16SinoScale, n, img + f * out, ls));
         }
     }
     for (int k = 0; k < lanes; k++) {
