@@ -64,30 +64,44 @@ __device__ __attribute__((noinline)) float rebin_ray(const float* __restrict__ f
 constexpr int kRebinBlock = 16;
 constexpr int kPatchMax = 512;
 // Workgroups a launch aims at before a plane's frames share one.  A workgroup
-// walks its frames one after another, each a load, two barriers and the rays:
-// 2 us a frame whatever the block count, so few blocks need more workgroups;
-// each further one reads the block's table entries again.  32 frames of
-// 256 x 500 (512 blocks): 57 us in one group, 25 / 22 / 28 aiming at 2048 /
-// 4096 / 16384; 8 frames of 512 x 1000 in two planes (2 x 2016 blocks): 25 /
-// 29 / 33, so the line lies between.
+// walks its frames one or two at a time, each step a load, two barriers and
+// the rays: about 2 us whatever the block count, so few blocks need more
+// workgroups; each further one reads the block's table entries again.  One
+// frame at a time, 32 frames of 256 x 500 (512 blocks): 57 us in one group,
+// 25 / 22 / 28 aiming at 2048 / 4096 / 16384; 8 frames of 512 x 1000 in two
+// planes (2 x 2016 blocks): 25 / 29 / 33, so the line lies between.
 constexpr long kRebinFill = 3072;
 
-// Ray of one slot from its LDS patch (no wrap inside a patch).
-__device__ __forceinline__ float patch_ray(const float* __restrict__ pt, int4 box, uint32_t idx, float ft, float fg)
-{
-    const int tb = (int)(idx & 0xFFFFu) - box.x;
-    const int gb = (int)((idx >> 16) & 0x7FFFu) - box.y;
-    const int a = tb * box.w + gb;
-    const float W1 = pt[a], W2 = pt[a + 1], W3 = pt[a + box.w], W4 = pt[a + box.w + 1];
-    const float V1 = W1 + ft * (W3 - W1);
-    const float V2 = W2 + ft * (W4 - W2);
-    return V1 + fg * (V2 - V1);
-}
+// The values of one sample in the NF frames a workgroup interpolates at once,
+// side by side in LDS.
+template <int NF>
+struct FrameVals {
+    float v[NF];
+};
 
-__device__ __forceinline__ float slot_ray(const float* __restrict__ fr, const float* __restrict__ pt, int4 box,
-                                          uint32_t idx, float ft, float fg, int Df, int Pf)
+// Rays of one slot from its LDS patch (no wrap inside a patch), or from global
+// memory.
+template <int NF>
+__device__ __forceinline__ FrameVals<NF> slot_rays(const float* const (&fr)[NF], const FrameVals<NF>* pt, int4 box,
+                                                   uint32_t idx, float ft, float fg, int Df, int Pf)
 {
-    return box.z > 0 ? patch_ray(pt, box, idx, ft, fg) : rebin_ray(fr, idx, ft, fg, Df, Pf);
+    FrameVals<NF> z;
+    if (box.z > 0) {
+        const int tb = (int)(idx & 0xFFFFu) - box.x;
+        const int gb = (int)((idx >> 16) & 0x7FFFu) - box.y;
+        const FrameVals<NF>* q = pt + tb * box.w + gb;
+        const FrameVals<NF> W1 = q[0], W2 = q[1], W3 = q[box.w], W4 = q[box.w + 1];
+#pragma unroll
+        for (int k = 0; k < NF; k++) {
+            const float V1 = W1.v[k] + ft * (W3.v[k] - W1.v[k]);
+            const float V2 = W2.v[k] + ft * (W4.v[k] - W2.v[k]);
+            z.v[k] = V1 + fg * (V2 - V1);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NF; k++) z.v[k] = rebin_ray(fr[k], idx, ft, fg, Df, Pf);
+    }
+    return z;
 }
 
 // Flag-weighted mean of the two rays of one internal sample (:153-158).
@@ -97,11 +111,16 @@ __device__ __forceinline__ float mix_rays(bool r1, bool r2, float z1, float z2)
     return r1 ? z1 : (r2 ? z2 : 0.0f);
 }
 
+// NF frames at once: a frame costs its workgroup a load's latency, two barriers
+// and the taps' addresses, and two frames share them (an odd last frame goes
+// with itself).  32 frames of 512 x 1000 in two planes: 66 -> 56 us, 16 frames
+// of 256 x 500 13.9 -> 12.4; four at once take 53 and 17.7 (32 KB of patches).
+template <int NF>
 __global__ void __launch_bounds__(256) rebin_kernel(const uint4* __restrict__ table, const int4* __restrict__ boxes,
                                                     const int2* __restrict__ order, int Df, int Pf, int D, int P,
                                                     long table_plane_stride, long box_plane_stride, FrameGroups fg)
 {
-    __shared__ float patch[4 * kPatchMax];
+    __shared__ __attribute__((aligned(8))) FrameVals<NF> patch[4 * kPatchMax];
     // workgroup x takes output block order[plane][x]: blocks with a slot that
     // gathers from global memory first, so the slowest blocks start early
     const int grp = blockIdx.y;
@@ -153,35 +172,49 @@ __global__ void __launch_bounds__(256) rebin_kernel(const uint4* __restrict__ ta
             goff[sl][j] = have[sl][j] ? (b.x + r) * Df + b.y + (t - r * b.w) : 0;
         }
     }
-    float pf[4][kPer];
-    auto load_frame = [&](int u) {
-        const float* __restrict__ fr = fg.fan[first + u];
+    FrameVals<NF> pf[4][kPer];
+    const float* fr[NF];
+    auto frames = [&](int u) {
+#pragma unroll
+        for (int k = 0; k < NF; k++) fr[k] = fg.fan[first + min(u + k, n - 1)];
+    };
+    auto load_frames = [&](int u) {
+        frames(u);
 #pragma unroll
         for (int sl = 0; sl < 4; sl++)
 #pragma unroll
             for (int j = 0; j < kPer; j++)
-                if (have[sl][j]) pf[sl][j] = fr[goff[sl][j]];
+                if (have[sl][j])
+#pragma unroll
+                    for (int k = 0; k < NF; k++) pf[sl][j].v[k] = fr[k][goff[sl][j]];
     };
-    if (n > 0) load_frame(0);
-    for (int u = 0; u < n; u++) {
-        const float* __restrict__ fr = fg.fan[first + u];
-        if (u > 0) __syncthreads();   // the previous frame's patches are consumed
+    if (n > 0) load_frames(0);
+    for (int u = 0; u < n; u += NF) {
+        if (u > 0) __syncthreads();   // the previous frames' patches are consumed
 #pragma unroll
         for (int sl = 0; sl < 4; sl++)
 #pragma unroll
             for (int j = 0; j < kPer; j++)
                 if (have[sl][j]) patch[sl * kPatchMax + threadIdx.x + j * 256] = pf[sl][j];
         __syncthreads();
-        if (u + 1 < n) load_frame(u + 1);
+        if (u + NF < n) load_frames(u + NF);
         if (!inside) continue;
-        float z[4];
+        frames(u);
+        FrameVals<NF> z[4];
 #pragma unroll
-        for (int sl = 0; sl < 4; sl++)
-            z[sl] = (id[sl] >> 31) ? slot_ray(fr, patch + sl * kPatchMax, box[sl], id[sl], ft[sl], fgm[sl], Df, Pf)
-                                   : 0.0f;
-        const float zA = mix_rays((id[0] >> 31) != 0, (id[1] >> 31) != 0, z[0], z[1]);
-        const float zB = mix_rays((id[2] >> 31) != 0, (id[3] >> 31) != 0, z[2], z[3]);
-        fg.par[first + u][e] = 0.5f * zA + 0.5f * zB;
+        for (int sl = 0; sl < 4; sl++) {
+#pragma unroll
+            for (int k = 0; k < NF; k++) z[sl].v[k] = 0.0f;
+            if (id[sl] >> 31)
+                z[sl] = slot_rays<NF>(fr, patch + sl * kPatchMax, box[sl], id[sl], ft[sl], fgm[sl], Df, Pf);
+        }
+#pragma unroll
+        for (int k = 0; k < NF; k++) {
+            if (u + k >= n) break;
+            const float zA = mix_rays((id[0] >> 31) != 0, (id[1] >> 31) != 0, z[0].v[k], z[1].v[k]);
+            const float zB = mix_rays((id[2] >> 31) != 0, (id[3] >> 31) != 0, z[2].v[k], z[3].v[k]);
+            fg.par[first + u + k][e] = 0.5f * zA + 0.5f * zB;
+        }
     }
 }
 
@@ -526,7 +559,9 @@ static void launch_rebin_at(risa_fan2para_t h, FanAt fan, const int32_t* planes,
             pos += cnt;
         }
         dim3 grid(blocks, groups);
-        hipLaunchKernelGGL(rebin_kernel, grid, dim3(256), 0, s, reinterpret_cast<const uint4*>(h->table.ptr),
+        bool shared = false;   // a workgroup with two frames or more
+        for (int q = 0; q < groups; q++) shared |= fg.count[q] > 1;
+        hipLaunchKernelGGL(shared ? rebin_kernel<2> : rebin_kernel<1>, grid, dim3(256), 0, s, reinterpret_cast<const uint4*>(h->table.ptr),
                            h->boxes.ptr, h->order.ptr, Df, Pf, D, P, (long)(h->plane_words / 4), h->box_plane, fg);
         check_launch("rebin_kernel");
         if (D % 2 != 0) {
