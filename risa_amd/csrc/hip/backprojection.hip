@@ -87,6 +87,10 @@ __device__ __forceinline__ int bp_work(const BpParams& p, int2& txy)
         txy = bp_tile_xy(blockIdx.x, p);
         return blockIdx.y;
     }
+    if (p.xg == 2) {   // one group: heaviest first over all XCDs
+        txy = bp_tile_of_rank(p.order[blockIdx.x], p);
+        return blockIdx.y;
+    }
     const int T = gridDim.x, G = gridDim.y;
     const long L = blockIdx.x + (long)blockIdx.y * T;
     const int xcd = (int)(L & 7);
@@ -910,7 +914,7 @@ __global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_kernel(const ui
 // two-address reads deliver, against about 195 clocks of vector and matrix
 // issue; more waves (6 or 8 per SIMD rather than 4) hide the rest: a wave
 // issues one instruction in 8 clocks at best.  512^2 x 1000 angles, 32 slices:
-// 14.7 us per slice with two launches in flight (packing included, 0.65),
+// 14.1 us per slice with two launches in flight (packing included, 0.65),
 // bp_linear_kernel 24.5; relative RMSE against float64 2.64e-6 and 2.60e-6.
 // ---------------------------------------------------------------------------
 typedef float f4_t __attribute__((ext_vector_type(4)));
@@ -2747,9 +2751,13 @@ extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, floa
         const int lds = split_lds(p.AE, p.W);
         if (lds > kMaxSplitLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %d B of LDS", lds);
         dim3 grid(p.tilesX * ceil_div(p.N, v.ty), 1);
-        p.xg = xcd_groups(grid.x, 1);
         const long off = h->order_off[(size_t)v.variant];
-        p.order = p.xg && off >= 0 ? h->tile_order.ptr + off : nullptr;
+        // heaviest tiles first over the whole chip: ranges of tiles per XCD
+        // leave the XCDs of the image's corners idle early (32 slices of
+        // 512^2 x 1000, two launches in flight: 450 us, 472 with ranges; 256
+        // frames 4.14 ms, 4.35)
+        p.order = off >= 0 ? h->tile_order.ptr + off : nullptr;
+        p.xg = p.order ? 2 : 0;
         unsigned* pk = reinterpret_cast<unsigned*>(packed);
         hipLaunchKernelGGL(split_pack_kernel, dim3(ceil_div(split_rows(p.D) - 2, 32), p.P), dim3(256), 0, s, sino,
                            slices, p.P, p.D, scale, pk);
@@ -2844,6 +2852,7 @@ extern "C" int risa_bp_run_f16_packed(risa_bp_t h, const uint16_t* sino_x4, floa
         const int lds = pack_lds(p.AE, p.W, kParts);
         if (lds > kMaxSplitLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %d B of LDS", lds);
         dim3 grid(p.tilesX * ceil_div(p.N, kTile), 1);
+        // ranges of tiles per XCD: 705 us, 720 heaviest first over the chip
         p.xg = xcd_groups(grid.x, 1);
         const long off = h->order_off[0];   // the first FP32 variant has this tile
         p.order = p.xg && off >= 0 ? h->tile_order.ptr + off : nullptr;

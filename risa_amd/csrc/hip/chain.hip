@@ -14,7 +14,7 @@
 //        frames take groups of 32 and backproject those of at least split_min
 //        frames on the matrix cores (bp_split_kernel), where timing both at
 //        creation finds that the faster way: 256 frames of 512^2 x 1000 angles
-//        4.28 ms a call, 6.70 with bp_linear_kernel; 256^2 x 500 stays with
+//        4.15 ms a call, 6.67 with bp_linear_kernel; 256^2 x 500 stays with
 //        the latter (158 us per 32 slices against 208).
 // MIXED: groups of `per` consecutive frames (a multiple of 4, up to 32) dealt
 //        to `lanes` streams the same way; per group the DFT-GEMM filter on
