@@ -40,7 +40,7 @@ struct BpParams {
     float out_scale;     // multiplies sum * norm (1/in_scale for FP16 input)
     int AE;              // angles per staged chunk
     int zx, zy;          // log2 of the tile grid's width / height for the XCD-aware order, or -1
-    int xg;              // slice groups dealt to XCDs whole (bp_work), set per launch
+    int xg;              // 1: slice groups dealt to XCDs whole, 2: heaviest tiles first (bp_work), set per launch
     const int* order;    // bp_work's dispatch order tables (4 of tilesX * tilesY ranks) or null
 };
 
@@ -68,14 +68,15 @@ __device__ __forceinline__ int2 bp_tile_xy(int b, const BpParams& p)
 }
 
 // Tile and slice group of workgroup (blockIdx.x, blockIdx.y) of a grid of
-// T = gridDim.x tiles x G = gridDim.y slice groups.  With p.xg (T a multiple
+// T = gridDim.x tiles x G = gridDim.y slice groups.  With p.xg = 1 (T a multiple
 // of 8, and G a multiple or a divisor of 8) whole slice groups go to XCDs:
 // workgroup L = x + y T runs on XCD L % 8 as that XCD's (L / 8)-th; for
 // G >= 8 each XCD takes G / 8 groups, all their tiles; for G < 8, 8 / G XCDs
 // share a group, each a contiguous range of its tile order.  One XCD's L2
 // then holds few sinograms and each is fetched from HBM about once, where
 // splitting every slice's tiles over all 8 XCDs fetches it up to 8 times.
-// Otherwise the tile order of bp_tile_xy and group blockIdx.y.  Within an
+// With p.xg = 2 the tiles go heaviest first over all XCDs, and without p.xg in
+// the tile order of bp_tile_xy, group blockIdx.y either way.  Within an
 // XCD's range the tiles are dispatched heaviest first when p.order is set
 // (table lm = log2 of the XCDs per group: each range of T / 2^lm ranks
 // sorted by the tile's pixels inside the mask), so the workgroups that end
@@ -87,7 +88,7 @@ __device__ __forceinline__ int bp_work(const BpParams& p, int2& txy)
         txy = bp_tile_xy(blockIdx.x, p);
         return blockIdx.y;
     }
-    if (p.xg == 2) {   // one group: heaviest first over all XCDs
+    if (p.xg == 2) {   // heaviest first over all XCDs, group by group
         txy = bp_tile_of_rank(p.order[blockIdx.x], p);
         return blockIdx.y;
     }
@@ -2569,6 +2570,22 @@ extern "C" int risa_hip_bp_create(const risa_geom* g, int device, risa_bp_t* out
     });
 }
 
+// bp_work's order for a launch whose tile shape's tables lie at `off` (-1: none,
+// the tiles no multiple of 8).  Whole slice groups go to XCDs where their
+// number divides; a single group, or a number that does not, takes its
+// heaviest tiles first over the whole chip instead: ranges of tiles per XCD
+// leave the XCDs of the image's corners idle early, and a row-major or
+// Morton order ends on full tiles.  32 slices of 512^2 x 1000 on the matrix
+// cores, two launches in flight: 450 us, 472 with ranges (256 frames 4.14 ms,
+// 4.35); one slice of 384^2 x 360 17.6 / 23.2 us, of 640^2 x 720 55 / 63; three
+// groups of 2 slices of 512^2 x 1000 199 us, 204 in tile order.
+static void set_dispatch(risa_bp_t h, BpParams& p, long off, dim3 grid)
+{
+    p.order = off >= 0 ? h->tile_order.ptr + off : nullptr;
+    p.xg = xcd_groups(grid.x, grid.y);
+    if (p.order && (grid.y == 1 || !p.xg)) p.xg = 2;
+}
+
 // Slice k of the call is sino(k) -> img(k); launches of up to kBpSlices
 // slices (a multiple of every variant's slices per workgroup).
 template <class SinoAt, class ImgAt>
@@ -2594,8 +2611,7 @@ static void launch_linear_at(risa_bp_t h, int variant, SinoAt sino, ImgAt img, i
             if (!L.sino[k] || !L.img[k]) fail(RISA_ERR_ARG, "null slice pointer");
         }
         dim3 grid(p.tilesX * ceil_div(p.N, v.ty), ceil_div(n, v.sb));
-        p.xg = xcd_groups(grid.x, grid.y);
-        p.order = p.xg && h->order_off[(size_t)variant] >= 0 ? h->tile_order.ptr + h->order_off[(size_t)variant] : nullptr;
+        set_dispatch(h, p, h->order_off[(size_t)variant], grid);
         hipLaunchKernelGGL(v.fn, grid, dim3(v.q * v.threads()), lds, s, L, h->cosT.ptr, h->sinT.ptr, n, p);
         check_launch("bp_linear_kernel");
     }
@@ -2668,9 +2684,7 @@ static void launch_f16x4(risa_bp_t h, int variant, const uint2* sino, float in_s
                                 sizeof(float) * (v.q - 1) * v.ppt * kF16Group * v.g * threads);
     if (lds > (v.q > 1 ? kMaxLds / 64 * 80 : kMaxLds)) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %zu B of LDS", lds);
     dim3 grid(p.tilesX * ceil_div(p.N, v.ty), ceil_div(ceil_div(slices, kF16Group), v.g));
-    p.xg = xcd_groups(grid.x, grid.y);
-    const long off = h->order_off[(size_t)(kNumVariants + variant)];
-    p.order = p.xg && off >= 0 ? h->tile_order.ptr + off : nullptr;
+    set_dispatch(h, p, h->order_off[(size_t)(kNumVariants + variant)], grid);
     hipLaunchKernelGGL(v.fn, grid, dim3(v.q * threads), lds, s, sino, img, h->cosT.ptr, h->sinT.ptr, slices, p);
     check_launch("bp_linear_f16_kernel");
 }
@@ -2751,13 +2765,7 @@ extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, floa
         const int lds = split_lds(p.AE, p.W);
         if (lds > kMaxSplitLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %d B of LDS", lds);
         dim3 grid(p.tilesX * ceil_div(p.N, v.ty), 1);
-        const long off = h->order_off[(size_t)v.variant];
-        // heaviest tiles first over the whole chip: ranges of tiles per XCD
-        // leave the XCDs of the image's corners idle early (32 slices of
-        // 512^2 x 1000, two launches in flight: 450 us, 472 with ranges; 256
-        // frames 4.14 ms, 4.35)
-        p.order = off >= 0 ? h->tile_order.ptr + off : nullptr;
-        p.xg = p.order ? 2 : 0;
+        set_dispatch(h, p, h->order_off[(size_t)v.variant], grid);
         unsigned* pk = reinterpret_cast<unsigned*>(packed);
         hipLaunchKernelGGL(split_pack_kernel, dim3(ceil_div(split_rows(p.D) - 2, 32), p.P), dim3(256), 0, s, sino,
                            slices, p.P, p.D, scale, pk);
