@@ -523,10 +523,9 @@ struct BpSlices {
     float* img[kBpSlices];
 };
 
-template <int TX, int TY, int PPT, int E, int U, int SB, int Q = 1>
-__global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_kernel(BpSlices L, const float* __restrict__ cosT,
-                                                                 const float* __restrict__ sinT, int slices,
-                                                                 BpParams p)
+template <int TX, int TY, int PPT, int E, int U, int SB, int Q>
+__device__ __forceinline__ void bp_slices(const BpSlices& L, const float* __restrict__ cosT,
+                                          const float* __restrict__ sinT, int slices, const BpParams& p)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     int2 txy;
@@ -545,6 +544,23 @@ __global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_kernel(BpSlices L, 
         }
         bp_tile<TX, TY, PPT, E, U, SB, Q>(sp[0], ip[0], cosT, sinT, p, x0, y0, 0, smem, sp, ip, nv);
     }
+}
+
+template <int TX, int TY, int PPT, int E, int U, int SB>
+__global__ void __launch_bounds__(TX* TY / PPT) bp_linear_kernel(BpSlices L, const float* __restrict__ cosT,
+                                                                 const float* __restrict__ sinT, int slices,
+                                                                 BpParams p)
+{
+    bp_slices<TX, TY, PPT, E, U, SB, 1>(L, cosT, sinT, slices, p);
+}
+
+// The angles shared by Q groups of threads.
+template <int TX, int TY, int PPT, int E, int U, int SB, int Q>
+__global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_groups_kernel(BpSlices L, const float* __restrict__ cosT,
+                                                                           const float* __restrict__ sinT, int slices,
+                                                                           BpParams p)
+{
+    bp_slices<TX, TY, PPT, E, U, SB, Q>(L, cosT, sinT, slices, p);
 }
 
 // A job of the persistent uneven batch (device copy of risa_bp_job + derived
@@ -638,12 +654,10 @@ __host__ __device__ constexpr size_t f16_lds(int G, int E, int threads, int AE)
 
 // G groups of 4 slices per workgroup: the per-pixel t, index and weight are
 // shared by 4G slices.  Q groups of threads share the angles as in bp_tile.
-template <int TX, int TY, int PPT, int E, int U, int G, int Q = 1>
-__global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_kernel(const uint2* __restrict__ sino,
-                                                                     float* __restrict__ img,
-                                                                     const float* __restrict__ cosT,
-                                                                     const float* __restrict__ sinT, int slices,
-                                                                     BpParams p)
+template <int TX, int TY, int PPT, int E, int U, int G, int Q>
+__device__ __forceinline__ void bp_f16_tile(const uint2* __restrict__ sino, float* __restrict__ img,
+                                            const float* __restrict__ cosT, const float* __restrict__ sinT, int slices,
+                                            const BpParams& p)
 {
     constexpr int NT = TX * TY / PPT;
     constexpr int RS = TY / PPT;
@@ -874,6 +888,27 @@ __global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_kernel(const ui
                 img[(long)(b0 + b) * p.N * p.N + (long)y * p.N + x] =
                     use[r] ? acc[r][b] * p.norm * p.out_scale : p.maskingValue;
         }
+}
+
+template <int TX, int TY, int PPT, int E, int U, int G>
+__global__ void __launch_bounds__(TX* TY / PPT) bp_linear_f16_kernel(const uint2* __restrict__ sino,
+                                                                     float* __restrict__ img,
+                                                                     const float* __restrict__ cosT,
+                                                                     const float* __restrict__ sinT, int slices,
+                                                                     BpParams p)
+{
+    bp_f16_tile<TX, TY, PPT, E, U, G, 1>(sino, img, cosT, sinT, slices, p);
+}
+
+// The angles shared by Q groups of threads.
+template <int TX, int TY, int PPT, int E, int U, int G, int Q>
+__global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_groups_kernel(const uint2* __restrict__ sino,
+                                                                               float* __restrict__ img,
+                                                                               const float* __restrict__ cosT,
+                                                                               const float* __restrict__ sinT,
+                                                                               int slices, BpParams p)
+{
+    bp_f16_tile<TX, TY, PPT, E, U, G, Q>(sino, img, cosT, sinT, slices, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -2219,7 +2254,7 @@ struct BpVariant {
 
 #define RISA_BPV(TX, TY, PPT, E, U, SB, AMAX) {TX, TY, PPT, E, U, SB, AMAX, bp_linear_kernel<TX, TY, PPT, E, U, SB>}
 #define RISA_BPQ(TX, TY, PPT, E, U, SB, AMAX, Q) \
-    {TX, TY, PPT, E, U, SB, AMAX, bp_linear_kernel<TX, TY, PPT, E, U, SB, Q>, Q}
+    {TX, TY, PPT, E, U, SB, AMAX, bp_linear_groups_kernel<TX, TY, PPT, E, U, SB, Q>, Q}
 static const BpVariant kVariants[] = {
     RISA_BPV(32, 32, 4, 8, 4, 1, 64), RISA_BPV(32, 16, 2, 8, 4, 1, 64), RISA_BPV(16, 16, 1, 4, 4, 1, 64),
     RISA_BPV(32, 32, 8, 16, 2, 1, 64), RISA_BPV(64, 16, 4, 16, 4, 1, 64), RISA_BPV(32, 16, 4, 16, 4, 1, 64),
@@ -2239,8 +2274,8 @@ static const BpVariant kVariants[] = {
     // 14.3 us; 512^2 x 1000 one slice 80 -> 53, four 145 -> 133; 384^2 x 360
     // six slices 67 -> 60.  Full launches stay with the variants above
     // (512^2 x 720, 16 slices: 314 us, 321 at best with groups).
-    RISA_BPQ(16, 16, 2, 4, 4, 1, 64, 4), RISA_BPQ(16, 16, 2, 4, 4, 1, 64, 8), RISA_BPQ(32, 32, 4, 4, 2, 1, 64, 4),
-    RISA_BPQ(16, 16, 2, 4, 4, 2, 64, 4), RISA_BPQ(16, 16, 1, 2, 4, 2, 64, 2), RISA_BPQ(32, 32, 4, 4, 2, 2, 64, 2),
+    RISA_BPQ(16, 16, 2, 4, 4, 1, 32, 4), RISA_BPQ(16, 16, 2, 4, 4, 1, 16, 8), RISA_BPQ(32, 32, 4, 4, 2, 1, 32, 4),
+    RISA_BPQ(16, 16, 2, 4, 4, 2, 32, 4), RISA_BPQ(16, 16, 1, 2, 4, 2, 32, 2), RISA_BPQ(32, 32, 4, 4, 2, 2, 32, 2),
 };
 #undef RISA_BPV
 #undef RISA_BPQ
@@ -2254,7 +2289,7 @@ struct BpF16Variant {
 #define RISA_BPH(TX, TY, PPT, E, U, G, AMAX) \
     {TX, TY, PPT, E, U, G, AMAX, bp_linear_f16_kernel<TX, TY, PPT, E, U, G>}
 #define RISA_BPG(TX, TY, PPT, E, U, G, AMAX, Q) \
-    {TX, TY, PPT, E, U, G, AMAX, bp_linear_f16_kernel<TX, TY, PPT, E, U, G, Q>, Q}
+    {TX, TY, PPT, E, U, G, AMAX, bp_linear_f16_groups_kernel<TX, TY, PPT, E, U, G, Q>, Q}
 // 16-pixel-wide tiles: the 16-byte LDS entries of a half-wave row then
 // stay clear of bank conflicts; G groups of 4 slices share each pixel's
 // weight.  The LDS planes take G * 2 * E * threads * 16 B, at most 32 KB
@@ -2268,8 +2303,8 @@ static const BpF16Variant kF16Variants[] = {
     // few waves (as in the FP32 table): 512^2 x 1000 angles, 4 slices 148 ->
     // 102 us, 8 slices 178 -> 162; 256^2 x 500, 4 slices 59 -> 26, 16 slices
     // 67 -> 49.  From 16 slices of 512^2 the variants above are at least as fast.
-    RISA_BPG(16, 32, 2, 2, 2, 1, 64, 4), RISA_BPG(16, 16, 1, 1, 4, 1, 64, 4), RISA_BPG(16, 16, 1, 2, 4, 2, 64, 2),
-    RISA_BPG(16, 32, 2, 2, 2, 2, 64, 2), RISA_BPG(16, 16, 1, 1, 2, 2, 64, 4),
+    RISA_BPG(16, 32, 2, 2, 2, 1, 32, 4), RISA_BPG(16, 16, 1, 1, 4, 1, 32, 4), RISA_BPG(16, 16, 1, 2, 4, 2, 32, 2),
+    RISA_BPG(16, 32, 2, 2, 2, 2, 32, 2), RISA_BPG(16, 16, 1, 1, 2, 2, 32, 4),
 };
 #undef RISA_BPH
 #undef RISA_BPG
@@ -3062,6 +3097,13 @@ extern "C" int risa_hip_bp_variant_shape(int f16, int variant, int shape[7])
             std::copy(s, s + 7, shape);
         }
     });
+}
+
+// Groups of threads that share a variant's angles (0 past the last variant).
+extern "C" int risa_bp_variant_groups(int f16, int variant)
+{
+    if (variant < 0 || variant >= (f16 ? kNumF16Variants : kNumVariants)) return 0;
+    return f16 ? kF16Variants[variant].q : kVariants[variant].q;
 }
 
 extern "C" int risa_hip_bp_get_variant(risa_bp_t h, int* variant)

@@ -236,9 +236,11 @@ def bp_variant_shape(f16: bool, variant: int) -> tuple:
 def bp_kernel_name(f16: bool, variant: int) -> str:
     """The backprojection kernel a variant launches, as profilers name it."""
     tx, ty, ppt, e, u, g, _ = bp_variant_shape(f16, variant)
-    if f16:
-        return f"risa::bp_linear_f16_kernel<{tx}, {ty}, {ppt}, {e}, {u}, {g}>"
-    return f"risa::bp_linear_kernel<{tx}, {ty}, {ppt}, {e}, {u}, {g}>"
+    q = load().risa_bp_variant_groups(1 if f16 else 0, variant)
+    base = "risa::bp_linear_f16" if f16 else "risa::bp_linear"
+    if q > 1:   # groups of threads share the angles
+        return f"{base}_groups_kernel<{tx}, {ty}, {ppt}, {e}, {u}, {g}, {q}>"
+    return f"{base}_kernel<{tx}, {ty}, {ppt}, {e}, {u}, {g}>"
 
 
 class Backprojection(_Handle):
