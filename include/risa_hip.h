@@ -404,9 +404,10 @@ int risa_hip_bp_batched_destroy(risa_bp_batched_t h);
 /* ------------------------------------------------------------------ Chain -- */
 /* The whole per-frame chain on one device with its own scratch buffers.
  * mode 0 = plain FP32 (FFT filter, FP32 backprojection), groups of up to 16
- * frames; mode 1 = mixed precision (DFT-GEMM filter with FP16 output,
- * FP16-sinogram / FP32-accumulate backprojection), groups of up to 32
- * frames.  A run's groups are dealt to two streams forked from and joined
+ * frames, or 32 where max_frames >= 64; mode 1 = mixed precision (DFT-GEMM
+ * filter with FP16 output, FP16-sinogram / FP32-accumulate backprojection),
+ * groups of up to 32 frames, or 64 where max_frames >= 128 and timing at
+ * creation finds them faster.  A run's groups are dealt to two streams forked from and joined
  * into the caller's stream.  max_frames bounds one run call. */
 enum risa_chain_mode { RISA_CHAIN_PLAIN = 0, RISA_CHAIN_MIXED = 1 };
 
