@@ -3119,9 +3119,16 @@ extern "C" int risa_hip_bp_get_variant(risa_bp_t h, int* variant)
 // in flight), FP16 variants at s16 slices per launch; 0 skips a precision.
 // max_sb: the FP32 variants considered take at most this many slices per
 // workgroup (1 for callers that launch one slice at a time).
-static void autotune(risa_bp_t h, int s32, int s16, hipStream_t s, int max_sb = 1)
+//
+// The FP16 tile shape is picked among the variants whose angles are not shared,
+// or kept (keep_tile), and the variant among those of that shape: a weight's
+// FP16 rounding depends on t's distance from the tile's origin, so results move
+// by up to 2e-5 (noise) from one shape to another, and by the order of the sums,
+// 1e-6, within one.
+static void autotune(risa_bp_t h, int s32, int s16, hipStream_t s, int max_sb = 1, bool keep_tile = false)
 {
     DeviceGuard dg(h->device);
+    const BpF16Variant kept = kF16Variants[h->variant_f16];
     const int N = h->g.numberOfPixels, P = h->g.numberOfParallelProjections, D = h->g.numberOfParallelDetectors;
     DeviceBuffer<float> sino((size_t)P * D * std::max(1, s32));
     DeviceBuffer<uint2> sino16((size_t)P * D * std::max(1, ceil_div(s16, kF16Group)));
@@ -3155,6 +3162,7 @@ static void autotune(risa_bp_t h, int s32, int s16, hipStream_t s, int max_sb = 
                 }
             }
             for (int v = 0; s16 > 0 && v < kNumF16Variants; v++) {
+                if (keep_tile && (kF16Variants[v].tx != kept.tx || kF16Variants[v].ty != kept.ty)) continue;
                 try {
                     t16[v] = std::min(t16[v],
                                       time_it([&] { launch_f16x4(h, v, sino16.ptr, 1.0f, s16, img.ptr, s); }));
@@ -3164,7 +3172,17 @@ static void autotune(risa_bp_t h, int s32, int s16, hipStream_t s, int max_sb = 
             }
         }
         const auto b32 = std::min_element(t32.begin(), t32.end());
-        const auto b16 = std::min_element(t16.begin(), t16.end());
+        auto b16 = std::min_element(t16.begin(), t16.end());
+        if (!keep_tile) {
+            int base = 0;
+            for (int v = 0; v < kNumF16Variants; v++)
+                if (kF16Variants[v].q == 1 && t16[v] < t16[base]) base = v;
+            b16 = t16.begin() + base;
+            for (int v = 0; v < kNumF16Variants; v++)
+                if (kF16Variants[v].tx == kF16Variants[base].tx && kF16Variants[v].ty == kF16Variants[base].ty &&
+                    t16[v] < *b16)
+                    b16 = t16.begin() + v;
+        }
         if (s32 > 0 && *b32 < 1e30f) h->variant = (int)(b32 - t32.begin());
         if (s16 > 0 && *b16 < 1e30f) h->variant_f16 = (int)(b16 - t16.begin());
     } catch (...) {
@@ -3197,6 +3215,15 @@ extern "C" int risa_hip_bp_slices_per_tile(risa_bp_t h, int* slices)
     return guarded("risa_hip_bp_slices_per_tile", [&] {
         if (!h || !slices) fail(RISA_ERR_ARG, "null argument");
         *slices = kVariants[h->variant].sb;
+    });
+}
+
+// The fastest FP16 variant of the current one's tile shape at `slices`.
+extern "C" int risa_bp_autotune_f16_tile(risa_bp_t h, int slices)
+{
+    return guarded("risa_bp_autotune_f16_tile", [&] {
+        if (!h || slices < 1) fail(RISA_ERR_ARG, "bad argument");
+        autotune(h, 0, slices, nullptr, 1, true);
     });
 }
 

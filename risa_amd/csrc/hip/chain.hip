@@ -37,6 +37,7 @@ int risa_filter_run_oop(risa_filter_t h, const float* in, float* out, long rows,
 double risa_filter_l1(risa_filter_t h);
 int risa_fan2para_gain(risa_fan2para_t h, double* gain);
 extern "C" size_t risa_bp_split_bytes(risa_bp_t h);
+extern "C" int risa_bp_autotune_f16_tile(risa_bp_t h, int slices);
 extern "C" size_t risa_bp_f16_pack_bytes(risa_bp_t h);
 extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int* min_slices);
 extern "C" int risa_bp_run_f16_packed(risa_bp_t h, const uint16_t* sino_x4, float in_scale, int slices, void* packed,
@@ -200,7 +201,11 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
                 // group 245 us, two of 4 in two lanes 292; 48 frames as 32 + 16
                 // 978, as 24 + 24 1160)
                 h->per = std::min(kMixedMaxPer, (max_frames + 3) / 4 * 4);
-                ok(risa_hip_bp_autotune_f16(h->bp, h->per, nullptr));
+                // the tile shape (and with it the results) as timed for half of the
+                // frames per lane, the variant for the group
+                const int half = (max_frames + kMixedLanes - 1) / kMixedLanes;
+                ok(risa_hip_bp_autotune_f16(h->bp, std::min(kMixedMaxPer, (half + 3) / 4 * 4), nullptr));
+                ok(risa_bp_autotune_f16_tile(h->bp, h->per));
                 if (max_frames >= kMixedLanes * kPackPer && (h->split_bytes = risa_bp_f16_pack_bytes(h->bp)) > 0) {
                     ok(risa_bp_tune_f16_packed(h->bp, nullptr, &h->split_min));
                     if (h->split_min <= kPackPer) {
