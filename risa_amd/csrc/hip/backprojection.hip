@@ -939,11 +939,13 @@ __global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_groups_kernel(c
 // adjacent detectors, row R (detectors 2R, 2R + 1) being 32 dwords of hi
 // pairs, one per slice, then 32 of lo pairs, with a zero row at either end.
 // A chunk's rows go from global memory straight to LDS (16 bytes per lane, no
-// registers or vector instructions); two row buffers, one barrier per chunk.  Odd angles' rows are
-// shifted by 64 bytes, so that the two angles whose lanes are read together
-// use different banks.  A block's 4 rows may run past its angle's rows: their
-// weights are zero and what they hold is finite (the next angle's rows, or
-// the zeroed end of the buffer).
+// registers or vector instructions); two row buffers, one barrier per chunk.
+// An angle's rows are followed by 64 spare bytes, so that the two angles whose
+// lanes are read together use different banks; every byte of a buffer belongs
+// to one angle, since different waves copy them.  A block's 4 rows may run past
+// its angle's rows: their weights are zero and what they hold is finite (the
+// next angle's rows, or the zeroed bytes between angles and at the end of the
+// buffer).
 //
 // Bound: LDS reads.  A block's operands take 5 KB per 64 (pixel, angle) pairs
 // (4 KB of samples, 1 KB of selectors) at the ~105 bytes per clock and CU that
@@ -966,10 +968,9 @@ __host__ __device__ constexpr int split_rows(int D) { return (D + 1) / 2 + 2; }
 // Staged rows of one angle, a multiple of the 4 a wave copies at once: W + 1
 // samples from up to three before the window.
 __host__ __device__ constexpr int split_staged(int W) { return ((W + 5) / 2 + 3) / 4 * 4; }
-__host__ __device__ constexpr int split_buffer(int AE, int W)
-{
-    return (AE * split_staged(W) + kSplitSlack) * kSplitRow + 64;
-}
+// Bytes from one staged angle to the next.
+__host__ __device__ constexpr int split_pitch(int W) { return split_staged(W) * kSplitRow + 64; }
+__host__ __device__ constexpr int split_buffer(int AE, int W) { return AE * split_pitch(W) + kSplitSlack * kSplitRow; }
 // Selector tables (2 x 8 x 16 B), two row buffers, the angle records (16 + 16 B).
 __host__ __device__ constexpr int split_lds(int AE, int W) { return 256 + 2 * split_buffer(AE, W) + kSplitInfo * 32; }
 
@@ -1064,7 +1065,8 @@ __global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* _
 {
     constexpr int NT = TX * TY, NW = NT / 64;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int AE = p.AE, RW = split_staged(p.W), bufsz = split_buffer(AE, p.W), RP = split_rows(p.D);
+    const int AE = p.AE, RW = split_staged(p.W), pitch = split_pitch(p.W), bufsz = split_buffer(AE, p.W);
+    const int RP = split_rows(p.D);
     uint4* tab = reinterpret_cast<uint4*>(smem);
     char* rows = smem + 256;
     float4* info = reinterpret_cast<float4*>(rows + 2 * bufsz);   // (cos, sin, -T, LDS address of sample k = 0)
@@ -1112,8 +1114,7 @@ __global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* _
         // the origin is moved down to an even detector
         const int odd = ((int)-w.negT + p.cI) & 1, first = (w.kmin + odd - 2) & ~1;
         info[r] = make_float4(w.c, w.s, w.negT + (float)odd,
-                              __uint_as_float(rbase + (unsigned)((ch & 1) * bufsz + a * RW * kSplitRow + (a & 1) * 64 -
-                                                                 first * (kSplitRow / 2))));
+                              __uint_as_float(rbase + (unsigned)((ch & 1) * bufsz + a * pitch - first * (kSplitRow / 2))));
         info2[r] = make_float4(3.0f * p.scale * (fminf(w.c, 0.0f) + fminf(w.s, 0.0f)) - 0.01f,
                                __uint_as_float(tbase + (pa < p.P ? 0u : 128u)),
                                __int_as_float((first + (int)-w.negT - odd + p.cI) / 2 + 1), 0.0f);
@@ -1128,7 +1129,7 @@ __global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* _
             const int R = __float_as_int(info2[(p0 + a) % kSplitInfo].z) + r + lane / 16;
             const unsigned* src = packed + ((long)(p0 + a) * RP + clamp_index(R, RP - 1)) * 64 + (lane & 15) * 4;
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                             buf + (a * RW + r) * kSplitRow + (a & 1) * 64, 16, 0, 0);
+                                             buf + a * pitch + r * kSplitRow, 16, 0, 0);
         }
     };
     if (nch) {
@@ -2773,6 +2774,28 @@ static const SplitShape kSplitShapes[] = {
 constexpr int kNumSplitShapes = sizeof(kSplitShapes) / sizeof(kSplitShapes[0]);
 constexpr int kMaxSplitLds = 160 * 1024;   // a gfx950 workgroup's LDS
 
+// Angles of a shape's chunk: the shape's most, or half as often as its LDS asks.
+static int split_angles(int shape, int W)
+{
+    int ae = kSplitShapes[shape].amax;
+    while (ae > 4 && split_lds(ae, W) > kMaxSplitLds) ae /= 2;
+    return ae;
+}
+
+// What a workgroup of `shape` stages at a detector scale, for checks on the
+// host: window samples W, angles per chunk, rows copied per angle, bytes of a
+// row, bytes between angles, bytes of a buffer, LDS bytes.
+extern "C" int risa_bp_split_layout(int shape, float scale, int layout[7])
+{
+    return guarded("risa_bp_split_layout", [&] {
+        if (shape < 0 || shape >= kNumSplitShapes || !(scale > 0.0f) || scale > kSplitMaxScale || !layout)
+            fail(RISA_ERR_ARG, "bad argument");
+        const int W = window_entries(kSplitShapes[shape].tx, kSplitShapes[shape].ty, scale), ae = split_angles(shape, W);
+        const int v[7] = {W, ae, split_staged(W), kSplitRow, split_pitch(W), split_buffer(ae, W), split_lds(ae, W)};
+        std::copy(v, v + 7, layout);
+    });
+}
+
 // Bytes of the packed sinograms of one launch (32 slices); 0 where the
 // geometry is outside what the kernel takes.
 extern "C" size_t risa_bp_split_bytes(risa_bp_t h)
@@ -2795,8 +2818,7 @@ extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, floa
         const SplitShape& v = kSplitShapes[shape];
         BpParams p = make_params(h, v.tx, v.ty);
         p.out_scale = 1.0f / scale;
-        p.AE = v.amax;
-        while (p.AE > 4 && split_lds(p.AE, p.W) > kMaxSplitLds) p.AE /= 2;
+        p.AE = split_angles(shape, p.W);
         const int lds = split_lds(p.AE, p.W);
         if (lds > kMaxSplitLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tile needs %d B of LDS", lds);
         dim3 grid(p.tilesX * ceil_div(p.N, v.ty), 1);
