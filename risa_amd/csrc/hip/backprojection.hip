@@ -2251,6 +2251,8 @@ struct BpVariant {
     void (*fn)(BpSlices, const float*, const float*, int, BpParams);
     int q = 1;                         // groups of threads that share the angles
     int threads() const { return tx * ty / ppt; }   // of one group
+    // a chunk holds at least one angle's window
+    bool stages(int W) const { return W <= e * threads(); }
 };
 
 #define RISA_BPV(TX, TY, PPT, E, U, SB, AMAX) {TX, TY, PPT, E, U, SB, AMAX, bp_linear_kernel<TX, TY, PPT, E, U, SB>}
@@ -2580,6 +2582,12 @@ extern "C" int risa_hip_bp_create(const risa_geom* g, int device, risa_bp_t* out
             h->sinT.resize(h->lut.sinT.size());
             h->sinT.upload(h->lut.sinT);
             h->fuse_mask = g->fusedMasking && !g->normalization;
+            // until a variant is set or timed: the first one whose staging holds
+            // a window (variant 0 up to 46 detectors per pixel, some up to 63)
+            for (int v = kNumVariants - 1; v >= 0; v--) {
+                const int W = window_entries(kVariants[v].tx, kVariants[v].ty, h->lut.scale);
+                if (kVariants[v].stages(W) && tile_lds(1, W, kVariants[v].sb) * kVariants[v].q <= kMaxLds) h->variant = v;
+            }
             // run-call scratch, sized here so run calls allocate nothing
             const size_t plane = (size_t)g->numberOfParallelProjections * g->numberOfParallelDetectors;
             h->x4.resize((size_t)kF16StageGroups * plane);
@@ -2629,6 +2637,7 @@ static void launch_linear_at(risa_bp_t h, int variant, SinoAt sino, ImgAt img, i
 {
     const BpVariant& v = kVariants[variant];
     BpParams p = make_params(h, v.tx, v.ty);
+    if (!v.stages(p.W)) fail(RISA_ERR_UNSUPPORTED, "backprojection window exceeds the tile's staging");
     p.AE = chunk_angles(v.threads(), v.e, v.amax, p.W, v.sb, v.q);
     if (v.q > 1) {   // a group's chunks of about the same length
         const int len = ceil_div(p.P, v.q);
