@@ -3365,7 +3365,8 @@ struct risa_bp_batched_s {
     size_t lds = 0;
 };
 
-// Job table and cost-sorted tile list for the current variant.
+// Job table and cost-sorted tile list for the current variant; refuses, before
+// it changes the layout, jobs whose windows the variant cannot stage.
 static void batched_layout(risa_bp_batched_s* h)
 {
     const PersistentVariant& v = kPersistent[h->variant];
@@ -3385,6 +3386,7 @@ static void batched_layout(risa_bp_batched_s* h)
         p.mask = j.mask ? 1 : 0;
         p.maskingValue = j.maskingValue;
         p.W = window_entries(v.tx, v.ty, p.scale);
+        if (p.W > v.e * threads) fail(RISA_ERR_UNSUPPORTED, "job %zu: backprojection window exceeds the tile's staging", i);
         p.tilesX = ceil_div(j.N, v.tx);
         p.zx = p.zy = -1;   // the persistent kernel takes tiles from its cost-sorted list
         const int tilesY = ceil_div(j.N, v.ty);
@@ -3413,9 +3415,9 @@ static void batched_layout(risa_bp_batched_s* h)
     std::stable_sort(order.begin(), order.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
     std::vector<int2> tl(order.size());
     for (size_t i = 0; i < order.size(); i++) tl[i] = order[i].second;
+    if (lds > kMaxLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tiles need %zu B of LDS", lds);
     h->ntiles = (int)tl.size();
     h->lds = lds;
-    if (h->lds > kMaxLds) fail(RISA_ERR_UNSUPPORTED, "backprojection tiles need %zu B of LDS", lds);
     h->djobs.resize(dj.size());
     h->djobs.upload(dj);
     h->tiles.resize(tl.size());
@@ -3457,7 +3459,15 @@ extern "C" int risa_hip_bp_batched_create(const risa_bp_job* jobs, int njobs, in
             h->sinT.resize(sn.size());
             h->sinT.upload(sn);
             h->counter.resize(1);
-            batched_layout(h);
+            // the first tile shape that holds every job's windows
+            for (;; h->variant++) {
+                try {
+                    batched_layout(h);
+                    break;
+                } catch (const Error& e) {
+                    if (e.code != RISA_ERR_UNSUPPORTED || h->variant + 1 >= kNumPersistent) throw;
+                }
+            }
         } catch (...) {
             delete h;
             throw;
@@ -3505,8 +3515,14 @@ extern "C" int risa_hip_bp_batched_set_variant(risa_bp_batched_t h, int variant)
     return guarded("risa_hip_bp_batched_set_variant", [&] {
         if (!h || variant < 0 || variant >= kNumPersistent) fail(RISA_ERR_ARG, "variant out of range");
         DeviceGuard dg(h->device);
+        const int before = h->variant;
         h->variant = variant;
-        batched_layout(h);
+        try {
+            batched_layout(h);
+        } catch (...) {
+            h->variant = before;   // the layout is still that variant's
+            throw;
+        }
     });
 }
 

@@ -82,3 +82,45 @@ def test_beyond_every_variant_is_refused(risa, geom_c0, cuda):
     with pytest.raises(risa.RisaError):
         bp(x, torch.empty((8, 8), dtype=torch.float32, device=cuda))
     bp.close()
+
+
+def test_uneven_batch_is_right_or_refused(risa, cuda):
+    """50 detectors per pixel (and 1): two of the persistent tile shapes stage
+    such a window, a refused one leaves the batch as it was."""
+    import torch
+    from risa_amd import device
+
+    rng = np.random.default_rng(5)
+    jobs, want, imgs = [], [], []
+    for N, P, D in ((16, 60, 800), (40, 50, 40)):
+        x = rng.standard_normal((1, P, D)).astype(np.float32)
+        imgs.append(torch.full((N, N), float("nan"), dtype=torch.float32, device=cuda))
+        jobs.append(dict(sino=torch.from_numpy(x[0]).to(cuda), img=imgs[-1], N=N, P=P, D=D, mask=0))
+        want.append(exact(x, N)[0])
+    batch = device.BatchedBackprojection(jobs)
+
+    def check(what):
+        for i in imgs:
+            i.fill_(float("nan"))
+        batch()
+        for i, w in zip(imgs, want):
+            err = np.linalg.norm(i.cpu().numpy() - w) / np.linalg.norm(w)
+            print(f"case: uneven batch {what}: N={w.shape[0]} rel error {err:.1e}", flush=True)
+            assert err < 4e-4   # 2^-23 * 44 * 50 * 1.4
+
+    check("as created")
+    refused = 0
+    for v in range(4):
+        try:
+            batch.set_variant(v)
+        except risa.RisaError:
+            refused += 1
+        check(f"variant {v} asked for")
+    assert refused == 2
+    batch.autotune()
+    check("tuned")
+    batch.close()
+    with pytest.raises(risa.RisaError):
+        N, P, D = 8, 9, 520
+        device.BatchedBackprojection([dict(sino=torch.zeros((P, D), device=cuda), img=torch.zeros((N, N), device=cuda),
+                                           N=N, P=P, D=D)])
