@@ -424,11 +424,16 @@ int risa_hip_chain_run(risa_chain_t h, const uint16_t* raw, const int32_t* plane
  * below the chain's frames in flight (later groups reuse the slots). */
 int risa_hip_chain_intermediate(risa_chain_t h, int which, const void** ptr);
 /* Backprojector variant of the chain (as risa_hip_bp_set_variant; replaces
- * the autotuner's pick).  A change synchronises the chain's device and
+ * the autotuner's pick).  A plain chain whose variant was set, to the one it
+ * reports too, backprojects every group of frames with that variant and none
+ * on the matrix cores.  A change synchronises the chain's device and
  * releases the captured graphs; the next graph run captures anew.  No
  * reference counterpart. */
 int risa_hip_chain_set_variant(risa_chain_t h, int variant);
 int risa_hip_chain_get_variant(risa_chain_t h, int* variant);
+/* From how many frames on a group is backprojected on the matrix cores
+ * (0: none is).  Tooling; no reference counterpart. */
+int risa_hip_chain_matrix_frames(risa_chain_t h, int* frames);
 /* Layout of the raw frames risa_hip_chain_run reads (risa_input_layout;
  * MODULE_MAJOR = the reference's H2D -> Reordering -> Attenuation, with the
  * reordering fused into the attenuation load).  A change synchronises the

@@ -78,9 +78,10 @@ struct risa_chain_s {
     risa_bp_t bp = nullptr;
     risa::DeviceBuffer<float> att_buf, par_buf, filt_buf;   // `per` frame slots per lane
     risa::DeviceBuffer<uint16_t> f16_buf;                   // MIXED: `per` slots per lane, x4 layout
-    // PLAIN, per = kSplitPer: groups of at least split_min frames go through
-    // the FP32 backprojector on the matrix cores (tile shape split_shape, -1:
-    // off), whose FP16 hi + lo operands hold filtered sample * split_scale
+    // Groups of at least split_min frames are backprojected on the matrix cores
+    // (split_shape -1: none).  PLAIN: tile shape split_shape, FP16 hi + lo
+    // operands that hold filtered sample * split_scale, until the caller sets a
+    // variant; MIXED: while the FP16 variant is one whose bits that kernel has
     int split_shape = -1, split_min = 0;
     float split_scale = 0.0f;
     risa::DeviceBuffer<char> split_buf;                     // packed sinograms, one launch per lane
@@ -102,6 +103,7 @@ struct risa_chain_s {
         (void)hipDeviceSynchronize();
         if (prev != device) (void)hipSetDevice(prev);
     }
+    bool on_matrix_cores(int n) const;
     void release_graphs()
     {
         for (auto& kv : graphs) (void)hipGraphExecDestroy(kv.second.exec);
@@ -121,6 +123,11 @@ struct risa_chain_s {
 };
 
 using namespace risa;
+
+bool risa_chain_s::on_matrix_cores(int n) const
+{
+    return split_shape >= 0 && n >= split_min && (mode == RISA_CHAIN_PLAIN || risa_bp_f16_pack_bytes(bp) > 0);
+}
 
 static void ok(int rc)
 {
@@ -278,7 +285,7 @@ static void enqueue(risa_chain_t h, const uint16_t* raw, const int32_t* planes, 
                 ok(risa_hip_attenuation_run_batch(h->att, raw + f * fan, planes + f, n, att, ls));
                 ok(risa_hip_fan2para_run_batch(h->f2p, att, planes + f, n, pb, ls));
                 ok(risa_filter_run_oop(h->filt, pb, fb, (long)n * g.numberOfParallelProjections, ls));
-                if (h->split_shape >= 0 && n >= h->split_min)
+                if (h->on_matrix_cores(n))
                     ok(risa_bp_run_split(h->bp, h->split_shape, fb, h->split_scale, n, h->split_buf.ptr + k * h->split_bytes,
                                          img + f * out, ls));
                 else
@@ -289,7 +296,7 @@ static void enqueue(risa_chain_t h, const uint16_t* raw, const int32_t* planes, 
             ok(risa_hip_attenuation_run_batch(h->att, raw + f * fan, planes + f, n, att, ls));
             ok(risa_hip_fan2para_run_batch(h->f2p, att, planes + f, n, pb, ls));
             ok(risa_hip_filter_run_f16x4(h->filt, pb, hb, n, kF16SinoScale, ls));
-            if (h->split_shape >= 0 && n >= h->split_min)
+            if (h->on_matrix_cores(n))
                 ok(risa_bp_run_f16_packed(h->bp, hb, kF16SinoScale, n, h->split_buf.ptr + k * h->split_bytes,
                                           img + f * out, ls));
             else
@@ -387,11 +394,22 @@ extern "C" int risa_hip_chain_set_variant(risa_chain_t h, int variant)
         if (!h) fail(RISA_ERR_ARG, "null handle");
         int cur = 0;
         ok(risa_hip_bp_get_variant(h->bp, &cur));
-        if (cur == variant) return;
+        // a plain chain runs a variant that was set for every group, also one
+        // that it reported itself
+        const bool pins = h->mode == RISA_CHAIN_PLAIN && h->split_shape >= 0;
+        if (cur == variant && !pins) return;
         h->drain();
         h->release_graphs();
         ok(risa_hip_bp_set_variant(h->bp, variant));
-        h->split_shape = -1;   // every group with the given variant
+        if (pins) h->split_shape = -1;
+    });
+}
+
+extern "C" int risa_hip_chain_matrix_frames(risa_chain_t h, int* frames)
+{
+    return guarded("risa_hip_chain_matrix_frames", [&] {
+        if (!h || !frames) fail(RISA_ERR_ARG, "null argument");
+        *frames = h->on_matrix_cores(h->per) ? h->split_min : 0;
     });
 }
 
