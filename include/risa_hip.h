@@ -404,7 +404,11 @@ int risa_hip_bp_batched_destroy(risa_bp_batched_t h);
 /* ------------------------------------------------------------------ Chain -- */
 /* The whole per-frame chain on one device with its own scratch buffers.
  * mode 0 = plain FP32 (FFT filter, FP32 backprojection), groups of up to 16
- * frames, or 32 where max_frames >= 64; mode 1 = mixed precision (DFT-GEMM
+ * frames, or 32 where max_frames >= 64; where timing at creation finds it
+ * faster, those groups are backprojected on the matrix cores, with samples and
+ * weights of 22 bits (FP16 hi + lo) and FP32 sums, no further from a float64
+ * result than the FP32 kernel's (risa_hip_chain_matrix_frames says from how
+ * many frames on, risa_hip_chain_set_variant turns it off); mode 1 = mixed precision (DFT-GEMM
  * filter with FP16 output, FP16-sinogram / FP32-accumulate backprojection),
  * groups of up to 32 frames, or 64 where max_frames >= 128 and timing at
  * creation finds them faster.  A run's groups are dealt to two streams forked from and joined

@@ -924,7 +924,20 @@ __global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_groups_kernel(c
 //     pixel m at angle g,
 //   B [4 angles x 8 samples][16 slices]: lane n + 16 g the samples of slice n.
 // Three products per 16 slices, hi hi + lo hi + hi lo, accumulate in FP32;
-// the dropped lo lo term is 2^-24 of a product.  The pixels' coordinates and
+// the dropped lo lo term is 2^-24 of a product.
+//
+// Precision: of the operands' and the sums' rounding only the latter shows, 750
+// additions to ever larger sums at 1000 angles.  Each block of 64 angles is
+// therefore summed for itself and the blocks' sums are added up (32 registers,
+// 32 additions per 64 angles).  Relative RMSE against float64 of a
+// backprojection of ramp-filtered phantoms, by tile 32 x 32 / 16 x 16, and
+// bp_linear_kernel's beside it: 512^2 x 1000 angles 2.68e-6 / 2.68e-6 (2.78e-6 /
+// 2.76e-6; most of it is the angles' own FP32 rounding), 256^2 x 500 1.22e-6 /
+// 1.20e-6 (1.35e-6 / 1.31e-6), 431 detectors on 501^2 x 776 8.4e-7 (1.09e-6),
+// 504 on 454^2 x 763 1.47e-6 (1.61e-6); below it in all 12 geometries of 200 to
+// 560 pixels tried.  As one running sum it was above it, by 1 to 11 per cent.
+//
+// The pixels' coordinates and
 // weights cost the vector unit about 24 instructions per 64 (pixel, angle)
 // pairs whatever the number of slices, where bp_linear_kernel spends 2.8 per
 // pair and slice.
@@ -950,10 +963,12 @@ __global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_groups_kernel(c
 // Bound: LDS reads.  A block's operands take 5 KB per 64 (pixel, angle) pairs
 // (4 KB of samples, 1 KB of selectors) at the ~105 bytes per clock and CU that
 // two-address reads deliver, against about 195 clocks of vector and matrix
-// issue; more waves (6 or 8 per SIMD rather than 4) hide the rest: a wave
-// issues one instruction in 8 clocks at best.  512^2 x 1000 angles, 32 slices:
-// 14.1 us per slice with two launches in flight (packing included, 0.65),
-// bp_linear_kernel 24.5; relative RMSE against float64 2.64e-6 and 2.60e-6.
+// issue.  Four waves per SIMD: the two sets of sums take 64 registers, and six
+// or eight waves would spill them (512^2 x 1000 angles, 32 slices alone, 32 x
+// 32 / 32 x 16 / 16 x 16 tiles: 510 / 505 / 524 us, 624 and 790 for the smaller
+// two with six and eight waves; 384^2 x 700 323 / 269 / 271, bp_linear_kernel
+// 356).  512^2 x 1000 angles, 32 slices: 14.1 us per slice with two launches in
+// flight (packing included, 0.65), bp_linear_kernel 24.5.
 // ---------------------------------------------------------------------------
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -1057,11 +1072,10 @@ __global__ void tune_fill_f16_kernel(uint16_t* out, long n)
 // pixel block as 2 x 2 blocks of 4 x 4.
 using lds_bytes = __attribute__((address_space(3))) char;
 
-template <int TX, int TY, int WPE>
-__global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* __restrict__ packed,
-                                                               float* __restrict__ img,
-                                                               const float* __restrict__ cosT,
-                                                               const float* __restrict__ sinT, int slices, BpParams p)
+template <int TX, int TY>
+__global__ void __launch_bounds__(TX* TY, 4) bp_split_kernel(const unsigned* __restrict__ packed,
+                                                             float* __restrict__ img, const float* __restrict__ cosT,
+                                                             const float* __restrict__ sinT, int slices, BpParams p)
 {
     constexpr int NT = TX * TY, NW = NT / 64;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -1094,11 +1108,20 @@ __global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* _
     const bool active = __any(use);
     const int nch = __syncthreads_or(use) ? (p.P + AE - 1) / AE : 0;
 
-    f4_t acc[4][2];
+    f4_t acc[4][2], sum[4][2];   // of the current block of 64 angles, and of those before
 #pragma unroll
     for (int sb = 0; sb < 4; sb++)
 #pragma unroll
-        for (int u = 0; u < 2; u++) acc[sb][u] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int u = 0; u < 2; u++) acc[sb][u] = sum[sb][u] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    auto add_block = [&]() {
+#pragma unroll
+        for (int sb = 0; sb < 4; sb++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                sum[sb][u] += acc[sb][u];
+                acc[sb][u] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+    };
 
     const unsigned rbase = lds_address(rows), tbase = lds_address(tab);
     // records of angles 64 b .. 64 b + 63 (AE divides 64), slot angle % 128, by
@@ -1213,11 +1236,15 @@ __global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* _
     for (int ch = 0; ch < nch; ch++) {
         // chunks ch and ch + 1 lie in blocks of 64 angles ch AE / 64 and the
         // next: the ring's other half is free for the block after
-        if (ch > 0 && ch * AE % 64 == 0 && ch * AE + 64 < p.P) make_info(ch * AE / 64 + 1);
+        if (ch > 0 && ch * AE % 64 == 0) {
+            if (ch * AE + 64 < p.P) make_info(ch * AE / 64 + 1);
+            add_block();
+        }
         chunk(ch, (lds_bytes*)rows + ((ch + 1) & 1) * bufsz);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's part of chunk ch + 1 is in LDS
         __syncthreads();
     }
+    add_block();
     // lane (n = m, g): pixels 4 g .. 4 g + 3 of a block (its row g), slice 16 u + n
 #pragma unroll
     for (int sb = 0; sb < 4; sb++) {
@@ -1232,7 +1259,7 @@ __global__ void __launch_bounds__(TX* TY, WPE) bp_split_kernel(const unsigned* _
             float* o = img + (long)(16 * u + m) * p.N * p.N + (long)y * p.N + x;
             f4_t r;
 #pragma unroll
-            for (int v = 0; v < 4; v++) r[v] = in[v] ? acc[sb][u][v] * p.norm * p.out_scale : p.maskingValue;
+            for (int v = 0; v < 4; v++) r[v] = in[v] ? sum[sb][u][v] * p.norm * p.out_scale : p.maskingValue;
             if (x + 4 <= p.N && reinterpret_cast<uintptr_t>(o) % 16 == 0) {
                 *reinterpret_cast<f4_t*>(o) = r;
             } else {
@@ -2770,15 +2797,15 @@ extern "C" int risa_hip_bp_run_f16(risa_bp_t h, const uint16_t* sino, float in_s
 
 // ------------------------------------------ FP32 split backprojection --
 // Used by the chain for groups of many frames (chain.hip); its sums are
-// rounded otherwise than bp_linear_kernel's, at the same accuracy.
+// rounded otherwise than bp_linear_kernel's, and no less exact.
 struct SplitShape {
     int tx, ty, amax, variant;   // variant: an FP32 variant of the same tile shape (its dispatch order)
     void (*fn)(const unsigned*, float*, const float*, const float*, int, BpParams);
 };
 static const SplitShape kSplitShapes[] = {
-    {32, 32, 8, 0, bp_split_kernel<32, 32, 4>},
-    {32, 16, 4, 1, bp_split_kernel<32, 16, 6>},
-    {16, 16, 4, 2, bp_split_kernel<16, 16, 8>},
+    {32, 32, 8, 0, bp_split_kernel<32, 32>},
+    {32, 16, 4, 1, bp_split_kernel<32, 16>},
+    {16, 16, 4, 2, bp_split_kernel<16, 16>},
 };
 constexpr int kNumSplitShapes = sizeof(kSplitShapes) / sizeof(kSplitShapes[0]);
 constexpr int kMaxSplitLds = 160 * 1024;   // a gfx950 workgroup's LDS

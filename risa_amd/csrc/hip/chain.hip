@@ -5,8 +5,9 @@
 // before handing the frame on, e.g. Backprojection.cu:203): launches are
 // stream-ordered, and a captured hipGraph replays the launch sequence.
 //
-// PLAIN: frame by frame, FP32 throughout (FFT filter, FP32 backprojector).
-//        Groups of `per` consecutive frames (up to 16, or 32; each stage runs
+// PLAIN: frame by frame, FP32 in and out of every stage (FFT filter, FP32
+//        backprojector; on the matrix cores its products are of FP16 hi + lo
+//        operands, 22 bits, its sums FP32).  Groups of `per` consecutive frames (up to 16, or 32; each stage runs
 //        once per group) are dealt round-robin to `lanes` streams (own scratch
 //        buffers each) forked from and joined back into the caller's stream,
 //        so lanes x per frames are in flight -- the way the reference
@@ -156,7 +157,10 @@ static float split_scale(risa_chain_t h, const float* avg_ref, const float* avg_
     ok(risa_fan2para_gain(h->f2p, &gain));
     const double att = std::max(std::fabs(std::log((double)num / lo)), std::fabs(std::log((double)tiny / hi)));
     const double bound = 1.001 * att * gain * risa_filter_l1(h->filt);
-    if (!(bound > 0.0) || !(bound < 1e6)) return 0.0f;
+    // counts over a flat field give 10 .. 100; with a bound of 4000 the operands'
+    // step (2^-25 / scale) is still 2e-6 of samples of 1e-3, far below the error
+    // of their sums, beyond it is not
+    if (!(bound > 0.0) || !(bound < 4000.0)) return 0.0f;
     return (float)std::exp2(std::floor(std::log2(65000.0 / bound)));
 }
 
