@@ -405,10 +405,14 @@ int risa_hip_bp_batched_destroy(risa_bp_batched_t h);
 /* The whole per-frame chain on one device with its own scratch buffers.
  * mode 0 = plain FP32 (FFT filter, FP32 backprojection), groups of up to 16
  * frames, or 32 where max_frames >= 64; where timing at creation finds it
- * faster, those groups are backprojected on the matrix cores, with samples and
- * weights of 22 bits (FP16 hi + lo) and FP32 sums, no further from a float64
- * result than the FP32 kernel's (risa_hip_chain_matrix_frames says from how
- * many frames on, risa_hip_chain_set_variant turns it off); mode 1 = mixed precision (DFT-GEMM
+ * faster, calls of many frames are backprojected on the matrix cores, with
+ * samples and weights of 22 bits (FP16 hi + lo) and FP32 sums, no further from a
+ * float64 result than the FP32 kernel's.  All frames of a call take the same
+ * way, so a frame's bits do not depend on its place in the call; they do on
+ * the way that calls of so many frames take (risa_hip_chain_on_matrix_cores),
+ * which like the tile shape follows from timing at creation.  Once
+ * risa_hip_chain_set_variant named a variant, they are that variant's in any
+ * call of any chain.  Mode 1 = mixed precision (DFT-GEMM
  * filter with FP16 output, FP16-sinogram / FP32-accumulate backprojection),
  * groups of up to 32 frames, or 64 where max_frames >= 128 and timing at
  * creation finds them faster.  A run's groups are dealt to two streams forked from and joined
@@ -435,9 +439,10 @@ int risa_hip_chain_intermediate(risa_chain_t h, int which, const void** ptr);
  * reference counterpart. */
 int risa_hip_chain_set_variant(risa_chain_t h, int variant);
 int risa_hip_chain_get_variant(risa_chain_t h, int* variant);
-/* From how many frames on a group is backprojected on the matrix cores
- * (0: none is).  Tooling; no reference counterpart. */
-int risa_hip_chain_matrix_frames(risa_chain_t h, int* frames);
+/* Whether a call of `frames` frames is backprojected on the matrix cores (mode 1:
+ * its full groups are; the same bits either way).  Tooling; no reference
+ * counterpart. */
+int risa_hip_chain_on_matrix_cores(risa_chain_t h, int frames, int* yes);
 /* Layout of the raw frames risa_hip_chain_run reads (risa_input_layout;
  * MODULE_MAJOR = the reference's H2D -> Reordering -> Attenuation, with the
  * reordering fused into the attenuation load).  A change synchronises the

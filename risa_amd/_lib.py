@@ -210,7 +210,7 @@ _SIGS = {
     "risa_hip_chain_intermediate": [P, C.c_int, C.POINTER(P)],
     "risa_hip_chain_set_variant": [P, C.c_int],
     "risa_hip_chain_get_variant": [P, C.POINTER(C.c_int)],
-    "risa_hip_chain_matrix_frames": [P, C.POINTER(C.c_int)],
+    "risa_hip_chain_on_matrix_cores": [P, C.c_int, C.POINTER(C.c_int)],
     "risa_hip_chain_set_input_layout": [P, C.c_int],
     "risa_hip_chain_graph_count": [P, C.POINTER(C.c_int)],
     "risa_hip_chain_destroy": [P],

@@ -1068,11 +1068,11 @@ __global__ void tune_fill_f16_kernel(uint16_t* out, long n)
         out[i] = float_to_half_bits((float)((int)((unsigned)i * 2654435761u) >> 8) * 0x1p-24f);
 }
 
-// Workgroup x: a TX x TY tile of the (up to) 32 slices; each wave an 8 x 8
-// pixel block as 2 x 2 blocks of 4 x 4.
+// Workgroup x: a TX x TY tile of up to 16 NU slices (a slice's bits do not depend
+// on NU); each wave an 8 x 8 pixel block as 2 x 2 blocks of 4 x 4.
 using lds_bytes = __attribute__((address_space(3))) char;
 
-template <int TX, int TY>
+template <int TX, int TY, int NU>
 __global__ void __launch_bounds__(TX* TY, 4) bp_split_kernel(const unsigned* __restrict__ packed,
                                                              float* __restrict__ img, const float* __restrict__ cosT,
                                                              const float* __restrict__ sinT, int slices, BpParams p)
@@ -1108,16 +1108,16 @@ __global__ void __launch_bounds__(TX* TY, 4) bp_split_kernel(const unsigned* __r
     const bool active = __any(use);
     const int nch = __syncthreads_or(use) ? (p.P + AE - 1) / AE : 0;
 
-    f4_t acc[4][2], sum[4][2];   // of the current block of 64 angles, and of those before
+    f4_t acc[4][NU], sum[4][NU];   // of the current block of 64 angles, and of those before
 #pragma unroll
     for (int sb = 0; sb < 4; sb++)
 #pragma unroll
-        for (int u = 0; u < 2; u++) acc[sb][u] = sum[sb][u] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int u = 0; u < NU; u++) acc[sb][u] = sum[sb][u] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
     auto add_block = [&]() {
 #pragma unroll
         for (int sb = 0; sb < 4; sb++)
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
+            for (int u = 0; u < NU; u++) {
                 sum[sb][u] += acc[sb][u];
                 acc[sb][u] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
             }
@@ -1199,9 +1199,9 @@ __global__ void __launch_bounds__(TX* TY, 4) bp_split_kernel(const unsigned* __r
                     unsigned at = rb + (unsigned)kb * (kSplitRow / 2);
                     unsigned hi, lo;
                     split_pair(1.0f - f, f, hi, lo);
-                    lds_u4 bh[2], bl[2];
+                    lds_u4 bh[NU], bl[NU];
 #pragma unroll
-                    for (int u = 0; u < 2; u++) {
+                    for (int u = 0; u < NU; u++) {
                         // opaque bases: each two-address read then fills two
                         // adjacent registers of one operand
                         asm("" : "+v"(at));
@@ -1224,11 +1224,11 @@ __global__ void __launch_bounds__(TX* TY, 4) bp_split_kernel(const unsigned* __r
                                                                    __builtin_bit_cast(h8_t, b), c, 0, 0, 0);
                     };
 #pragma unroll
-                    for (int u = 0; u < 2; u++) mma(acc[sb][u], al, bh[u]);
+                    for (int u = 0; u < NU; u++) mma(acc[sb][u], al, bh[u]);
 #pragma unroll
-                    for (int u = 0; u < 2; u++) mma(acc[sb][u], ah, bl[u]);
+                    for (int u = 0; u < NU; u++) mma(acc[sb][u], ah, bl[u]);
 #pragma unroll
-                    for (int u = 0; u < 2; u++) mma(acc[sb][u], ah, bh[u]);
+                    for (int u = 0; u < NU; u++) mma(acc[sb][u], ah, bh[u]);
                 }
             }
         }
@@ -1254,7 +1254,7 @@ __global__ void __launch_bounds__(TX* TY, 4) bp_split_kernel(const unsigned* __r
 #pragma unroll
         for (int v = 0; v < 4; v++) in[v] = !(p.mask && bp_outside(x + v, y, p.N, p.center));
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
+        for (int u = 0; u < NU; u++) {
             if (16 * u + m >= slices) continue;
             float* o = img + (long)(16 * u + m) * p.N * p.N + (long)y * p.N + x;
             f4_t r;
@@ -2800,12 +2800,12 @@ extern "C" int risa_hip_bp_run_f16(risa_bp_t h, const uint16_t* sino, float in_s
 // rounded otherwise than bp_linear_kernel's, and no less exact.
 struct SplitShape {
     int tx, ty, amax, variant;   // variant: an FP32 variant of the same tile shape (its dispatch order)
-    void (*fn)(const unsigned*, float*, const float*, const float*, int, BpParams);
+    void (*fn[2])(const unsigned*, float*, const float*, const float*, int, BpParams);   // up to 16 and 32 slices
 };
 static const SplitShape kSplitShapes[] = {
-    {32, 32, 8, 0, bp_split_kernel<32, 32>},
-    {32, 16, 4, 1, bp_split_kernel<32, 16>},
-    {16, 16, 4, 2, bp_split_kernel<16, 16>},
+    {32, 32, 8, 0, {bp_split_kernel<32, 32, 1>, bp_split_kernel<32, 32, 2>}},
+    {32, 16, 4, 1, {bp_split_kernel<32, 16, 1>, bp_split_kernel<32, 16, 2>}},
+    {16, 16, 4, 2, {bp_split_kernel<16, 16, 1>, bp_split_kernel<16, 16, 2>}},
 };
 constexpr int kNumSplitShapes = sizeof(kSplitShapes) / sizeof(kSplitShapes[0]);
 constexpr int kMaxSplitLds = 160 * 1024;   // a gfx950 workgroup's LDS
@@ -2863,16 +2863,17 @@ extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, floa
         hipLaunchKernelGGL(split_pack_kernel, dim3(ceil_div(split_rows(p.D) - 2, 32), p.P), dim3(256), 0, s, sino,
                            slices, p.P, p.D, scale, pk);
         check_launch("split_pack_kernel");
-        hipLaunchKernelGGL(v.fn, grid, dim3(v.tx * v.ty), lds, s, pk, img, h->cosT.ptr, h->sinT.ptr, slices, p);
+        hipLaunchKernelGGL(v.fn[slices > kSplitSlices / 2], grid, dim3(v.tx * v.ty), lds, s, pk, img, h->cosT.ptr,
+                           h->sinT.ptr, slices, p);
         check_launch("bp_split_kernel");
     });
 }
 
 // Times the split shapes at 32 slices against the handle's FP32 variant on
-// the same launch: `shape` gets the fastest one and `min_slices` the batch
-// from which it beats the variant (its cost does not depend on the slices up
-// to 32, the variant's is about proportional), or more than 32 if never.
-extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, int* min_slices)
+// the same launch: `shape` gets the fastest one, cost[0] and cost[1] what its
+// launches of up to 16 and up to 32 slices take, in slices of the variant (whose
+// time is about proportional).
+extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, float cost[2])
 {
     return guarded("risa_bp_tune_split", [&] {
         DeviceGuard dg(h->device);
@@ -2903,22 +2904,27 @@ extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, int* m
             RISA_HIP_CHECK(hipEventElapsedTime(&ms, ev.a, ev.b));
             return ms;
         };
-        float plain = 1e30f, best = 1e30f;
+        auto time_split = [&](int v, int slices) {
+            return time_it([&] {
+                if (risa_bp_run_split(h, v, sino.ptr, 1024.0f, slices, packed.ptr, img.ptr, s) != RISA_OK)
+                    fail(RISA_ERR_HIP, "%s", risa_last_error());
+            });
+        };
+        float plain = 1e30f, best = 1e30f, half = 1e30f;
         *shape = 0;
         for (int round = 0; round < 2; round++) {
             plain = std::min(plain, time_it([&] { launch_linear(h, h->variant, sino.ptr, img.ptr, kSplitSlices, s); }));
             for (int v = 0; v < kNumSplitShapes; v++) {
-                const float ms = time_it([&] {
-                    if (risa_bp_run_split(h, v, sino.ptr, 1024.0f, kSplitSlices, packed.ptr, img.ptr, s) != RISA_OK)
-                        fail(RISA_ERR_HIP, "%s", risa_last_error());
-                });
+                const float ms = time_split(v, kSplitSlices);
                 if (ms < best) {
                     best = ms;
                     *shape = v;
                 }
             }
         }
-        *min_slices = 1 + (int)(kSplitSlices * best / plain);
+        for (int round = 0; round < 2; round++) half = std::min(half, time_split(*shape, kSplitSlices / 2));
+        cost[0] = kSplitSlices * half / plain;
+        cost[1] = kSplitSlices * best / plain;
     });
 }
 

@@ -12,9 +12,9 @@
 //        buffers each) forked from and joined back into the caller's stream,
 //        so lanes x per frames are in flight -- the way the reference
 //        overlaps frames across its per-stage threads.  Chains of at least 64
-//        frames take groups of 32 and backproject those of at least split_min
-//        frames on the matrix cores (bp_split_kernel), where timing both at
-//        creation finds that the faster way: 256 frames of 512^2 x 1000 angles
+//        frames take groups of 32 and backproject a call on the matrix cores
+//        (bp_split_kernel) where timing both at creation says that this is the
+//        faster way for its number of frames: 256 frames of 512^2 x 1000 angles
 //        4.15 ms a call, 6.67 with bp_linear_kernel; 256^2 x 500 stays with
 //        the latter (158 us per 32 slices against 208).
 // MIXED: groups of `per` consecutive frames (a multiple of 4, up to 32) dealt
@@ -43,7 +43,7 @@ extern "C" size_t risa_bp_f16_pack_bytes(risa_bp_t h);
 extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int* min_slices);
 extern "C" int risa_bp_run_f16_packed(risa_bp_t h, const uint16_t* sino_x4, float in_scale, int slices, void* packed,
                                       float* img, hipStream_t s);
-extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, int* min_slices);
+extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, float cost[2]);
 extern "C" int risa_bp_run_split(risa_bp_t h, int shape, const float* sino, float scale, int slices, void* packed, float* img,
                       hipStream_t s);
 
@@ -79,11 +79,15 @@ struct risa_chain_s {
     risa_bp_t bp = nullptr;
     risa::DeviceBuffer<float> att_buf, par_buf, filt_buf;   // `per` frame slots per lane
     risa::DeviceBuffer<uint16_t> f16_buf;                   // MIXED: `per` slots per lane, x4 layout
-    // Groups of at least split_min frames are backprojected on the matrix cores
-    // (split_shape -1: none).  PLAIN: tile shape split_shape, FP16 hi + lo
+    // Backprojection on the matrix cores (split_shape -1: none).  PLAIN: all
+    // groups of a call or none (split_call), so that a frame's bits do not depend
+    // on its place in the call, with tile shape split_shape and FP16 hi + lo
     // operands that hold filtered sample * split_scale, until the caller sets a
-    // variant; MIXED: while the FP16 variant is one whose bits that kernel has
+    // variant; split_cost: of a group of up to 16 and up to 32 frames, in frames of
+    // the FP32 variant.  MIXED: groups of at least split_min frames, while the
+    // FP16 variant is one whose bits that kernel has
     int split_shape = -1, split_min = 0;
+    float split_cost[2] = {0.0f, 0.0f};
     float split_scale = 0.0f;
     risa::DeviceBuffer<char> split_buf;                     // packed sinograms, one launch per lane
     size_t split_bytes = 0;
@@ -104,7 +108,8 @@ struct risa_chain_s {
         (void)hipDeviceSynchronize();
         if (prev != device) (void)hipSetDevice(prev);
     }
-    bool on_matrix_cores(int n) const;
+    bool split_call(int frames) const;
+    bool packed_group(int n) const;
     void release_graphs()
     {
         for (auto& kv : graphs) (void)hipGraphExecDestroy(kv.second.exec);
@@ -125,9 +130,20 @@ struct risa_chain_s {
 
 using namespace risa;
 
-bool risa_chain_s::on_matrix_cores(int n) const
+// Whether a plain call takes no longer on the matrix cores, tail included, than
+// with the FP32 variant.  512^2 x 1000 angles, 32 / 48 / 65 frames on the matrix
+// cores 630 / 1030 / 1580 us, 32 / 33 with the variant 890 / 1060; with only the
+// full groups on the matrix cores 65 took 1370.
+bool risa_chain_s::split_call(int frames) const
 {
-    return split_shape >= 0 && n >= split_min && (mode == RISA_CHAIN_PLAIN || risa_bp_f16_pack_bytes(bp) > 0);
+    if (mode != RISA_CHAIN_PLAIN || split_shape < 0) return false;
+    const int tail = frames % kSplitPer;
+    const float last = tail == 0 ? 0.0f : split_cost[tail > kSplitPer / 2];
+    return (float)(frames / kSplitPer) * split_cost[1] + last <= (float)frames;
+}
+bool risa_chain_s::packed_group(int n) const
+{
+    return mode == RISA_CHAIN_MIXED && split_shape >= 0 && n >= split_min && risa_bp_f16_pack_bytes(bp) > 0;
 }
 
 static void ok(int rc)
@@ -193,9 +209,8 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
                 if (max_frames >= kPlainLanes * kSplitPer && (h->split_bytes = risa_bp_split_bytes(h->bp)) > 0 &&
                     (h->split_scale = split_scale(h, avg_ref, avg_dark)) > 0.0f) {
                     ok(risa_hip_bp_autotune_batch(h->bp, kPlainLanes * kPlainMaxPer, nullptr));
-                    ok(risa_bp_tune_split(h->bp, nullptr, &h->split_shape, &h->split_min));
-                    if (h->split_min <= kSplitPer) {
-                        h->per = kSplitPer;
+                    ok(risa_bp_tune_split(h->bp, nullptr, &h->split_shape, h->split_cost));
+                    if (h->split_cost[1] <= (float)kSplitPer) {
                         h->split_bytes = (h->split_bytes + 255) / 256 * 256;
                         h->split_buf.resize(h->split_bytes * h->lanes);
                     } else {
@@ -248,7 +263,7 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
             // itself per variant, eagerly, proved too noisy to rank the closest
             // shapes
             if (mode == RISA_CHAIN_PLAIN) {
-                if (h->split_min > 0) {
+                if (h->split_cost[1] > 0.0f) {
                     // tuned above
                 } else if (h->per > 1) ok(risa_hip_bp_autotune_batch(h->bp, std::min(kPlainLanes * kPlainMaxPer, h->lanes * h->per), nullptr));
                 else ok(risa_hip_bp_autotune_slices(h->bp, h->lanes, nullptr));
@@ -271,6 +286,7 @@ static void enqueue(risa_chain_t h, const uint16_t* raw, const int32_t* planes, 
     const int per = h->per;
     const int groups = (frames + per - 1) / per;
     const int lanes = std::min(h->lanes, groups);
+    const bool matrix = h->split_call(frames);
     RISA_HIP_CHECK(hipEventRecord(h->lane_events[0], s));
     for (int k = 0; k < lanes; k++) RISA_HIP_CHECK(hipStreamWaitEvent(h->lane_streams[k], h->lane_events[0], 0));
     for (int q = 0; q < groups; q++) {
@@ -283,24 +299,24 @@ static void enqueue(risa_chain_t h, const uint16_t* raw, const int32_t* planes, 
             if (n == 1) {
                 ok(risa_hip_attenuation_run(h->att, raw + f * fan, planes[f], att, ls));
                 ok(risa_hip_fan2para_run(h->f2p, att, planes[f], pb, ls));
-                ok(risa_filter_run_oop(h->filt, pb, fb, g.numberOfParallelProjections, ls));
-                ok(risa_hip_bp_run(h->bp, fb, img + f * out, ls));
             } else {
                 ok(risa_hip_attenuation_run_batch(h->att, raw + f * fan, planes + f, n, att, ls));
                 ok(risa_hip_fan2para_run_batch(h->f2p, att, planes + f, n, pb, ls));
-                ok(risa_filter_run_oop(h->filt, pb, fb, (long)n * g.numberOfParallelProjections, ls));
-                if (h->on_matrix_cores(n))
-                    ok(risa_bp_run_split(h->bp, h->split_shape, fb, h->split_scale, n, h->split_buf.ptr + k * h->split_bytes,
-                                         img + f * out, ls));
-                else
-                    ok(risa_hip_bp_run_batch(h->bp, fb, n, img + f * out, ls));
             }
+            ok(risa_filter_run_oop(h->filt, pb, fb, (long)n * g.numberOfParallelProjections, ls));
+            if (matrix)
+                ok(risa_bp_run_split(h->bp, h->split_shape, fb, h->split_scale, n, h->split_buf.ptr + k * h->split_bytes,
+                                     img + f * out, ls));
+            else if (n == 1)
+                ok(risa_hip_bp_run(h->bp, fb, img + f * out, ls));
+            else
+                ok(risa_hip_bp_run_batch(h->bp, fb, n, img + f * out, ls));
         } else {
             uint16_t* hb = h->f16_buf.ptr + (size_t)k * per * par;
             ok(risa_hip_attenuation_run_batch(h->att, raw + f * fan, planes + f, n, att, ls));
             ok(risa_hip_fan2para_run_batch(h->f2p, att, planes + f, n, pb, ls));
             ok(risa_hip_filter_run_f16x4(h->filt, pb, hb, n, kF16SinoScale, ls));
-            if (h->on_matrix_cores(n))
+            if (h->packed_group(n))
                 ok(risa_bp_run_f16_packed(h->bp, hb, kF16SinoScale, n, h->split_buf.ptr + k * h->split_bytes,
                                           img + f * out, ls));
             else
@@ -409,11 +425,11 @@ extern "C" int risa_hip_chain_set_variant(risa_chain_t h, int variant)
     });
 }
 
-extern "C" int risa_hip_chain_matrix_frames(risa_chain_t h, int* frames)
+extern "C" int risa_hip_chain_on_matrix_cores(risa_chain_t h, int frames, int* yes)
 {
-    return guarded("risa_hip_chain_matrix_frames", [&] {
-        if (!h || !frames) fail(RISA_ERR_ARG, "null argument");
-        *frames = h->on_matrix_cores(h->per) ? h->split_min : 0;
+    return guarded("risa_hip_chain_on_matrix_cores", [&] {
+        if (!h || !yes || frames < 1) fail(RISA_ERR_ARG, "bad argument");
+        *yes = h->split_call(frames) || h->packed_group(std::min(frames, h->per)) ? 1 : 0;
     });
 }
 

@@ -396,12 +396,11 @@ class Chain(_Handle):
     def variant(self, v: int):
         check(load().risa_hip_chain_set_variant(self.h, v))
 
-    @property
-    def matrix_frames(self) -> int:
-        """Groups of at least this many frames are backprojected on the matrix cores (0: none)."""
-        n = C.c_int()
-        check(load().risa_hip_chain_matrix_frames(self.h, C.byref(n)))
-        return n.value
+    def on_matrix_cores(self, frames: int) -> bool:
+        """Whether a call of `frames` frames is backprojected on the matrix cores (mixed: its full groups)."""
+        yes = C.c_int()
+        check(load().risa_hip_chain_on_matrix_cores(self.h, frames, C.byref(yes)))
+        return bool(yes.value)
 
     def set_input_layout(self, layout: int):
         check(load().risa_hip_chain_set_input_layout(self.h, layout))

@@ -29,7 +29,7 @@ def test_set_variant_pins_every_frame(risa, geom_c1, cuda):
     fs, raw, planes = _frames(geom_c1, cuda, F)
     a = device.Chain(geom_c1, fs.avg_ref, fs.avg_dark, mode=risa.CHAIN_PLAIN, max_frames=F)
     b = device.Chain(geom_c1, fs.avg_ref, fs.avg_dark, mode=risa.CHAIN_PLAIN, max_frames=1)
-    assert 0 < a.matrix_frames <= 32 and b.matrix_frames == 0
+    assert a.on_matrix_cores(F) and not b.on_matrix_cores(1)
     s = torch.cuda.Stream()
     img = torch.full((F,) + geom_c1.img_shape, float("nan"), dtype=torch.float32, device=cuda)
     with torch.cuda.stream(s):
@@ -37,7 +37,7 @@ def test_set_variant_pins_every_frame(risa, geom_c1, cuda):
     s.synchronize()
     a.variant = a.variant
     b.variant = a.variant
-    assert a.matrix_frames == 0 and a.graph_count() == 0
+    assert not a.on_matrix_cores(F) and a.graph_count() == 0
     print(f"case: plain C1, {F} frames, variant {a.variant & 0xff} set", flush=True)
     one = torch.empty((1,) + geom_c1.img_shape, dtype=torch.float32, device=cuda)
     for graph in (False, True):
@@ -61,14 +61,72 @@ def test_mixed_variants_keep_the_matrix_path(risa, geom_c1, cuda):
 
     fs = FrameSet(geom_c1, 1, 2, R=2)
     a = device.Chain(geom_c1, fs.avg_ref, fs.avg_dark, mode=risa.CHAIN_MIXED, max_frames=128)
-    own, frames = a.variant, a.matrix_frames
-    print(f"case: mixed C1, variant {own >> 8}, groups of {frames} frames on the matrix cores", flush=True)
+    own, frames = a.variant, a.on_matrix_cores(64)
+    print(f"case: mixed C1, variant {own >> 8}, groups of 64 frames on the matrix cores: {frames}", flush=True)
     a.variant = own
     a.variant = own ^ 1                 # another FP32 variant, which this chain does not run
-    assert a.matrix_frames == frames
+    assert a.on_matrix_cores(64) == frames
     wide = next(v for v in range(device.bp_num_variants(True)) if device.bp_variant_shape(True, v)[1] == 32)
     a.variant = wide << 8
-    assert a.matrix_frames == 0
+    assert not a.on_matrix_cores(64)
     a.variant = own
-    assert a.matrix_frames == frames
+    assert a.on_matrix_cores(64) == frames
     a.close()
+
+
+def test_a_frames_place_does_not_matter(risa, geom_c1, cuda):
+    """The same raw frame at every place of plain calls of several lengths: one
+    image, bit for bit, within a call and for all calls of one way; the two
+    ways within rounding of each other (5e-6, as the kernels)."""
+    import torch
+    from risa_amd import device
+
+    F = 97
+    fs, raw, _ = _frames(geom_c1, cuda, F)
+    raw[:] = raw[0].clone()
+    a = device.Chain(geom_c1, fs.avg_ref, fs.avg_dark, mode=risa.CHAIN_PLAIN, max_frames=F)
+    assert a.on_matrix_cores(64)
+    first = {}
+    for n in (1, 2, 17, 32, 33, 64, 65, 70, 97):
+        way = a.on_matrix_cores(n)
+        print(f"case: plain C1, {n} equal frames, matrix cores: {way}", flush=True)
+        img = torch.full((n,) + geom_c1.img_shape, float("nan"), dtype=torch.float32, device=cuda)
+        a(raw[:n], np.zeros(n, np.int32), img)
+        torch.cuda.synchronize()
+        assert bool((img == img[0]).all())
+        if way in first:
+            assert torch.equal(img[0], first[way])
+        first[way] = img[0]
+    if len(first) == 2:
+        assert float((first[True] - first[False]).norm() / first[False].norm()) < 5e-6
+    a.close()
+
+
+@pytest.mark.parametrize("N,P,D,S", [(64, 70, 61, 16), (48, 5, 50, 1), (130, 64, 100, 9)])
+def test_few_slices_have_the_same_bits(risa, geom_c0, cuda, N, P, D, S):
+    """Launches of up to 16 slices read half of each packed row: the bits of the
+    same slices in a launch of 32."""
+    import ctypes as C
+
+    import torch
+    from risa_amd import device
+
+    lib = risa.load()
+    run, size = lib.risa_bp_run_split, lib.risa_bp_split_bytes
+    run.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_float, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]
+    run.restype, size.argtypes, size.restype = C.c_int, [C.c_void_p], C.c_size_t
+    bp = device.Backprojection(geom_c0.replace(numberOfPixels=N, numberOfParallelProjections=P,
+                                               numberOfParallelDetectors=D))
+    x = torch.from_numpy(np.random.default_rng(N).standard_normal((32, P, D)).astype(np.float32)).to(cuda)
+    packed = torch.full((size(bp.h),), 0x7f, dtype=torch.uint8, device=cuda)
+    for shape in range(3):
+        out = []
+        for n in (32, S):
+            out.append(torch.full((n + 1, N, N), 7.0, dtype=torch.float32, device=cuda))
+            rc = run(bp.h, shape, x.data_ptr(), 1024.0, n, packed.data_ptr(), out[-1].data_ptr(),
+                     torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, lib.risa_last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0][:S], out[1][:S])
+        assert bool((out[1][S] == 7.0).all() and (out[0][32] == 7.0).all())
+    bp.close()
