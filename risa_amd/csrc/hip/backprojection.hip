@@ -20,6 +20,7 @@
 #include "device_common.h"
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 #include <vector>
 #include <cmath>
@@ -2928,18 +2929,26 @@ extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, float 
     });
 }
 
+static void autotune(risa_bp_t h, int s32, int s16, hipStream_t s, int max_sb = 1, bool keep_tile = false,
+                     int max_q = INT_MAX);
+
 // -------------------------------- FP16 backprojection of 64 slices at once --
 // Used by the mixed chain for groups of many frames (chain.hip), in place of an
 // FP16 variant whose results it has bit for bit.
+static bool f16_packable(risa_bp_t h)
+{
+    const risa_geom& g = h->g;
+    const BpF16Variant& v = kF16Variants[h->variant_f16];
+    return !g.useTextureMemory && g.interpolationType != 1 && h->lut.scale <= kSplitMaxScale && v.tx == 16 && v.ty == 16;
+}
+
 // Bytes of packed samples for 64 slices, or 0 where the handle's geometry or
 // its FP16 variant (another tile than 16 x 16, or shared angles) has no
 // counterpart there.
 extern "C" size_t risa_bp_f16_pack_bytes(risa_bp_t h)
 {
     const risa_geom& g = h->g;
-    const BpF16Variant& v = kF16Variants[h->variant_f16];
-    if (g.useTextureMemory || g.interpolationType == 1 || h->lut.scale > kSplitMaxScale || v.tx != 16 || v.ty != 16 || v.q != 1)
-        return 0;
+    if (!f16_packable(h) || kF16Variants[h->variant_f16].q != 1) return 0;
     return (size_t)g.numberOfParallelProjections * pack_rows(g.numberOfParallelDetectors) * kPackSlices * 4;
 }
 
@@ -2973,15 +2982,23 @@ extern "C" int risa_bp_run_f16_packed(risa_bp_t h, const uint16_t* sino_x4, floa
     });
 }
 
-// Times it at 64 slices against the handle's FP16 variant: `min_slices` is the
-// batch from which it is the faster one (its cost does not depend on the
-// slices up to 64), or more than 64 if never.
-extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int* min_slices)
+// Times it at 64 slices against the handle's FP16 variant, where that has a
+// 16 x 16 tile: `min_slices` is the batch from which it is the faster one (its
+// cost does not depend on the slices up to 64), or more than 64 if never.  If it
+// is, a variant with shared angles gives way to the fastest one of the same tile
+// without at `slices` slices, whose bits the packed kernel has, for the batches
+// below.
+extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int slices, int* min_slices)
 {
     return guarded("risa_bp_tune_f16_packed", [&] {
+        *min_slices = kPackSlices + 1;
+        if (!f16_packable(h)) return;
         DeviceGuard dg(h->device);
         const size_t ns = (size_t)h->g.numberOfParallelProjections * h->g.numberOfParallelDetectors;
         const size_t ni = (size_t)h->g.numberOfPixels * h->g.numberOfPixels;
+        const int own = h->variant_f16;
+        if (kF16Variants[own].q != 1) autotune(h, 0, slices, s, 1, true, 1);
+        const int whole = h->variant_f16;
         DeviceBuffer<uint16_t> sino(ns * kPackSlices);
         DeviceBuffer<float> img(ni * kPackSlices);
         DeviceBuffer<char> packed(risa_bp_f16_pack_bytes(h));
@@ -3007,8 +3024,8 @@ extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int* min_slic
             float plain = 1e30f, best = 1e30f;
             for (int round = 0; round < 2; round++) {
                 plain = std::min(plain, time_it([&] {
-                                     launch_f16x4(h, h->variant_f16, reinterpret_cast<const uint2*>(sino.ptr), 1.0f,
-                                                  kPackSlices, img.ptr, s);
+                                     launch_f16x4(h, own, reinterpret_cast<const uint2*>(sino.ptr), 1.0f, kPackSlices,
+                                                  img.ptr, s);
                                  }));
                 best = std::min(best, time_it([&] {
                                     if (risa_bp_run_f16_packed(h, sino.ptr, 1.0f, kPackSlices, packed.ptr, img.ptr, s) !=
@@ -3019,9 +3036,11 @@ extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int* min_slic
             *min_slices = 1 + (int)(kPackSlices * best / plain);
         } catch (...) {
             destroy();
+            h->variant_f16 = own;
             throw;
         }
         destroy();
+        h->variant_f16 = *min_slices <= kPackSlices ? whole : own;
     });
 }
 
@@ -3185,11 +3204,12 @@ extern "C" int risa_hip_bp_get_variant(risa_bp_t h, int* variant)
 // workgroup (1 for callers that launch one slice at a time).
 //
 // The FP16 tile shape is picked among the variants whose angles are not shared,
-// or kept (keep_tile), and the variant among those of that shape: a weight's
+// or kept (keep_tile), and the variant among those of that shape, with angles
+// shared by at most max_q groups: a weight's
 // FP16 rounding depends on t's distance from the tile's origin, so results move
 // by up to 2e-5 (noise) from one shape to another, and by the order of the sums,
 // 1e-6, within one.
-static void autotune(risa_bp_t h, int s32, int s16, hipStream_t s, int max_sb = 1, bool keep_tile = false)
+static void autotune(risa_bp_t h, int s32, int s16, hipStream_t s, int max_sb, bool keep_tile, int max_q)
 {
     DeviceGuard dg(h->device);
     const BpF16Variant kept = kF16Variants[h->variant_f16];
@@ -3227,6 +3247,7 @@ static void autotune(risa_bp_t h, int s32, int s16, hipStream_t s, int max_sb = 
             }
             for (int v = 0; s16 > 0 && v < kNumF16Variants; v++) {
                 if (keep_tile && (kF16Variants[v].tx != kept.tx || kF16Variants[v].ty != kept.ty)) continue;
+                if (kF16Variants[v].q > max_q) continue;
                 try {
                     t16[v] = std::min(t16[v],
                                       time_it([&] { launch_f16x4(h, v, sino16.ptr, 1.0f, s16, img.ptr, s); }));

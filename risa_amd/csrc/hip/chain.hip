@@ -40,7 +40,7 @@ int risa_fan2para_gain(risa_fan2para_t h, double* gain);
 extern "C" size_t risa_bp_split_bytes(risa_bp_t h);
 extern "C" int risa_bp_autotune_f16_tile(risa_bp_t h, int slices);
 extern "C" size_t risa_bp_f16_pack_bytes(risa_bp_t h);
-extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int* min_slices);
+extern "C" int risa_bp_tune_f16_packed(risa_bp_t h, hipStream_t s, int slices, int* min_slices);
 extern "C" int risa_bp_run_f16_packed(risa_bp_t h, const uint16_t* sino_x4, float in_scale, int slices, void* packed,
                                       float* img, hipStream_t s);
 extern "C" int risa_bp_tune_split(risa_bp_t h, hipStream_t s, int* shape, float cost[2]);
@@ -232,12 +232,12 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
                 const int half = (max_frames + kMixedLanes - 1) / kMixedLanes;
                 ok(risa_hip_bp_autotune_f16(h->bp, std::min(kMixedMaxPer, (half + 3) / 4 * 4), nullptr));
                 ok(risa_bp_autotune_f16_tile(h->bp, h->per));
-                if (max_frames >= kMixedLanes * kPackPer && (h->split_bytes = risa_bp_f16_pack_bytes(h->bp)) > 0) {
-                    ok(risa_bp_tune_f16_packed(h->bp, nullptr, &h->split_min));
+                if (max_frames >= kMixedLanes * kPackPer) {
+                    ok(risa_bp_tune_f16_packed(h->bp, nullptr, h->per, &h->split_min));
                     if (h->split_min <= kPackPer) {
                         h->per = kPackPer;
                         h->split_shape = 0;
-                        h->split_bytes = (h->split_bytes + 255) / 256 * 256;
+                        h->split_bytes = (risa_bp_f16_pack_bytes(h->bp) + 255) / 256 * 256;
                         h->split_buf.resize(h->split_bytes * kMixedLanes);
                     }
                 }

@@ -130,3 +130,32 @@ def test_few_slices_have_the_same_bits(risa, geom_c0, cuda, N, P, D, S):
         assert torch.equal(out[0][:S], out[1][:S])
         assert bool((out[1][S] == 7.0).all() and (out[0][32] == 7.0).all())
     bp.close()
+
+
+def test_packed_kernel_is_tried_whatever_shares_the_angles(risa, geom_c1, cuda):
+    """The 64-slice kernel is timed for every 16 x 16 tile; where it is taken, a
+    variant with shared angles gives way to one whose bits it has, and a variant
+    of another tile stays and is not replaced."""
+    import ctypes as C
+
+    from risa_amd import device
+
+    lib = risa.load()
+    tune, size = lib.risa_bp_tune_f16_packed, lib.risa_bp_f16_pack_bytes
+    tune.argtypes, tune.restype = [C.c_void_p, C.c_void_p, C.c_int, C.POINTER(C.c_int)], C.c_int
+    size.argtypes, size.restype = [C.c_void_p], C.c_size_t
+    bp = device.Backprojection(geom_c1)
+    for v in range(device.bp_num_variants(True)):
+        square = device.bp_variant_shape(True, v)[:2] == (16, 16)
+        shared = lib.risa_bp_variant_groups(1, v) > 1
+        bp.variant = v << 8
+        n = C.c_int()
+        assert tune(bp.h, None, 32, C.byref(n)) == 0, lib.risa_last_error()
+        now = bp.variant >> 8
+        print(f"case: FP16 variant {v} (16 x 16: {square}, shared angles: {shared}): packed from {n.value}, then {now}",
+              flush=True)
+        assert (n.value <= 64) == square   # 512^2 x 1000 angles: 11 us a slice, 14 and more with any variant
+        if square:
+            assert size(bp.h) > 0 and device.bp_variant_shape(True, now)[:2] == (16, 16)
+        assert now == v or (square and shared)
+    bp.close()
