@@ -2810,6 +2810,7 @@ static const SplitShape kSplitShapes[] = {
 };
 constexpr int kNumSplitShapes = sizeof(kSplitShapes) / sizeof(kSplitShapes[0]);
 constexpr int kMaxSplitLds = 160 * 1024;   // a gfx950 workgroup's LDS
+constexpr int kMaxPackAngles = 65535;      // the packing kernels take one grid row per angle
 
 // Angles of a shape's chunk: the shape's most, or half as often as its LDS asks.
 static int split_angles(int shape, int W)
@@ -2838,7 +2839,9 @@ extern "C" int risa_bp_split_layout(int shape, float scale, int layout[7])
 extern "C" size_t risa_bp_split_bytes(risa_bp_t h)
 {
     const risa_geom& g = h->g;
-    if (g.useTextureMemory || g.interpolationType == 1 || h->lut.scale > kSplitMaxScale) return 0;
+    if (g.useTextureMemory || g.interpolationType == 1 || h->lut.scale > kSplitMaxScale ||
+        g.numberOfParallelProjections > kMaxPackAngles)
+        return 0;
     return (size_t)g.numberOfParallelProjections * split_rows(g.numberOfParallelDetectors) * kSplitRow;
 }
 
@@ -2939,7 +2942,8 @@ static bool f16_packable(risa_bp_t h)
 {
     const risa_geom& g = h->g;
     const BpF16Variant& v = kF16Variants[h->variant_f16];
-    return !g.useTextureMemory && g.interpolationType != 1 && h->lut.scale <= kSplitMaxScale && v.tx == 16 && v.ty == 16;
+    return !g.useTextureMemory && g.interpolationType != 1 && h->lut.scale <= kSplitMaxScale &&
+           g.numberOfParallelProjections <= kMaxPackAngles && v.tx == 16 && v.ty == 16;
 }
 
 // Bytes of packed samples for 64 slices, or 0 where the handle's geometry or

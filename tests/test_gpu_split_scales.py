@@ -50,3 +50,21 @@ def test_split_scales(risa, geom_c0, cuda, N, D, P):
         print(f"  worst rel RMSE of a slice {max(err):.2e}", flush=True)
         assert max(err) < TOL
     bp.close()
+
+
+def test_more_angles_than_a_grid_has_rows(risa, geom_c0, cuda):
+    """The packing kernels launch a grid row per angle, 65535 at most; a geometry
+    with more keeps the FP32 and FP16 variants."""
+    from risa_amd import device
+
+    lib = risa.load()
+    sizes = [lib.risa_bp_split_bytes, lib.risa_bp_f16_pack_bytes]
+    for size in sizes:
+        size.argtypes, size.restype = [C.c_void_p], C.c_size_t
+    square = next(v for v in range(device.bp_num_variants(True)) if device.bp_variant_shape(True, v)[:2] == (16, 16))
+    for P, fits in ((65535, True), (65536, False)):
+        bp = device.Backprojection(geom_c0.replace(numberOfPixels=8, numberOfParallelProjections=P,
+                                                   numberOfParallelDetectors=8))
+        bp.variant = square << 8
+        assert [size(bp.h) > 0 for size in sizes] == [fits, fits]
+        bp.close()
