@@ -217,11 +217,11 @@ struct RowFrames {
 template <int T, bool PAD>
 __global__ void __launch_bounds__(T) fft_filter_kernel(RowFrames fr, uint16_t* __restrict__ out16, float out_scale,
                                                        const float2* __restrict__ tw, const float* __restrict__ H,
-                                                       FftPlan plan, int D, long rows)
+                                                       FftPlan plan, int D, long rows, long pair0)
 {
     extern __shared__ float2 lds[];
     const int M = plan.D, t0 = threadIdx.x;
-    const long ra = (long)blockIdx.x * 2, rb = ra + 1;
+    const long ra = (pair0 + blockIdx.x) * 2, rb = ra + 1;
     float2* b0 = lds;
     float2* b1 = b0 + row_index<PAD>(M);
     float2* twl = b1 + row_index<PAD>(M);
@@ -1413,9 +1413,14 @@ static void launch_fft(risa_filter_t h, const RowFrames& fr, uint16_t* out16, fl
         check_launch("fft512_filter_kernel");
         return;
     }
-    hipLaunchKernelGGL(RISA_ROW_KERNEL(fft_filter_kernel, h->plan), dim3((unsigned)pairs), dim3(row_threads(M)),
-                       row_lds(h->plan, 1), s, fr, out16, out_scale, h->tw.ptr, h->H.ptr, h->plan, D, rows);
-    check_launch("fft_filter_kernel");
+    // a launch has fewer than 2^32 threads
+    const long per = (1L << 31) / row_threads(M);
+    for (long p0 = 0; p0 < pairs; p0 += per) {
+        hipLaunchKernelGGL(RISA_ROW_KERNEL(fft_filter_kernel, h->plan), dim3((unsigned)std::min(per, pairs - p0)),
+                           dim3(row_threads(M)), row_lds(h->plan, 1), s, fr, out16, out_scale, h->tw.ptr, h->H.ptr,
+                           h->plan, D, rows, p0);
+        check_launch("fft_filter_kernel");
+    }
 }
 // `rows` consecutive rows in -> out (out null: FP16 output only).
 static void launch_fft(risa_filter_t h, const float* in, float* out, uint16_t* out16, float out_scale, long rows,
