@@ -2527,7 +2527,12 @@ static void setup_adjoint(risa_bp_s* h)
     }
     int nbmax = 0;
     for (int a = 0; a < P; a++) nbmax = std::max(nbmax, nb[a]);
-    if ((size_t)nbmax * kAdjRec * sizeof(float) > kMaxLds) return;   // a row's band records must fit the reduce's LDS
+    // a row's band records must fit the reduce's LDS; 224 bands are at most 14336
+    // pixels, so that a padded group of four images stays below 2^32 bytes, the
+    // range of the path kernel's offsets
+    if ((size_t)nbmax * kAdjRec * sizeof(float) > kMaxLds) return;
+    static_assert(kMaxLds / (kAdjRec * sizeof(float)) * 64 * (kMaxLds / (kAdjRec * sizeof(float)) * 64 + 2 * kAdjPad) * 16 <
+                      (size_t)1 << 32, "four padded images within 32-bit offsets");
     // rows of each band whose path segment meets the mask (one pixel of
     // margin); every row in between must stay inside the padded row
     std::vector<int2> bands((size_t)P * nbmax, make_int2(1, 0));
@@ -3106,10 +3111,8 @@ static void adjoint_run(risa_bp_t h, const float* img, int slices, float* sino, 
     hipLaunchKernelGGL(adj_tile_origin_kernel, dim3((unsigned)ceil_div(work, 256L)), dim3(256), 0, s, h->cosT.ptr,
                        h->sinT.ptr, q, h->adj_T.ptr, h->adj_coord.ptr);
     check_launch("adj_tile_origin_kernel");
-    // a group of 4 is read with 32-bit byte offsets
-    const int per = (unsigned long)q.img_stride * 16 >> 32 ? 2 : kAdjSlices;
-    for (int s0 = 0; s0 < slices; s0 += per) {
-        const int n = std::min(per, slices - s0);
+    for (int s0 = 0; s0 < slices; s0 += kAdjSlices) {
+        const int n = std::min(kAdjSlices, slices - s0);
         // 3 left over run as a group of 4
         q.quads = (n + 1) / 4;
         q.tail = n % 4 == 3 ? 0 : n % 4;
