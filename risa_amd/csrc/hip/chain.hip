@@ -201,9 +201,11 @@ extern "C" int risa_hip_chain_create(const risa_geom* g, const float* avg_ref, c
             const size_t fan = (size_t)g->numberOfFanDetectors * g->numberOfFanProjections;
             const size_t par = (size_t)g->numberOfParallelDetectors * g->numberOfParallelProjections;
             if (mode == RISA_CHAIN_PLAIN) {
-                // one group while it holds every frame (8 frames of 256^2 x 500:
-                // 97 us, 125 as two groups of 4 in two lanes), 32 to a group
-                // from 64 frames on (100 frames 539 us, 588 with 16)
+                // one group while it holds every frame (8 frames of 256^2 x 500 /
+                // 384^2 x 700 / 512^2 x 1000 / 560^2 x 300: 96 / 181 / 305 / 129
+                // us, 124 / 237 / 321 / 132 as two groups of 4 in two lanes; 2 to
+                // 16 frames of these 1.02 to 1.64 times faster), 32 to a group
+                // from 64 frames on (100 frames of 256^2 x 500 539 us, 588 with 16)
                 h->lanes = max_frames > kPlainMaxPer ? kPlainLanes : 1;
                 h->per = std::min(max_frames >= kPlainLanes * kSplitPer ? kSplitPer : kPlainMaxPer, max_frames);
                 if (max_frames >= kPlainLanes * kSplitPer && (h->split_bytes = risa_bp_split_bytes(h->bp)) > 0 &&

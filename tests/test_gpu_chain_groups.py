@@ -159,3 +159,79 @@ def test_packed_kernel_is_tried_whatever_shares_the_angles(risa, geom_c1, cuda):
             assert size(bp.h) > 0 and device.bp_variant_shape(True, now)[:2] == (16, 16)
         assert now == v or (square and shared)
     bp.close()
+
+
+def test_extreme_counts_stay_in_range(risa, orc, geom_c0, cuda):
+    """A plain call on the matrix cores with counts of 0 and 65535 side by side,
+    dead detectors (reference at or below the dark current) and blank frames:
+    finite, and near the float64 oracle.  Tolerance 1e-4: the FP32 angles (rounded
+    by 2^-23) move a ray by up to 3e-5 of a sample at 256 pixels from the centre,
+    neighbouring samples differ by up to twice their size."""
+    import torch
+    from conftest import rel_rmse
+    from risa_amd import device
+
+    g = geom_c0.replace(numberOfPixels=512, numberOfParallelDetectors=512, numberOfParallelProjections=300)
+    Pf, Df = g.fan_shape
+    rng = np.random.default_rng(3)
+    ref = np.full((1, Pf, Df), 60000.0, np.float32)
+    dark = np.full((1, Df), 300.0, np.float32)
+    ref[0, :, 50:53], ref[0, :, 200] = 300.0, 100.0
+    ref[0, 7, :] = 300.5
+    F = 64
+    raw = np.empty((F, Pf, Df), np.uint16)
+    p, d = np.mgrid[0:Pf, 0:Df]
+    for f in range(F):
+        raw[f] = ((p + d + f) % 2 * 65535, rng.integers(0, 2, (Pf, Df)) * 65535, np.zeros((Pf, Df)),
+                  np.full((Pf, Df), 65535))[f % 4]
+    chain = device.Chain(g, ref, dark, mode=risa.CHAIN_PLAIN, max_frames=F)
+    assert chain.on_matrix_cores(F)
+    img = torch.full((F,) + g.img_shape, float("nan"), dtype=torch.float32, device=cuda)
+    chain(torch.from_numpy(raw).to(cuda), np.zeros(F, np.int32), img)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(img).all())
+    want = orc.Chain(g, ref, dark)
+    for f in range(4):
+        err = rel_rmse(img[f].cpu().numpy(), want.f64(raw[f], 0))
+        print(f"case: extreme counts, frame {f}: rel RMSE against the oracle {err:.2e}", flush=True)
+        assert err < 1e-4
+    chain.close()
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_references_without_a_bound_keep_the_fp32_kernel(risa, geom_c1, cuda, bad):
+    from risa_amd import device
+
+    fs = FrameSet(geom_c1, 1, 1, R=2)
+    ref = fs.avg_ref.copy()
+    ref[1, 5, 17] = bad
+    chain = device.Chain(geom_c1, ref, fs.avg_dark, mode=risa.CHAIN_PLAIN, max_frames=64)
+    assert not chain.on_matrix_cores(64)
+    chain.close()
+
+
+def test_mixed_tail_on_the_matrix_cores(risa, geom_c1, cuda):
+    """Groups of 64 and 61 frames, the last x4 group partly empty: the bits of a
+    small chain with the same variants."""
+    import torch
+    from risa_amd import device
+
+    F = 125
+    fs, raw, planes = _frames(geom_c1, cuda, F)
+    a = device.Chain(geom_c1, fs.avg_ref, fs.avg_dark, mode=risa.CHAIN_MIXED, max_frames=128)
+    b = device.Chain(geom_c1, fs.avg_ref, fs.avg_dark, mode=risa.CHAIN_MIXED, max_frames=4)
+    b.variant = a.variant
+    square = device.bp_variant_shape(True, a.variant >> 8)[:2] == (16, 16)
+    assert a.on_matrix_cores(61) == a.on_matrix_cores(64) == square   # from 49 frames on or fewer
+    img = torch.full((F,) + geom_c1.img_shape, float("nan"), dtype=torch.float32, device=cuda)
+    a(raw, planes, img)
+    part = torch.empty((4,) + geom_c1.img_shape, dtype=torch.float32, device=cuda)
+    for f in (0, 60, 64, 120):
+        b(raw[f:f + 4], planes[f:f + 4], part)
+        torch.cuda.synchronize()
+        assert torch.equal(img[f:f + 4], part), f"frames {f} .. {f + 3}"
+    b(raw[124:], planes[124:], part[:1])
+    torch.cuda.synchronize()
+    assert torch.equal(img[124], part[0])
+    a.close()
+    b.close()
