@@ -11,7 +11,8 @@ value       : plain FP32 chain (frame by frame, FFT filter, FP32 BP), slices/s.
 mixed       : mixed-precision batched chain (DFT-GEMM filter on MFMA with
               FP16 output, FP16-sinogram / FP32-accumulate BP), slices/s and
               its relative RMSE / max error against the FP64 oracle.
-roofline    : the dominant kernel (backprojection), FP32-ALU bound.
+roofline    : the FP32 vector backprojector (batches, short chain calls),
+              FP32-ALU bound; config names what the chains' calls run.
 cpu_baseline: the faithful-FP32 CPU restatement (the oracle) on a bounded
               sample, on this host's cores.
 
@@ -35,7 +36,7 @@ METRIC = "512² slices/sec on 1 GPU (mixed vs plain FP32) at stated RMSE; BP HBM
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3
 FLOP_PER_UPDATE = 10          # t: mul+fma; two weights; two accumulate FMAs
-BP_SLICES_IN_FLIGHT = 32      # the plain chain keeps 2 lanes x 16 frames in flight
+BP_SLICES_IN_FLIGHT = 32      # slices per launch of the roofline leg
 
 
 def log(*a):
@@ -288,18 +289,20 @@ def main():
         return ms
 
     plain = device.Chain(g, avg_ref, avg_dark, mode=risa_amd.CHAIN_PLAIN, max_frames=chunk)
-    log(f"plain chain: backprojector variant {plain.variant & 0xFF} (autotuned)")
+    plain_bp = ("bp_split_kernel (FP16 hi + lo operands, 22 bits; FP32 sums)" if plain.on_matrix_cores(chunk)
+                else device.bp_kernel_name(False, plain.variant & 0xFF))
+    log(f"plain chain: {plain_bp}; FP32 variant {plain.variant & 0xFF} (autotuned)")
     ms_plain = timed(plain, "plain FP32")
     img_plain_sample = img[:planes].cpu().numpy()
 
     mixed = device.Chain(g, avg_ref, avg_dark, mode=risa_amd.CHAIN_MIXED, max_frames=chunk)
-    log(f"mixed chain: FP16 backprojector variant {mixed.variant >> 8} (autotuned)")
+    mixed_bp = "bp_f16_mfma_kernel" if mixed.on_matrix_cores(chunk) else device.bp_kernel_name(True, mixed.variant >> 8)
+    log(f"mixed chain: {mixed_bp}; FP16 variant {mixed.variant >> 8} (autotuned)")
     ms_mixed = timed(mixed, "mixed FP16/FP32")
     img_mixed_sample = img[:planes].cpu().numpy()
 
-    # Dominant kernel: backprojection, timed with HIP events on its stream,
-    # at the concurrency the plain chain runs it (2 lanes x 16 frames in
-    # flight = one launch of 32 slices here, tile shape autotuned for it).
+    # The FP32 vector backprojector, timed with HIP events on its stream, in
+    # launches of 32 slices, tile shape autotuned for them.
     P, D = g.numberOfParallelProjections, g.numberOfParallelDetectors
     S = BP_SLICES_IN_FLIGHT
     bp = device.Backprojection(g)
@@ -454,7 +457,7 @@ def main():
                        "forward_us_per_slice": round(times["forward"] * 1e3 / S4, 1),
                        "backward_us_per_slice": round(times["backward"] * 1e3 / S4, 1),
                        "what": "C4 geometry; forward = filter + batched backprojection; backward = "
-                               "bp_adjoint_path_kernel (batched, 16 slices per pass, 2 per wave) + fft_grad_taps_kernel + "
+                               "bp_adjoint_path_kernel (batched, 16 slices per pass, 4 per wave) + fft512_grad_taps_kernel + "
                                "conjugate filter; one step of the autograd function"}
             log(f"differentiable FBP: {adjoint}")
         except Exception as exc:  # reported, not fatal
@@ -609,7 +612,8 @@ def main():
                  f"in HBM; every frame is reconstructed"),
         "config": {"workload": "C1: 2 planes x 2000 frames, fan 768x1000 uint16 -> parallel 512x1000 -> "
                                "512^2 FP32, Shepp-Logan, circular mask; plain FP32 chain frame by frame",
-                   "slices_per_step": total, "frames_per_graph": chunk},
+                   "slices_per_step": total, "frames_per_graph": chunk, "plain_backprojection": plain_bp,
+                   "mixed_backprojection": mixed_bp},
         "mixed": {"value": round(mixed_value, 1), "unit": "slices/s", "ms_per_step": round(ms_mixed, 3),
                   "vs_plain": round(mixed_value / plain_value, 3), "dtype": "f16 storage / f32 accumulate"},
         "accuracy_vs_fp64_oracle": rmse,

@@ -931,17 +931,16 @@ __global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_groups_kernel(c
 // additions to ever larger sums at 1000 angles.  Each block of 64 angles is
 // therefore summed for itself and the blocks' sums are added up (32 registers,
 // 32 additions per 64 angles).  Relative RMSE against float64 of a
-// backprojection of ramp-filtered phantoms, by tile 32 x 32 / 16 x 16, and
+// backprojection of filtered phantoms, by tile 32 x 32 / 16 x 16, and
 // bp_linear_kernel's beside it: 512^2 x 1000 angles 2.68e-6 / 2.68e-6 (2.78e-6 /
 // 2.76e-6; most of it is the angles' own FP32 rounding), 256^2 x 500 1.22e-6 /
 // 1.20e-6 (1.35e-6 / 1.31e-6), 431 detectors on 501^2 x 776 8.4e-7 (1.09e-6),
-// 504 on 454^2 x 763 1.47e-6 (1.61e-6); below it in all 12 geometries of 200 to
-// 560 pixels tried.  As one running sum it was above it, by 1 to 11 per cent.
+// 504 on 454^2 x 763 1.47e-6 (1.61e-6); below it in all 11 geometries of 246 to
+// 552 pixels tried.  As one running sum it was above it, by 1 to 11 per cent.
 //
-// The pixels' coordinates and
-// weights cost the vector unit about 24 instructions per 64 (pixel, angle)
-// pairs whatever the number of slices, where bp_linear_kernel spends 2.8 per
-// pair and slice.
+// The pixels' coordinates and weights cost the vector unit about 24 instructions
+// per 64 (pixel, angle) pairs whatever the number of slices, where
+// bp_linear_kernel spends 2.8 per pair and slice.
 //
 // Weight placement: with kb the block's first sample (an even detector, so
 // two samples share a dword) and q = floor(t) - kb in [0, 6], the eight
@@ -961,15 +960,17 @@ __global__ void __launch_bounds__(TX* TY / PPT* Q) bp_linear_f16_groups_kernel(c
 // next angle's rows, or the zeroed bytes between angles and at the end of the
 // buffer).
 //
-// Bound: LDS reads.  A block's operands take 5 KB per 64 (pixel, angle) pairs
-// (4 KB of samples, 1 KB of selectors) at the ~105 bytes per clock and CU that
-// two-address reads deliver, against about 195 clocks of vector and matrix
-// issue.  Four waves per SIMD: the two sets of sums take 64 registers, and six
-// or eight waves would spill them (512^2 x 1000 angles, 32 slices alone, 32 x
-// 32 / 32 x 16 / 16 x 16 tiles: 510 / 505 / 524 us, 624 and 790 for the smaller
-// two with six and eight waves; 384^2 x 700 323 / 269 / 271, bp_linear_kernel
-// 356).  512^2 x 1000 angles, 32 slices: 14.1 us per slice with two launches in
-// flight (packing included, 0.65), bp_linear_kernel 24.5.
+// Bound: issue, LDS reads beside it, and too few waves to fill either.  In a
+// launch of 32 slices of 512^2 x 1000 angles the vector unit issues in 46 % of a
+// SIMD's clocks and the matrix cores are busy in 28 %, the LDS in 45 % of a CU's
+// (5 KB of operands per 64 (pixel, angle) pairs, no bank conflicts), and a wave
+// waits for 43 % of its time.  Four waves per SIMD: the two sets of sums take 64
+// registers, and six or eight waves would spill them.  512^2 x 1000 angles, 32
+// slices with their packing (20 us), 32 x 32 / 32 x 16 / 16 x 16 tiles: 510 / 505
+// / 524 us (624 and 790 for the smaller two with six and eight waves),
+// bp_linear_kernel 745; 384^2 x 700 323 / 269 / 271 and 356.  Up to 16 slices
+// read half of the samples and take 397 / 443 / 481 us without the packing, 32
+// take 516 / 552 / 568.
 // ---------------------------------------------------------------------------
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -1302,7 +1303,9 @@ __global__ void __launch_bounds__(TX* TY, 4) bp_split_kernel(const unsigned* __r
 // of its neighbours as NaN: a wave that ends with a non-finite sum evaluates
 // its pixels again one by one (bp_f16_pixel).
 //
-// Bound: LDS latency under load and instruction issue.  A wave spends about 65
+// Bound: issue and LDS latency under load (vector issue in 47 % of a SIMD's
+// clocks, matrix cores busy in 28 %, LDS in 42 % of a CU's without conflicts, a
+// wave waiting for 46 % of its time).  A wave spends about 65
 // instructions, 6.4 KB of LDS reads and 4 products per angle on 64 pixels of 64
 // slices (bp_linear_f16_kernel 1.4 vector operations and 4 bytes of LDS per
 // pixel and slice), so the 64 slices share what a pixel costs; the sums take

@@ -15,8 +15,8 @@
 //        frames take groups of 32 and backproject a call on the matrix cores
 //        (bp_split_kernel) where timing both at creation says that this is the
 //        faster way for its number of frames: 256 frames of 512^2 x 1000 angles
-//        4.15 ms a call, 6.67 with bp_linear_kernel; 256^2 x 500 stays with
-//        the latter (158 us per 32 slices against 208).
+//        4.29 ms a call, 6.67 with bp_linear_kernel; 256^2 x 500 stays with
+//        the latter (125 us per 32 slices against 179).
 // MIXED: groups of `per` consecutive frames (a multiple of 4, up to 32) dealt
 //        to `lanes` streams the same way; per group the DFT-GEMM filter on
 //        MFMA writes the FP16 sinogram in the 4-slice interleaved layout and
