@@ -7,11 +7,12 @@
 //
 // PLAIN: frame by frame, FP32 in and out of every stage (FFT filter, FP32
 //        backprojector; on the matrix cores its products are of FP16 hi + lo
-//        operands, 22 bits, its sums FP32).  Groups of `per` consecutive frames (up to 16, or 32; each stage runs
-//        once per group) are dealt round-robin to `lanes` streams (own scratch
-//        buffers each) forked from and joined back into the caller's stream,
-//        so lanes x per frames are in flight -- the way the reference
-//        overlaps frames across its per-stage threads.  Chains of at least 64
+//        operands, 22 bits, its sums FP32).  Groups of `per` consecutive
+//        frames (up to 16, or 32; each stage runs once per group) are dealt
+//        round-robin to `lanes` streams (own scratch buffers each) forked from
+//        and joined back into the caller's stream, so lanes x per frames are in
+//        flight -- the way the reference overlaps frames across its per-stage
+//        threads.  Chains of at least 64
 //        frames take groups of 32 and backproject a call on the matrix cores
 //        (bp_split_kernel) where timing both at creation says that this is the
 //        faster way for its number of frames: 256 frames of 512^2 x 1000 angles
